@@ -265,6 +265,15 @@ __device__ __forceinline__ void fc_hidden(const float4* fr, int lane, int g, int
     // a scalar index (see IDX)
     const bool mine = g == ((mb & 15) >> 2);
     const int sel = __builtin_amdgcn_readfirstlane(((mb >> 4) << 2) | (mb & 3));
+    if constexpr (IDX) {
+      // The indexed read names only the array's first register, so the
+      // compiler's own wait covers that one alone: the last MFMA's results
+      // take up to 11 wait states more (read too early, the bias dot of a
+      // layer whose bias row falls in its last two entries is a stale value).
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_nop 15");
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       float v = 0.f;
