@@ -295,6 +295,31 @@ int vc_backward_relu_conv(const float *ew_in, int64_t M, int64_t R, int ew_share
                           int kh, int kw, int sh, int sw, int ph, int pw,
                           float *ew_out, float *acc, vc_stream_t stream);
 
+/* The conv backward on the bf16 matrix cores, each fp32 value and weight as
+ * three bf16 parts (at least the accuracy of the fp32 matrix products), with
+ * the relu backward before it in its loads when lo_s, up_s and up_t are given:
+ *   e = pos(x) lo_s + neg(x) up_s [+ beta];  acc[m] += neg(x) . up_t + e . bias;
+ *   ew_out[m] = conv_transpose2d(e)
+ * for M = B * R rows, x from input row m or, with ew_shared, row m mod R of the
+ * R rows every domain shares.  Slopes and beta as in vc_backward_relu_conv.
+ * packed: the kernel's parts from vc_conv_split_pack (16-byte aligned,
+ * vc_conv_split_pack_bytes of them), laid out once per kernel; kernel itself is
+ * read where an infinity or NaN among the values asks for the plain sum.
+ * vc_backward_conv_split_ok says whether a geometry qualifies, else
+ * VC_ERR_UNSUPPORTED.
+ * Replaces verify_zono_bnb.py:4409-4453 followed by 4568-4593. */
+int64_t vc_conv_split_pack_bytes(int C_out, int C_in, int kh, int kw, int sh, int sw);
+int vc_conv_split_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,
+                       int sw, void *out, vc_stream_t stream);
+int vc_backward_conv_split_ok(int C_out, int H_out, int W_out, int C_in, int H, int W,
+                              int kh, int kw, int sh, int sw, int ph, int pw);
+int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shared,
+                           const float *lo_s, const float *up_s, const float *up_t,
+                           const float *beta, const float *kernel, const void *packed,
+                           const float *bias, int C_out, int H_out, int W_out, int C_in,
+                           int H, int W, int kh, int kw, int sh, int sw, int ph, int pw,
+                           float *ew_out, float *acc, vc_stream_t stream);
+
 /* Concretization over the input boxes:
  *   lb[m] = acc[m] + sum_i pos(A[m,i]) xl[b,i] + neg(A[m,i]) xh[b,i].
  * A (M, n_in), acc/lb (M), xl/xh (B, n_in), M = B * R.  With a_bcast != 0,

@@ -197,6 +197,22 @@ def _conv_t_taps(p, st):
     return packed
 
 
+def _conv_split_parts(p, st):
+    """The conv kernel's bf16 parts for vc_backward_conv_split, made on first
+    use by a backward pass and cached with the op's other device tensors;
+    None where the geometry is outside that kernel."""
+    if 'KS' not in p:
+        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+        p['KS'] = None
+        if _lib.load().vc_backward_conv_split_ok(C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph,
+                                                 pw):
+            n = _lib.load().vc_conv_split_pack_bytes(C_out, C_in, kh, kw, sh, sw)
+            parts = torch.empty(n, dtype=torch.uint8, device=p['K'].device)
+            call('vc_conv_split_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ptr(parts), st)
+            p['KS'] = parts
+    return p['KS']
+
+
 def _pair(v):
     if isinstance(v, int):
         return v, v
@@ -649,19 +665,27 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              ptr(acc), st)
         return _Rows(out, False)
 
-    def relu_conv(rows, op, p):
-        """The pending relu relaxation fused into the conv backward that
-        follows it (vc_backward_relu_conv), or None when the geometry or
-        the relaxation's form is outside the fused kernel."""
-        if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
-            return None
+    def few_channels(p):
+        """Whether the conv is the fold kernel's (vc_backward_relu_conv): a
+        few input channels, the network's first layer."""
         ok = p.get('relu_conv_ok')
         if ok is None:
             C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
             ok = bool(_lib.load().vc_backward_relu_conv_ok(C_out, Ho, Wo, C_in, H, W, kh, kw,
                                                            sh, sw, ph, pw))
             p['relu_conv_ok'] = ok
-        if not ok:
+        return ok
+
+    def relu_conv(rows, op, p):
+        """The pending relu relaxation fused into the conv backward that
+        follows it (vc_backward_relu_conv for a few input channels, else
+        vc_backward_conv_split), or None when the geometry or the
+        relaxation's form is outside the fused kernels."""
+        if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
+            return None
+        fold = few_channels(p)
+        parts = None if fold else _conv_split_parts(p, st)
+        if not fold and parts is None:
             return None
         L = rows.relu
         lo, hi = f32(tight[L][0]), f32(tight[L][1])
@@ -674,6 +698,11 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              ptr(ut), st)
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
         out = torch.empty(B * R, p['n_in'], device=dev)
+        if parts is not None:
+            call('vc_backward_conv_split', ptr(rows.ew), B * R, R, 1 if rows.shared else 0,
+                 ptr(ls), ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(parts), ptr(p['b']),
+                 C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
+            return out
         call('vc_backward_relu_conv', ptr(rows.ew), B * R, R, 1 if rows.shared else 0, ptr(ls),
              ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(p['b']), C_out, Ho, Wo, C_in,
              H, W, kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
@@ -816,6 +845,13 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 per_domain_acc()
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
+            parts = None if few_channels(p) else _conv_split_parts(p, st)
+            if parts is not None:
+                call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
+                     ptr(p['K']), ptr(parts), ptr(p['b']), C_out, Ho, Wo, C_in, H, W, kh, kw,
+                     sh, sw, ph, pw, ptr(out), ptr(acc), st)
+                put(inp, _Rows(out, rows.shared))
+                continue
             call('vc_backward_conv_packed', ptr(rows.ew), M, ptr(p['K']),
                  ptr(_conv_t_taps(p, st)), ptr(p['b']), C_out, Ho, Wo, C_in, H, W,
                  kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
