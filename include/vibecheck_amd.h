@@ -318,7 +318,35 @@ int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shar
                            const float *beta, const float *kernel, const void *packed,
                            const float *bias, int C_out, int H_out, int W_out, int C_in,
                            int H, int W, int kh, int kw, int sh, int sw, int ph, int pw,
-                           float *ew_out, float *acc, vc_stream_t stream);
+                           const int32_t *origin, int H_img, int W_img, float *ew_out,
+                           float *acc, vc_stream_t stream);
+
+/* Rows that are zero outside a window, as the rows of single conv neurons are:
+ * the backward of one neuron through a conv is its own kernel, a kh x kw window
+ * of the conv's input, and every further conv widens the window to
+ * (wh - 1) sh + kh.  A row holds (C, wh, ww) values; origin (R, 2) is its
+ * window's first row and column in the (H, W) image of its layer, part of the
+ * window may lie outside.  Row m of a batch sits at origin[m mod R].
+ * The reference carries these rows whole (verify_zono_bnb.py:4123-4147).
+ * vc_patch_seed: the conv backward of the one-hot rows of neurons idx (k), "+"
+ *   rows then "-" rows: rows (2k, C_in kh kw), origin (2k, 2), and acc (2k) =
+ *   +- bias.
+ * vc_backward_conv_split with origin: H_out x W_out is the window, H_img x
+ *   W_img the image that slopes and beta cover, H = (H_out - 1) sh + kh (and W),
+ *   ph = pw = 0; vc_patch_shift gives the output windows' origin (ph, pw the
+ *   conv's own padding).
+ * vc_patch_concretize: vc_concretize of M = B * R window rows (a_shared: R).
+ * vc_patch_dense: N window rows into whole (C, H, W) images. */
+int vc_patch_seed(const float *kernel, const float *bias, const int32_t *idx, int k, int C_out,
+                  int H_out, int W_out, int C_in, int kh, int kw, int sh, int sw, int ph,
+                  int pw, float *rows, int32_t *origin, float *acc, vc_stream_t stream);
+int vc_patch_shift(const int32_t *origin_in, int R, int sh, int sw, int ph, int pw,
+                   int32_t *origin_out, vc_stream_t stream);
+int vc_patch_concretize(const float *A, int a_shared, const int32_t *origin, const float *acc,
+                        const float *xl, const float *xh, int64_t M, int64_t R, int C, int H,
+                        int W, int wh, int ww, float *lb, vc_stream_t stream);
+int vc_patch_dense(const float *A, const int32_t *origin, int64_t N, int64_t R, int C, int H,
+                   int W, int wh, int ww, float *out, vc_stream_t stream);
 
 /* Concretization over the input boxes:
  *   lb[m] = acc[m] + sum_i pos(A[m,i]) xl[b,i] + neg(A[m,i]) xh[b,i].

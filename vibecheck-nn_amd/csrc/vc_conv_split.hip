@@ -56,6 +56,7 @@ struct SplitArgs {
   const float* ew;  // R rows (shared) or M rows of C_out Hs Ws
   int64_t M, R;
   int shared;
+  const int* origin;  // (R, 2): image position of each row's window, or null
   const float *ls, *us, *ut, *beta;  // (M / R, C_out Hi Wi) or null
   const float* K;                    // (C_out, C_in, kh, kw): the exact form's
   const uint4* A;                    // packed parts
@@ -88,7 +89,9 @@ __device__ __forceinline__ const SplitArgs& reread() {
 template <int RL>
 __device__ __forceinline__ float plain_sum(const SplitArgs& a, int64_t m, int ci, int y, int x) {
   const int64_t d = m / a.R;
-  const float* s = a.ew + (a.shared ? m - d * a.R : m) * a.C_out * a.Hs * a.Ws;
+  const int64_t row = m - d * a.R;
+  const float* s = a.ew + (a.shared ? row : m) * a.C_out * a.Hs * a.Ws;
+  const int oy = a.origin ? a.origin[2 * row] : 0, ox = a.origin ? a.origin[2 * row + 1] : 0;
   double sum = 0.0;
   for (int ky = 0; ky < a.kh; ++ky) {
     const int ty = y + a.ph - ky, qy = ty / a.sh;
@@ -96,8 +99,9 @@ __device__ __forceinline__ float plain_sum(const SplitArgs& a, int64_t m, int ci
     for (int kx = 0; kx < a.kw; ++kx) {
       const int tx = x + a.pw - kx, qx = tx / a.sw;
       if (tx < 0 || qx * a.sw != tx || qx >= a.Ws) continue;
+      if ((unsigned)(oy + qy) >= (unsigned)a.Hi || (unsigned)(ox + qx) >= (unsigned)a.Wi) continue;
       for (int co = 0; co < a.C_out; ++co) {
-        const int64_t i = ((d * a.C_out + co) * a.Hi + qy) * a.Wi + qx;
+        const int64_t i = ((d * a.C_out + co) * a.Hi + oy + qy) * a.Wi + ox + qx;
         float e = s[((int64_t)co * a.Hs + qy) * a.Ws + qx];
         if (RL > 0) e = e * (e < 0.f ? a.us[i] : a.ls[i]);
         if (RL > 0 && a.beta) e = e + a.beta[i];
@@ -180,8 +184,11 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
             // row) and first domain on, this thread's image by its byte offset
             const uint32_t dom0 = b.f_R.div((uint32_t)m0);
             const uint32_t dom = ok ? b.f_R.div((uint32_t)m) : dom0;
+            const int64_t row = ok ? m - dom * b.R : 0;
+            const int oy = b.origin ? b.origin[2 * row] : 0;
+            const int ox = b.origin ? b.origin[2 * row + 1] : 0;
             const int64_t xb = b.shared ? 0 : m0 * n_e, ib = (int64_t)dom0 * n_i;
-            const uint32_t gx = 4 * (uint32_t)((b.shared ? (ok ? m - dom * b.R : 0) : g) * n_e);
+            const uint32_t gx = 4 * (uint32_t)((b.shared ? row : g) * n_e);
             const uint32_t gi = 4 * (uint32_t)((dom - dom0) * n_i);
             const Buf bx = buffer(b.ew + xb, ((b.shared ? b.R : b.M) * n_e - xb) * 4);
             const int64_t left = (b.M / b.R * n_i - ib) * 4;
@@ -200,10 +207,12 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
               const int ukg = (int)b.f_npx.div((uint32_t)j), up = j - ukg * npx;
               const int rr = (int)b.f_ws.div((uint32_t)up), x = up - rr * b.Ws;
               const int q = qa + rr, co0 = ch * CK + 8 * ukg;
-              const bool in = ok && (unsigned)q < (unsigned)b.Hs && co0 < b.C_out;
+              const int iy = oy + q, ix = ox + x;
+              const bool in = ok && (unsigned)q < (unsigned)b.Hs && co0 < b.C_out &&
+                              (unsigned)iy < (unsigned)b.Hi && (unsigned)ix < (unsigned)b.Wi;
               // outside the image: past the buffer, which reads as zero
               const uint32_t xo = in ? gx + 4 * ((co0 * b.Hs + q) * b.Ws + x) : kOut;
-              const uint32_t io = in ? gi + 4 * ((co0 * b.Hi + q) * b.Wi + x) : kOut;
+              const uint32_t io = in ? gi + 4 * ((co0 * b.Hi + iy) * b.Wi + ix) : kOut;
               float e[8], lv[8], uv[8], tv[8], bv[8];
 #pragma unroll
               for (int i = 0; i < 8; ++i) {
@@ -562,6 +571,90 @@ int launch_split(SplitArgs& a, hipStream_t st) {
   return VC_OK;
 }
 
+// Rows of a window: C x kh x kw values of each seeded neuron's own kernel and
+// their place in the image, "+" rows then "-" rows, and the bias as their
+// constant term (the conv backward of one-hot rows).
+__global__ void k_patch_seed(const float* K, const float* bias, const int* idx, int k, int sp,
+                             int Wo, int n, int sh, int sw, int ph, int pw, float* rows,
+                             int* origin, float* acc) {
+  const int64_t total = (int64_t)2 * k * n;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
+       t += (int64_t)gridDim.x * blockDim.x) {
+    const int r = (int)(t / n), i = (int)(t - (int64_t)r * n);
+    const int j = idx[r < k ? r : r - k];
+    const int c = j / sp, y = (j - c * sp) / Wo, x = (j - c * sp) - y * Wo;
+    const float v = K[(int64_t)c * n + i];
+    rows[t] = r < k ? v : -v;
+    if (i == 0) {
+      origin[2 * r] = y * sh - ph;
+      origin[2 * r + 1] = x * sw - pw;
+      const float b = bias ? bias[c] : 0.f;
+      acc[r] = r < k ? b : -b;
+    }
+  }
+}
+
+// The image positions of a conv's output windows from those of its input's.
+__global__ void k_patch_shift(const int* in, int n, int sh, int sw, int ph, int pw, int* out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) {
+    out[2 * t] = in[2 * t] * sh - ph;
+    out[2 * t + 1] = in[2 * t + 1] * sw - pw;
+  }
+}
+
+// lb[m] = acc[m] + sum over the window's pixels inside the image of
+// pos(A) xl + neg(A) xh; 16 lanes per row, summed in 64 bits.
+__global__ __launch_bounds__(CNT) void k_patch_concretize(const float* A, int shared,
+                                                          const int* origin, const float* acc,
+                                                          const float* xl, const float* xh,
+                                                          int64_t M, int64_t R, int C, int H,
+                                                          int W, int wh, int ww, FastDiv f_ww,
+                                                          FastDiv f_wp, float* lb) {
+  const int wp = wh * ww, n = C * wp;
+  for (int64_t m0 = (int64_t)blockIdx.x * (CNT / 16); m0 < M;
+       m0 += (int64_t)gridDim.x * (CNT / 16)) {
+    const int64_t mm = m0 + (threadIdx.x >> 4);
+    const int64_t m = mm < M ? mm : M - 1;  // past the end: recompute the last row, no store
+    const int64_t d = m / R, row = m - d * R;
+    const float* a = A + (shared ? row : m) * n;
+    const float *l = xl + d * C * H * W, *h = xh + d * C * H * W;
+    const int oy = origin[2 * row], ox = origin[2 * row + 1];
+    double s = 0.0;
+    for (int i = threadIdx.x & 15; i < n; i += 16) {
+      const int c = (int)f_wp.div((uint32_t)i), p = i - c * wp;
+      const int dy = (int)f_ww.div((uint32_t)p), dx = p - dy * ww;
+      const int y = oy + dy, x = ox + dx;
+      if ((unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W) {
+        const int o = (c * H + y) * W + x;
+        const float v = a[i];
+        s += (double)(v * (v < 0.f ? h[o] : l[o]));
+      }
+    }
+    s = row_sum16(s);
+    if ((threadIdx.x & 15) == 0 && mm < M) lb[mm] = (float)((double)acc[mm] + s);
+  }
+}
+
+// Windows into whole images: rows (N, C, H, W), zero outside the window.
+// Row n's window sits at origin[n mod R].
+__global__ __launch_bounds__(CNT) void k_patch_dense(const float* A, const int* origin, int64_t N,
+                                                     int64_t R, int C, int H, int W, int wh,
+                                                     int ww, FastDiv f_w, FastDiv f_hw,
+                                                     float* out) {
+  const int hw = H * W;
+  for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
+    const int64_t row = n % R;
+    const int oy = origin[2 * row], ox = origin[2 * row + 1];
+    for (int i = threadIdx.x; i < C * hw; i += CNT) {
+      const int c = (int)f_hw.div((uint32_t)i), p = i - c * hw;
+      const int y = (int)f_w.div((uint32_t)p) - oy, x = p - (y + oy) * W - ox;
+      const bool in = (unsigned)y < (unsigned)wh && (unsigned)x < (unsigned)ww;
+      out[n * C * hw + i] = in ? A[((n * C + c) * wh + y) * ww + x] : 0.f;
+    }
+  }
+}
+
 bool geom_ok(int C_out, int Hs, int Ws, int C_in, int H, int W, int kh, int kw, int sh, int sw,
              int ph, int pw) {
   return C_out > 0 && Hs > 0 && Ws > 0 && C_in > 0 && H > 0 && W > 0 && kh > 0 && kw > 0 &&
@@ -602,8 +695,10 @@ extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, 
                                       const float* beta, const float* kernel, const void* packed,
                                       const float* bias, int C_out, int H_out, int W_out,
                                       int C_in, int H, int W, int kh, int kw, int sh, int sw,
-                                      int ph, int pw, float* ew_out, float* acc,
-                                      vc_stream_t stream) {
+                                      int ph, int pw, const int* origin, int H_img, int W_img,
+                                      float* ew_out, float* acc, vc_stream_t stream) {
+  if (!origin) H_img = H_out, W_img = W_out;
+  if (H_img <= 0 || W_img <= 0) return VC_ERR_ARG;
   if (!geom_ok(C_out, H_out, W_out, C_in, H, W, kh, kw, sh, sw, ph, pw) || !ew_in || !kernel ||
       !packed || !aligned16(packed) || !ew_out || M < 0 || R <= 0 || M % R)
     return VC_ERR_ARG;
@@ -615,8 +710,66 @@ extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, 
   a.ew = ew_in, a.M = M, a.R = R, a.shared = ew_shared ? 1 : 0;
   a.ls = lo_s, a.us = up_s, a.ut = up_t, a.beta = beta;
   a.K = kernel, a.A = (const uint4*)packed, a.bias = bias, a.out = ew_out, a.acc = acc;
-  a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_out, a.Wi = W_out;
+  a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_img, a.Wi = W_img;
+  a.origin = origin;
   a.C_in = C_in, a.H = H, a.W = W;
   a.kh = kh, a.kw = kw, a.sh = sh, a.sw = sw, a.ph = ph, a.pw = pw;
   return launch_split(a, (hipStream_t)stream);
+}
+
+extern "C" int vc_patch_seed(const float* kernel, const float* bias, const int32_t* idx, int k,
+                             int C_out, int H_out, int W_out, int C_in, int kh, int kw, int sh,
+                             int sw, int ph, int pw, float* rows, int32_t* origin, float* acc,
+                             vc_stream_t stream) {
+  if (!kernel || !idx || !rows || !origin || !acc || k < 0 || C_out <= 0 || H_out <= 0 ||
+      W_out <= 0 || C_in <= 0 || kh <= 0 || kw <= 0 || sh <= 0 || sw <= 0 || ph < 0 || pw < 0)
+    return VC_ERR_ARG;
+  const int64_t n = (int64_t)C_in * kh * kw;
+  if (n > (1 << 30) || (int64_t)C_out * H_out * W_out > (1 << 30)) return VC_ERR_UNSUPPORTED;
+  if (k == 0) return VC_OK;
+  hipLaunchKernelGGL(k_patch_seed, dim3(vc_blocks(2 * k * n, CNT)), dim3(CNT), 0,
+                     (hipStream_t)stream, kernel, bias, idx, k, H_out * W_out, W_out, (int)n, sh,
+                     sw, ph, pw, rows, origin, acc);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_patch_shift(const int32_t* origin_in, int R, int sh, int sw, int ph, int pw,
+                              int32_t* origin_out, vc_stream_t stream) {
+  if (!origin_in || !origin_out || R < 0 || sh <= 0 || sw <= 0 || ph < 0 || pw < 0)
+    return VC_ERR_ARG;
+  if (R == 0) return VC_OK;
+  hipLaunchKernelGGL(k_patch_shift, dim3((R + CNT - 1) / CNT), dim3(CNT), 0, (hipStream_t)stream,
+                     origin_in, R, sh, sw, ph, pw, origin_out);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_patch_concretize(const float* A, int a_shared, const int32_t* origin,
+                                   const float* acc, const float* xl, const float* xh, int64_t M,
+                                   int64_t R, int C, int H, int W, int wh, int ww, float* lb,
+                                   vc_stream_t stream) {
+  if (!A || !origin || !acc || !xl || !xh || !lb || M < 0 || R <= 0 || M % R || C <= 0 ||
+      H <= 0 || W <= 0 || wh <= 0 || ww <= 0)
+    return VC_ERR_ARG;
+  if ((int64_t)C * wh * ww > (1 << 30) || (int64_t)C * H * W > (1 << 30)) return VC_ERR_UNSUPPORTED;
+  if (M == 0) return VC_OK;
+  hipLaunchKernelGGL(k_patch_concretize, dim3(vc_blocks(16 * M, CNT)), dim3(CNT), 0,
+                     (hipStream_t)stream, A, a_shared ? 1 : 0, origin, acc, xl, xh, M, R, C, H, W,
+                     wh, ww, FastDiv::make((uint32_t)ww), FastDiv::make((uint32_t)(wh * ww)), lb);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_patch_dense(const float* A, const int32_t* origin, int64_t N, int64_t R, int C,
+                              int H, int W, int wh, int ww, float* out, vc_stream_t stream) {
+  if (!A || !origin || !out || N < 0 || R <= 0 || C <= 0 || H <= 0 || W <= 0 || wh <= 0 || ww <= 0)
+    return VC_ERR_ARG;
+  if ((int64_t)C * H * W > (1 << 30)) return VC_ERR_UNSUPPORTED;
+  if (N == 0) return VC_OK;
+  hipLaunchKernelGGL(k_patch_dense, dim3((unsigned)(N < vcg::kMaxGrid ? N : vcg::kMaxGrid)),
+                     dim3(CNT), 0, (hipStream_t)stream, A, origin, N, R, C, H, W, wh, ww,
+                     FastDiv::make((uint32_t)W), FastDiv::make((uint32_t)(H * W)), out);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
 }

@@ -62,7 +62,11 @@ SIGNATURES = {
     'vc_conv_split_pack': [_P, _I, _I, _I, _I, _I, _I, _P, _P],
     'vc_backward_conv_split_ok': [_I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I],
     'vc_backward_conv_split': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
-                               _I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
+                               _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _P, _P],
+    'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
+    'vc_patch_shift': [_P, _I, _I, _I, _I, _I, _P, _P],
+    'vc_patch_concretize': [_P, _I, _P, _P, _P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
+    'vc_patch_dense': [_P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
     'vc_concretize': [_P, _P, _P, _P, _L, _I, _I, _I, _P, _P],
     'vc_crown_intersect': [_P, _P, _I, _L, _I, _P, _P, _P],
     'vc_unstable_union': [_P, _P, _L, _I, _P, _P],

@@ -551,9 +551,11 @@ class _Rows:
     whose relaxation is still to be applied (it is fused into the next fc).
     ``alpha``/``beta`` belong to that pending relu; ``alpha_group`` (B,)
     int64 makes ``alpha`` (G*R, n) the rows of each domain's group.
+    ``window`` (a _Window) says that ``ew`` holds only that part of each row's
+    image, the rest being zero.
     """
     __slots__ = ('ew', 'shared', 'relu', 'alpha', 'alpha_row', 'beta', 'alpha_group',
-                 'n_groups')
+                 'n_groups', 'window')
 
     def __init__(self, ew, shared):
         self.ew = ew
@@ -564,6 +566,21 @@ class _Rows:
         self.beta = None
         self.alpha_group = None
         self.n_groups = 0
+        self.window = None
+
+
+class _Window:
+    """Rows (.., C, wh, ww) at ``origin`` (R, 2) of (C, H, W) images: what a
+    few conv neurons' rows meet of the layers below them."""
+    __slots__ = ('origin', 'wh', 'ww', 'C', 'H', 'W')
+
+    def __init__(self, origin, wh, ww, C, H, W):
+        self.origin, self.wh, self.ww, self.C, self.H, self.W = origin, wh, ww, C, H, W
+
+    def worth(self):
+        """Windows up to half of the image are carried as such: beyond, the
+        part outside the image and the wider steps cost what is saved."""
+        return 2 * self.wh * self.ww <= self.H * self.W
 
 
 class BackwardTrace:
@@ -593,17 +610,19 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
               alpha_at_layer=None, relu_split_beta=None, trace=None):
     """Walk the ops backward from ``seed_name`` and concretize.
 
-    seed: (R, n) rows when ``seed_shared`` else (B*R, n); acc0: (R,) when
-    shared else (B*R,).  Returns (lb (B, R), A, a_shared, acc (B*R,)).
+    seed: (R, n) rows when ``seed_shared`` else (B*R, n), or a _Rows; acc0:
+    (R,) when shared else (B*R,).  Returns (lb (B, R), A, a_shared, acc (B*R,));
+    A of window rows is None.
     """
     B, n_in = xl.shape
     dev = xl.device
     st = stream()
     widths = _widths(gg, n_in)
-    R = seed.shape[0] if seed_shared else seed.shape[0] // max(B, 1)
+    rows = seed if isinstance(seed, _Rows) else _Rows(seed, seed_shared)
+    R = rows.ew.shape[0] if seed_shared else rows.ew.shape[0] // max(B, 1)
     acc = acc0.clone()
     acc_shared = seed_shared
-    ew_at = {seed_name: _Rows(seed, seed_shared)}
+    ew_at = {seed_name: rows}
     ops = gg['ops']
 
     def per_domain_acc():
@@ -644,8 +663,20 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             call('vc_rows_bias_dot', ptr(rows.ew), B * R, R, n, 1 if rows.shared else 0,
                  ptr(v), v.numel(), sign, ptr(acc), st)
 
+    def dense(rows):
+        """Window rows as whole images (other rows as they are)."""
+        w = rows.window
+        if w is not None:
+            N = rows.ew.shape[0]
+            out = torch.empty(N, w.C * w.H * w.W, device=dev)
+            call('vc_patch_dense', ptr(rows.ew), ptr(w.origin), N, R, w.C, w.H, w.W, w.wh, w.ww,
+                 ptr(out), st)
+            rows.ew, rows.window = out, None
+        return rows
+
     def materialize(rows):
         """Apply a pending relu relaxation with the standalone kernel."""
+        rows = dense(rows)
         if rows.relu is None:
             return rows
         if rows.alpha_group is not None:
@@ -676,6 +707,50 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             p['relu_conv_ok'] = ok
         return ok
 
+    def slopes(rows):
+        """The pending relu's slopes per (domain, neuron) for a conv that
+        relaxes its rows as it loads them."""
+        lo, hi = f32(tight[rows.relu][0]), f32(tight[rows.relu][1])
+        n = lo.shape[1]
+        per_domain_acc()
+        if trace is not None:
+            trace.relus.append((rows.relu, rows.ew, rows.shared))
+        out = [torch.empty(B, n, device=dev) for _ in range(3)]
+        call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(rows.alpha), B * n, ptr(out[0]),
+             ptr(out[1]), ptr(out[2]), st)
+        return out
+
+    def window_conv(rows, p):
+        """Window rows through a conv (vc_backward_conv_split), the pending
+        relu relaxed on the way; None where the window is no longer worth
+        it or the step is outside that kernel."""
+        w = rows.window
+        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+        if (not w.worth() or rows.alpha_group is not None
+                or (rows.alpha is not None and rows.alpha_row)):
+            return None
+        oh, ow = (w.wh - 1) * sh + kh, (w.ww - 1) * sw + kw
+        parts = _conv_split_parts(p, st)
+        if parts is None or not _lib.load().vc_backward_conv_split_ok(
+                C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0):
+            return None
+        ls = us = ut = None
+        if rows.relu is not None:
+            ls, us, ut = slopes(rows)
+        elif not rows.shared:
+            per_domain_acc()
+        M = R if rows.shared and rows.relu is None else B * R
+        out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
+                    and rows.relu is None)
+        call('vc_backward_conv_split', ptr(rows.ew), M, R, 1 if rows.shared else 0, ptr(ls),
+             ptr(us), ptr(ut), ptr(rows.beta) if rows.relu is not None else None, ptr(p['K']),
+             ptr(parts), ptr(p['b']), C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0,
+             ptr(w.origin), w.H, w.W, ptr(out.ew), ptr(acc), st)
+        origin = torch.empty_like(w.origin)
+        call('vc_patch_shift', ptr(w.origin), R, sh, sw, ph, pw, ptr(origin), st)
+        out.window = _Window(origin, oh, ow, C_in, H, W)
+        return out
+
     def relu_conv(rows, op, p):
         """The pending relu relaxation fused into the conv backward that
         follows it (vc_backward_relu_conv for a few input channels, else
@@ -687,21 +762,14 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         parts = None if fold else _conv_split_parts(p, st)
         if not fold and parts is None:
             return None
-        L = rows.relu
-        lo, hi = f32(tight[L][0]), f32(tight[L][1])
-        n = lo.shape[1]
-        per_domain_acc()
-        if trace is not None:
-            trace.relus.append((L, rows.ew, rows.shared))
-        ls, us, ut = (torch.empty(B, n, device=dev) for _ in range(3))
-        call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(rows.alpha), B * n, ptr(ls), ptr(us),
-             ptr(ut), st)
+        ls, us, ut = slopes(rows)
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
         out = torch.empty(B * R, p['n_in'], device=dev)
         if parts is not None:
             call('vc_backward_conv_split', ptr(rows.ew), B * R, R, 1 if rows.shared else 0,
                  ptr(ls), ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(parts), ptr(p['b']),
-                 C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
+                 C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, None, Ho, Wo, ptr(out),
+                 ptr(acc), st)
             return out
         call('vc_backward_relu_conv', ptr(rows.ew), B * R, R, 1 if rows.shared else 0, ptr(ls),
              ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(p['b']), C_out, Ho, Wo, C_in,
@@ -715,6 +783,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         rows = ew_at.pop(name)
         t = op['type']
         inp = op['inputs'][0]
+        if t not in ('conv', 'relu'):
+            rows = dense(rows)
         if t in ('add', 'sub', 'mul') and trace is not None:
             trace.other = trace.other or t
         if t == 'add' and op.get('is_merge'):
@@ -807,7 +877,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 put(inp, _Rows(out, rows.shared))
         elif t == 'relu':
             if 'layer_idx' in op:
-                rows = materialize(rows)
+                if rows.relu is not None:
+                    rows = materialize(rows)
                 L = op['layer_idx']
                 rows.relu = L
                 if alpha_at_layer is not None and L in alpha_at_layer:
@@ -834,6 +905,12 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             put(inp, rows)
         elif t == 'conv':
             p = _op_params(op, dev)
+            if rows.window is not None:
+                out = window_conv(rows, p)
+                if out is not None:
+                    put(inp, out)
+                    continue
+                rows = dense(rows)
             if rows.relu is not None and FUSED_RELU_CONV:
                 out = relu_conv(rows, op, p)
                 if out is not None:
@@ -849,7 +926,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
                      ptr(p['K']), ptr(parts), ptr(p['b']), C_out, Ho, Wo, C_in, H, W, kh, kw,
-                     sh, sw, ph, pw, ptr(out), ptr(acc), st)
+                     sh, sw, ph, pw, None, Ho, Wo, ptr(out), ptr(acc), st)
                 put(inp, _Rows(out, rows.shared))
                 continue
             call('vc_backward_conv_packed', ptr(rows.ew), M, ptr(p['K']),
@@ -865,10 +942,16 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     if rows is None:
         per_domain_acc()
         return acc.reshape(B, R).clone(), None, False, acc
+    lb = torch.empty(B * R, device=dev)
+    if rows.window is not None and rows.relu is None:
+        per_domain_acc()
+        w = rows.window
+        call('vc_patch_concretize', ptr(rows.ew), 1 if rows.shared else 0, ptr(w.origin),
+             ptr(acc), ptr(xl), ptr(xh), B * R, R, w.C, w.H, w.W, w.wh, w.ww, ptr(lb), st)
+        return lb.reshape(B, R), None, False, acc
     rows = materialize(rows)
     A = rows.ew
     per_domain_acc()
-    lb = torch.empty(B * R, device=dev)
     call('vc_concretize', ptr(A), ptr(acc), ptr(xl), ptr(xh), B * R, R, n_in,
          1 if rows.shared else 0, ptr(lb), st)
     return lb.reshape(B, R), A, rows.shared, acc
@@ -1015,9 +1098,31 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
         if m == 0:
             continue
         new_lo, new_hi = lo_L.clone(), hi_L.clone()
+        window = below = None
+        feed_op = next(op for op in gg['ops'] if op['name'] == feed)
+        if feed_op['type'] == 'conv':
+            p = _op_params(feed_op, dev)
+            C_in, H, W, _, kh, kw = p['geom'][:6]
+            if _Window(None, kh, kw, C_in, H, W).worth():
+                window, below = p, feed_op['inputs'][0]
         for c0 in range(0, m, ch):
             cidx = idx[c0:c0 + ch].contiguous()
             k = int(cidx.numel())
+            if window is not None:
+                # one conv neuron's row is its own kernel, a window of the
+                # conv's input (and acc its bias): no product, no whole rows
+                C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = window['geom']
+                rows = _Rows(torch.empty(2 * k, C_in * kh * kw, device=dev), True)
+                origin = torch.empty(2 * k, 2, dtype=torch.int32, device=dev)
+                acc0 = torch.empty(2 * k, device=dev)
+                call('vc_patch_seed', ptr(window['K']), ptr(window['b']), ptr(cidx), k, C_out,
+                     Ho, Wo, C_in, kh, kw, sh, sw, ph, pw, ptr(rows.ew), ptr(origin), ptr(acc0),
+                     st)
+                rows.window = _Window(origin, kh, kw, C_in, H, W)
+                sl, _, _, _ = _backward(tight, xl, xh, gg, below, rows, True, acc0)
+                call('vc_crown_intersect', ptr(sl.contiguous()), ptr(cidx), k, B, n,
+                     ptr(new_lo), ptr(new_hi), st)
+                continue
             seed = torch.zeros(2 * k, n, device=dev)
             ar = torch.arange(k, device=dev)
             seed[ar, cidx.long()] = 1.0
