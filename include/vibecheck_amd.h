@@ -318,8 +318,7 @@ int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shar
                            const float *beta, const float *kernel, const void *packed,
                            const float *bias, int C_out, int H_out, int W_out, int C_in,
                            int H, int W, int kh, int kw, int sh, int sw, int ph, int pw,
-                           const int32_t *origin, int H_img, int W_img, float *ew_out,
-                           float *acc, vc_stream_t stream);
+                           float *ew_out, float *acc, vc_stream_t stream);
 
 /* Rows that are zero outside a window, as the rows of single conv neurons are:
  * the backward of one neuron through a conv is its own kernel, a kh x kw window
@@ -331,10 +330,11 @@ int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shar
  * vc_patch_seed: the conv backward of the one-hot rows of neurons idx (k), "+"
  *   rows then "-" rows: rows (2k, C_in kh kw), origin (2k, 2), and acc (2k) =
  *   +- bias.
- * vc_backward_conv_split with origin: H_out x W_out is the window, H_img x
- *   W_img the image that slopes and beta cover, H = (H_out - 1) sh + kh (and W),
- *   ph = pw = 0; vc_patch_shift gives the output windows' origin (ph, pw the
- *   conv's own padding).
+ * vc_patch_relax: vc_backward_relu of M = B * R window rows (ew_shared: R) by
+ *   their images' slopes (B, C H W; null: copied), zero outside the image.
+ *   The conv backward of the relaxed windows is vc_backward_conv(_packed) of
+ *   (wh, ww) to ((wh - 1) sh + kh, (ww - 1) sw + kw) without padding.
+ * vc_patch_shift: that conv's windows' origin (ph, pw the conv's own padding).
  * vc_patch_concretize: vc_concretize of M = B * R window rows (a_shared: R).
  * vc_patch_dense: N window rows into whole (C, H, W) images. */
 int vc_patch_seed(const float *kernel, const float *bias, const int32_t *idx, int k, int C_out,
@@ -342,6 +342,10 @@ int vc_patch_seed(const float *kernel, const float *bias, const int32_t *idx, in
                   int pw, float *rows, int32_t *origin, float *acc, vc_stream_t stream);
 int vc_patch_shift(const int32_t *origin_in, int R, int sh, int sw, int ph, int pw,
                    int32_t *origin_out, vc_stream_t stream);
+int vc_patch_relax(const float *ew_in, int64_t M, int64_t R, int ew_shared, const float *lo_s,
+                   const float *up_s, const float *up_t, const float *beta,
+                   const int32_t *origin, int C, int H, int W, int wh, int ww, float *ew_out,
+                   float *acc, vc_stream_t stream);
 int vc_patch_concretize(const float *A, int a_shared, const int32_t *origin, const float *acc,
                         const float *xl, const float *xh, int64_t M, int64_t R, int C, int H,
                         int W, int wh, int ww, float *lb, vc_stream_t stream);

@@ -52,8 +52,8 @@ def _run(gpu, t, Ho, Wo, B, R, shared, relu, beta, C_out, C_in, H, W, kh, kw, sh
     acc = t['acc'].clone()
     call('vc_backward_conv_split', ptr(t['x']), B * R, R, shared, ptr(t.get('ls')),
          ptr(t.get('us')), ptr(t.get('ut')), ptr(t.get('beta')), ptr(t['K']), ptr(parts),
-         ptr(t['b']), C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, None, Ho, Wo, ptr(out),
-         ptr(acc), stream())
+         ptr(t['b']), C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc),
+         stream())
     return out, acc
 
 

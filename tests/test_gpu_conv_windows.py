@@ -1,6 +1,5 @@
 """CROWN bounds of conv neurons carried as windows of their images
-(vc_patch_seed, vc_backward_conv_split with origin, vc_patch_concretize,
-vc_patch_dense) against the whole-image oracle in 64 bits."""
+(vc_patch_seed, vc_patch_relax, vc_patch_concretize, vc_patch_dense) against the whole-image oracle in 64 bits."""
 import copy
 
 import pytest

@@ -40,23 +40,10 @@ constexpr int PXB = 3 * PTB + 16;  // per pixel: 208, so that 16 consecutive pix
                                    // on 16 distinct groups of four banks
 constexpr int kMaxLds = 78 * 1024;  // two workgroups per CU
 
-// Loads with the base in scalar registers, a 32-bit byte offset per lane and
-// a scalar one per channel; past the buffer's end (kOut) they return zero.
-typedef __amdgpu_buffer_rsrc_t Buf;
-constexpr uint32_t kOut = 0xffffffffu;
-__device__ __forceinline__ Buf buffer(const float* p, int64_t bytes) {
-  const int n = (int)(uint32_t)(bytes < 0xfffffff0ll ? bytes : 0xfffffff0ll);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, n, 0x00027000);
-}
-__device__ __forceinline__ float ldb(Buf b, uint32_t off, int soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, off, soff, 0));
-}
-
 struct SplitArgs {
   const float* ew;  // R rows (shared) or M rows of C_out Hs Ws
   int64_t M, R;
   int shared;
-  const int* origin;  // (R, 2): image position of each row's window, or null
   const float *ls, *us, *ut, *beta;  // (M / R, C_out Hi Wi) or null
   const float* K;                    // (C_out, C_in, kh, kw): the exact form's
   const uint4* A;                    // packed parts
@@ -89,9 +76,7 @@ __device__ __forceinline__ const SplitArgs& reread() {
 template <int RL>
 __device__ __forceinline__ float plain_sum(const SplitArgs& a, int64_t m, int ci, int y, int x) {
   const int64_t d = m / a.R;
-  const int64_t row = m - d * a.R;
-  const float* s = a.ew + (a.shared ? row : m) * a.C_out * a.Hs * a.Ws;
-  const int oy = a.origin ? a.origin[2 * row] : 0, ox = a.origin ? a.origin[2 * row + 1] : 0;
+  const float* s = a.ew + (a.shared ? m - d * a.R : m) * a.C_out * a.Hs * a.Ws;
   double sum = 0.0;
   for (int ky = 0; ky < a.kh; ++ky) {
     const int ty = y + a.ph - ky, qy = ty / a.sh;
@@ -99,9 +84,8 @@ __device__ __forceinline__ float plain_sum(const SplitArgs& a, int64_t m, int ci
     for (int kx = 0; kx < a.kw; ++kx) {
       const int tx = x + a.pw - kx, qx = tx / a.sw;
       if (tx < 0 || qx * a.sw != tx || qx >= a.Ws) continue;
-      if ((unsigned)(oy + qy) >= (unsigned)a.Hi || (unsigned)(ox + qx) >= (unsigned)a.Wi) continue;
       for (int co = 0; co < a.C_out; ++co) {
-        const int64_t i = ((d * a.C_out + co) * a.Hi + oy + qy) * a.Wi + ox + qx;
+        const int64_t i = ((d * a.C_out + co) * a.Hi + qy) * a.Wi + qx;
         float e = s[((int64_t)co * a.Hs + qy) * a.Ws + qx];
         if (RL > 0) e = e * (e < 0.f ? a.us[i] : a.ls[i]);
         if (RL > 0 && a.beta) e = e + a.beta[i];
@@ -184,11 +168,8 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
             // row) and first domain on, this thread's image by its byte offset
             const uint32_t dom0 = b.f_R.div((uint32_t)m0);
             const uint32_t dom = ok ? b.f_R.div((uint32_t)m) : dom0;
-            const int64_t row = ok ? m - dom * b.R : 0;
-            const int oy = b.origin ? b.origin[2 * row] : 0;
-            const int ox = b.origin ? b.origin[2 * row + 1] : 0;
             const int64_t xb = b.shared ? 0 : m0 * n_e, ib = (int64_t)dom0 * n_i;
-            const uint32_t gx = 4 * (uint32_t)((b.shared ? row : g) * n_e);
+            const uint32_t gx = 4 * (uint32_t)((b.shared ? (ok ? m - dom * b.R : 0) : g) * n_e);
             const uint32_t gi = 4 * (uint32_t)((dom - dom0) * n_i);
             const Buf bx = buffer(b.ew + xb, ((b.shared ? b.R : b.M) * n_e - xb) * 4);
             const int64_t left = (b.M / b.R * n_i - ib) * 4;
@@ -207,12 +188,10 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
               const int ukg = (int)b.f_npx.div((uint32_t)j), up = j - ukg * npx;
               const int rr = (int)b.f_ws.div((uint32_t)up), x = up - rr * b.Ws;
               const int q = qa + rr, co0 = ch * CK + 8 * ukg;
-              const int iy = oy + q, ix = ox + x;
-              const bool in = ok && (unsigned)q < (unsigned)b.Hs && co0 < b.C_out &&
-                              (unsigned)iy < (unsigned)b.Hi && (unsigned)ix < (unsigned)b.Wi;
+              const bool in = ok && (unsigned)q < (unsigned)b.Hs && co0 < b.C_out;
               // outside the image: past the buffer, which reads as zero
               const uint32_t xo = in ? gx + 4 * ((co0 * b.Hs + q) * b.Ws + x) : kOut;
-              const uint32_t io = in ? gi + 4 * ((co0 * b.Hi + iy) * b.Wi + ix) : kOut;
+              const uint32_t io = in ? gi + 4 * ((co0 * b.Hi + q) * b.Wi + x) : kOut;
               float e[8], lv[8], uv[8], tv[8], bv[8];
 #pragma unroll
               for (int i = 0; i < 8; ++i) {
@@ -320,6 +299,9 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
                     } else {
                       acc[mt][n0 + k] += z[mt][k] + t[mt][k];
                     }
+                    // summed here: sunk to the end, the parts of every tile would
+                    // live at once
+                    asm volatile("" : "+v"(acc[mt][n0 + k]));
                   }
 #pragma unroll
               for (int k = 0; k < NB; ++k)
@@ -603,6 +585,47 @@ __global__ void k_patch_shift(const int* in, int n, int sh, int sw, int ph, int 
   }
 }
 
+// Rows of windows relaxed by their domains' slopes at the windows' places in
+// the image (ls null: copied), zero outside the image, and the intercepts
+// added to acc in 64 bits: the separate relu step on windows.  One wave per
+// row, lanes along it: each row is read and written once, coalesced.
+__global__ __launch_bounds__(CNT) void k_patch_relax(const float* x, int shared, const float* ls,
+                                                     const float* us, const float* ut,
+                                                     const float* beta, const int* origin,
+                                                     int64_t M, int64_t R, int C, int H, int W,
+                                                     int wh, int ww, FastDiv f_ww, FastDiv f_wp,
+                                                     float* out, float* acc) {
+  const int wp = wh * ww, n = C * wp, lane = threadIdx.x & 63;
+  for (int64_t m = (int64_t)blockIdx.x * (CNT / 64) + (threadIdx.x >> 6); m < M;
+       m += (int64_t)gridDim.x * (CNT / 64)) {
+    const int64_t d = m / R, row = m - d * R, img = d * C * H * W;
+    const float* a = x + (shared ? row : m) * n;
+    const int oy = origin[2 * row], ox = origin[2 * row + 1];
+    double s = 0.0;
+    for (int i = lane; i < n; i += 64) {
+      const int c = (int)f_wp.div((uint32_t)i), p = i - c * wp;
+      const int dy = (int)f_ww.div((uint32_t)p), dx = p - dy * ww;
+      const int y = oy + dy, xx = ox + dx;
+      float e = 0.f;
+      if ((unsigned)y < (unsigned)H && (unsigned)xx < (unsigned)W) {
+        e = a[i];
+        if (ls) {
+          const int64_t o = img + (c * H + y) * W + xx;
+          const float en = e > 0.f ? 0.f : e, ep = e < 0.f ? 0.f : e;
+          s += (double)(en * ut[o]);
+          e = ep * ls[o] + en * us[o];
+          if (beta) e = e + beta[o];
+        }
+      }
+      out[m * n + i] = e;
+    }
+    if (ls) {
+      s = wave_sum_f64(s);
+      if (lane == 0) acc[m] = (float)((double)acc[m] + s);
+    }
+  }
+}
+
 // lb[m] = acc[m] + sum over the window's pixels inside the image of
 // pos(A) xl + neg(A) xh; 16 lanes per row, summed in 64 bits.
 __global__ __launch_bounds__(CNT) void k_patch_concretize(const float* A, int shared,
@@ -695,10 +718,7 @@ extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, 
                                       const float* beta, const float* kernel, const void* packed,
                                       const float* bias, int C_out, int H_out, int W_out,
                                       int C_in, int H, int W, int kh, int kw, int sh, int sw,
-                                      int ph, int pw, const int* origin, int H_img, int W_img,
-                                      float* ew_out, float* acc, vc_stream_t stream) {
-  if (!origin) H_img = H_out, W_img = W_out;
-  if (H_img <= 0 || W_img <= 0) return VC_ERR_ARG;
+                                      int ph, int pw, float* ew_out, float* acc, vc_stream_t stream) {
   if (!geom_ok(C_out, H_out, W_out, C_in, H, W, kh, kw, sh, sw, ph, pw) || !ew_in || !kernel ||
       !packed || !aligned16(packed) || !ew_out || M < 0 || R <= 0 || M % R)
     return VC_ERR_ARG;
@@ -710,8 +730,7 @@ extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, 
   a.ew = ew_in, a.M = M, a.R = R, a.shared = ew_shared ? 1 : 0;
   a.ls = lo_s, a.us = up_s, a.ut = up_t, a.beta = beta;
   a.K = kernel, a.A = (const uint4*)packed, a.bias = bias, a.out = ew_out, a.acc = acc;
-  a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_img, a.Wi = W_img;
-  a.origin = origin;
+  a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_out, a.Wi = W_out;
   a.C_in = C_in, a.H = H, a.W = W;
   a.kh = kh, a.kw = kw, a.sh = sh, a.sw = sw, a.ph = ph, a.pw = pw;
   return launch_split(a, (hipStream_t)stream);
@@ -741,6 +760,26 @@ extern "C" int vc_patch_shift(const int32_t* origin_in, int R, int sh, int sw, i
   if (R == 0) return VC_OK;
   hipLaunchKernelGGL(k_patch_shift, dim3((R + CNT - 1) / CNT), dim3(CNT), 0, (hipStream_t)stream,
                      origin_in, R, sh, sw, ph, pw, origin_out);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_patch_relax(const float* ew_in, int64_t M, int64_t R, int ew_shared,
+                              const float* lo_s, const float* up_s, const float* up_t,
+                              const float* beta, const int32_t* origin, int C, int H, int W,
+                              int wh, int ww, float* ew_out, float* acc, vc_stream_t stream) {
+  if (!ew_in || !origin || !ew_out || M < 0 || R <= 0 || M % R || C <= 0 || H <= 0 || W <= 0 ||
+      wh <= 0 || ww <= 0)
+    return VC_ERR_ARG;
+  if ((lo_s == nullptr) != (up_s == nullptr) || (lo_s == nullptr) != (up_t == nullptr) ||
+      (beta && !lo_s) || (lo_s && !acc))
+    return VC_ERR_ARG;
+  if ((int64_t)C * wh * ww > (1 << 30) || (int64_t)C * H * W > (1 << 30)) return VC_ERR_UNSUPPORTED;
+  if (M == 0) return VC_OK;
+  hipLaunchKernelGGL(k_patch_relax, dim3(vc_blocks(64 * M, CNT)), dim3(CNT), 0,
+                     (hipStream_t)stream, ew_in, ew_shared ? 1 : 0, lo_s, up_s, up_t, beta, origin,
+                     M, R, C, H, W, wh, ww, FastDiv::make((uint32_t)ww),
+                     FastDiv::make((uint32_t)(wh * ww)), ew_out, acc);
   VC_LAUNCH_CHECK();
   return VC_OK;
 }

@@ -56,6 +56,22 @@ __device__ __forceinline__ v4f mfma_bf16(const uint4& a, const uint4& b, v4f acc
 constexpr int kPartA[6] = {2, 0, 1, 1, 0, 0};
 constexpr int kPartB[6] = {0, 2, 1, 0, 1, 0};
 
+// Loads with the base in scalar registers, a 32-bit byte offset per lane and
+// a scalar one beside it; past the buffer's end (kOut) they return zero and
+// stores are dropped, so that edges need no branches.
+typedef __amdgpu_buffer_rsrc_t Buf;
+constexpr uint32_t kOut = 0xffffffffu;
+__device__ __forceinline__ Buf buffer(const float* p, int64_t bytes) {
+  const int n = (int)(uint32_t)(bytes < 0xfffffff0ll ? bytes : 0xfffffff0ll);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, n, 0x00027000);
+}
+__device__ __forceinline__ float ldb(Buf b, uint32_t off, int soff) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, off, soff, 0));
+}
+__device__ __forceinline__ v4f ldb4(Buf b, uint32_t off) {
+  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
+}
+
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 
 }  // namespace vcs

@@ -62,9 +62,10 @@ SIGNATURES = {
     'vc_conv_split_pack': [_P, _I, _I, _I, _I, _I, _I, _P, _P],
     'vc_backward_conv_split_ok': [_I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I],
     'vc_backward_conv_split': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
-                               _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _P, _P],
+                               _I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
     'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     'vc_patch_shift': [_P, _I, _I, _I, _I, _I, _P, _P],
+    'vc_patch_relax': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P],
     'vc_patch_concretize': [_P, _I, _P, _P, _P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
     'vc_patch_dense': [_P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
     'vc_concretize': [_P, _P, _P, _P, _L, _I, _I, _I, _P, _P],
@@ -138,6 +139,7 @@ SIGNATURES = {
 _RESTYPE = {'vc_compact_workspace': ctypes.c_int64,
             'vc_conv_t_pack_floats': ctypes.c_int64,
             'vc_conv_split_pack_bytes': ctypes.c_int64,
+            'vc_fc_split_pack_bytes': ctypes.c_int64,
             'vc_mlp_crown_rows_workspace': ctypes.c_int64,
             'vc_mlp_bab_round_workspace': ctypes.c_int64,
             'vc_mlp_bab_round_lookahead_workspace': ctypes.c_int64,

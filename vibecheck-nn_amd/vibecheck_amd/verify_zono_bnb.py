@@ -180,20 +180,24 @@ def _widths(gg, n_in):
     return w
 
 
-def _conv_t_taps(p, st):
+def _conv_t_taps(p, st, window=False):
     """The conv kernel's transposed taps packed per output-parity class
     (vc_conv_t_pack), made on first use by a backward pass and cached with
-    the op's other device tensors."""
-    packed = p.get('KT')
+    the op's other device tensors; ``window``: without the padding, for rows
+    that carry their place in the image."""
+    key = 'KT_window' if window else 'KT'
+    packed = p.get(key)
     if packed is None:
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
         n = _lib.load().vc_conv_t_pack_floats(C_out, C_in, kh, kw, sh, sw)
         if n < 0:
             raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {p["geom"]}')
         packed = torch.empty(n, device=p['K'].device)
+        if window:
+            ph = pw = 0
         call('vc_conv_t_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ph, pw,
              ptr(packed), st)
-        p['KT'] = packed
+        p[key] = packed
     return packed
 
 
@@ -607,11 +611,14 @@ def _expand_rows(t, B):
 
 
 def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
-              alpha_at_layer=None, relu_split_beta=None, trace=None):
+              alpha_at_layer=None, relu_split_beta=None, trace=None, split=True):
     """Walk the ops backward from ``seed_name`` and concretize.
 
     seed: (R, n) rows when ``seed_shared`` else (B*R, n), or a _Rows; acc0:
-    (R,) when shared else (B*R,).  Returns (lb (B, R), A, a_shared, acc (B*R,));
+    (R,) when shared else (B*R,).  split: products may run as bf16 parts on
+    the matrix cores; off where the bounds choose slopes, whose step at 1/2
+    turns a last-bit change of a bound into another lower slope (on 512 boxes
+    through 1024-wide layers one run in four).  Returns (lb (B, R), A, a_shared, acc (B*R,));
     A of window rows is None.
     """
     B, n_in = xl.shape
@@ -721,31 +728,32 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         return out
 
     def window_conv(rows, p):
-        """Window rows through a conv (vc_backward_conv_split), the pending
-        relu relaxed on the way; None where the window is no longer worth
-        it or the step is outside that kernel."""
+        """Window rows through a conv: the pending relu relaxed at their
+        places in the image, then the conv of the windows alone; None where
+        the window is no longer worth it or the alpha's form is another."""
         w = rows.window
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        if (not w.worth() or rows.alpha_group is not None
-                or (rows.alpha is not None and rows.alpha_row)):
-            return None
         oh, ow = (w.wh - 1) * sh + kh, (w.ww - 1) * sw + kw
-        parts = _conv_split_parts(p, st)
-        if parts is None or not _lib.load().vc_backward_conv_split_ok(
-                C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0):
+        if (not w.worth() or rows.alpha_group is not None
+                or (rows.alpha is not None and rows.alpha_row)
+                or B * R * C_in * oh * ow >= 1 << 31):
             return None
-        ls = us = ut = None
+        ls = us = ut = beta = None
         if rows.relu is not None:
             ls, us, ut = slopes(rows)
+            beta = rows.beta
         elif not rows.shared:
             per_domain_acc()
         M = R if rows.shared and rows.relu is None else B * R
+        rel = torch.empty(M, C_out * w.wh * w.ww, device=dev)
+        call('vc_patch_relax', ptr(rows.ew), M, R, 1 if rows.shared else 0, ptr(ls), ptr(us),
+             ptr(ut), ptr(beta), ptr(w.origin), C_out, w.H, w.W, w.wh, w.ww, ptr(rel), ptr(acc),
+             st)
         out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
                     and rows.relu is None)
-        call('vc_backward_conv_split', ptr(rows.ew), M, R, 1 if rows.shared else 0, ptr(ls),
-             ptr(us), ptr(ut), ptr(rows.beta) if rows.relu is not None else None, ptr(p['K']),
-             ptr(parts), ptr(p['b']), C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0,
-             ptr(w.origin), w.H, w.W, ptr(out.ew), ptr(acc), st)
+        call('vc_backward_conv_packed', ptr(rel), M, ptr(p['K']), ptr(_conv_t_taps(p, st, True)),
+             ptr(p['b']), C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0, ptr(out.ew),
+             ptr(acc), st)
         origin = torch.empty_like(w.origin)
         call('vc_patch_shift', ptr(w.origin), R, sh, sw, ph, pw, ptr(origin), st)
         out.window = _Window(origin, oh, ow, C_in, H, W)
@@ -759,7 +767,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
             return None
         fold = few_channels(p)
-        parts = None if fold else _conv_split_parts(p, st)
+        parts = None if fold or not split else _conv_split_parts(p, st)
         if not fold and parts is None:
             return None
         ls, us, ut = slopes(rows)
@@ -768,8 +776,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         if parts is not None:
             call('vc_backward_conv_split', ptr(rows.ew), B * R, R, 1 if rows.shared else 0,
                  ptr(ls), ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(parts), ptr(p['b']),
-                 C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, None, Ho, Wo, ptr(out),
-                 ptr(acc), st)
+                 C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
             return out
         call('vc_backward_relu_conv', ptr(rows.ew), B * R, R, 1 if rows.shared else 0, ptr(ls),
              ptr(us), ptr(ut), ptr(rows.beta), ptr(p['K']), ptr(p['b']), C_out, Ho, Wo, C_in,
@@ -922,11 +929,11 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 per_domain_acc()
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
-            parts = None if few_channels(p) else _conv_split_parts(p, st)
+            parts = None if not split or few_channels(p) else _conv_split_parts(p, st)
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
                      ptr(p['K']), ptr(parts), ptr(p['b']), C_out, Ho, Wo, C_in, H, W, kh, kw,
-                     sh, sw, ph, pw, None, Ho, Wo, ptr(out), ptr(acc), st)
+                     sh, sw, ph, pw, ptr(out), ptr(acc), st)
                 put(inp, _Rows(out, rows.shared))
                 continue
             call('vc_backward_conv_packed', ptr(rows.ew), M, ptr(p['K']),
@@ -1119,7 +1126,8 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
                      Ho, Wo, C_in, kh, kw, sh, sw, ph, pw, ptr(rows.ew), ptr(origin), ptr(acc0),
                      st)
                 rows.window = _Window(origin, kh, kw, C_in, H, W)
-                sl, _, _, _ = _backward(tight, xl, xh, gg, below, rows, True, acc0)
+                sl, _, _, _ = _backward(tight, xl, xh, gg, below, rows, True, acc0,
+                                        split=False)
                 call('vc_crown_intersect', ptr(sl.contiguous()), ptr(cidx), k, B, n,
                      ptr(new_lo), ptr(new_hi), st)
                 continue
@@ -1128,7 +1136,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
             seed[ar, cidx.long()] = 1.0
             seed[ar + k, cidx.long()] = -1.0
             acc0 = torch.zeros(2 * k, device=dev)
-            sl, _, _, _ = _backward(tight, xl, xh, gg, feed, seed, True, acc0)
+            sl, _, _, _ = _backward(tight, xl, xh, gg, feed, seed, True, acc0, split=False)
             sl = sl.contiguous()
             call('vc_crown_intersect', ptr(sl), ptr(cidx), k, B, n,
                  ptr(new_lo), ptr(new_hi), st)
