@@ -233,6 +233,31 @@ int vc_relax_slopes(const float *relu_lo, const float *relu_hi,
                     const float *alpha, int64_t n, float *lo_s, float *up_s,
                     float *up_t, vc_stream_t stream);
 
+/* The fc products on the bf16 matrix cores, each fp32 value and weight as three
+ * bf16 parts (at least the accuracy of the fp32 products), after a pass that
+ * forms the rows' parts in work (vc_fc_split_pack_bytes(K, M) of them, 16-byte
+ * aligned).  Slopes (M / R, K) as from vc_relax_slopes; packed: W's parts from
+ * vc_fc_split_pack (vc_fc_split_pack_bytes(K, N), 16-byte aligned), of W (K, N)
+ * or with trans of W (N, K) whose transpose is meant.  M < 2^31.
+ * vc_backward_fc_split: e = pos(x) lo_s + neg(x) up_s [+ beta (M / R, n_out)],
+ *   ew_out (M, n_in) = e W, acc[m] += neg(x) . up_t + e . bias, x from row m or,
+ *   with ew_shared, row m mod R.  Replaces verify_zono_bnb.py:4379-4453.
+ * vc_alpha_grad_step_split, vc_alpha_grad_input_split: as
+ *   vc_alpha_grad_step_slopes and vc_alpha_grad_input, with the packed transpose. */
+int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N);
+int vc_fc_split_pack(const float *W, int K, int N, int trans, void *out, vc_stream_t stream);
+int vc_backward_fc_split(const float *ew_in, int64_t M, int R, int ew_shared, int n_out,
+                         const float *lo_s, const float *up_s, const float *up_t,
+                         const float *beta, const void *packed, const float *bias, int n_in,
+                         float *ew_out, float *acc, void *work, vc_stream_t stream);
+int vc_alpha_grad_step_split(const float *gE, const float *P, int64_t M, int R, int n,
+                             const float *lo_s, const float *up_s, const float *up_t,
+                             int p_shared, const void *packed_t, const float *bias_next,
+                             int n_next, float *g_out, void *work, vc_stream_t stream);
+int vc_alpha_grad_input_split(const float *A, const float *xl, const float *xh, int64_t M,
+                              int R, int n_in, const void *packed_t, const float *bias0, int n1,
+                              float *g_out, void *work, vc_stream_t stream);
+
 /* relu backward step alone (for a relu that is not fed by an fc):
  * ew_out (M, n) = relaxed rows, acc += neg(ew) . up_t.  Same arguments as
  * the relu part of vc_backward_fc.  Replaces verify_zono_bnb.py:4409-4453. */

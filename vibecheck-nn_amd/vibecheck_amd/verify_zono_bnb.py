@@ -217,6 +217,33 @@ def _conv_split_parts(p, st):
     return p['KS']
 
 
+def _fc_split_parts(p, M, st, trans=False, sweep=False):
+    """The fc weights' bf16 parts for M rows' vc_backward_fc_split (``trans``:
+    for the gradient's products with W^T), made on first use and cached with
+    the op's other device tensors; None where the fp32 product is the faster
+    one.  ``sweep``: a gradient sweep follows that uses the backward's slopes."""
+    K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
+    if trans:
+        ok = M >= _FC_SPLIT_SWEEP_ROWS and min(K, N) >= _FC_SPLIT_WIDTH
+    else:
+        ok = (M >= (_FC_SPLIT_SWEEP_ROWS if sweep else _FC_SPLIT_ROWS)
+              and K >= _TWO_PHASE_MIN_WIDTH and max(K, N) >= _FC_SPLIT_WIDTH)
+    if not ok or M >= 1 << 31:
+        return None
+    key, version = 'WST' if trans else 'WS', p['W']._version  # W may be the caller's own
+    if key not in p or p[key][0] != version:
+        parts = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, N), dtype=torch.uint8,
+                            device=p['W'].device)
+        call('vc_fc_split_pack', ptr(p['W']), K, N, 1 if trans else 0, ptr(parts), st)
+        p[key] = (version, parts)
+    return p[key][1]
+
+
+def _fc_split_work(M, K, dev):
+    """The buffer of M rows' parts that a vc_fc_split product forms first."""
+    return torch.empty(_lib.load().vc_fc_split_pack_bytes(K, M), dtype=torch.uint8, device=dev)
+
+
 def _pair(v):
     if isinstance(v, int):
         return v, v
@@ -590,11 +617,13 @@ class _Window:
 class BackwardTrace:
     """Per-relu stored pre-relaxation rows of one backward, for the alpha
     gradient sweep: entries (L, P, p_shared) in backward order.  ``other``
-    names an op the sweep does not replay (add, sub, mul, a fan-in)."""
+    names an op the sweep does not replay (add, sub, mul, a fan-in); ``slopes``
+    holds the layers' slopes where the backward had to form them."""
 
     def __init__(self):
         self.relus = []
         self.fcs = []
+        self.slopes = {}
         self.other = None
 
 
@@ -602,6 +631,17 @@ class BackwardTrace:
 # width up when given a relaxed-rows buffer (measured 2x faster on 1024-wide
 # layers than relaxing inside the GEMM's loads).
 _TWO_PHASE_MIN_WIDTH = 64
+
+# Products of bf16 parts, against the fp32 ones (us, slopes included): 256 x 256
+# at 1,152 rows 16 and 16, at 18,432 90 -> 46; 1024 x 1024 at 288 rows 20 -> 32,
+# at 4,608 130 -> 94.  The gradient's, whose fp32 product sums in 64 bits: 256 x
+# 256 at 9 rows 16 -> 9, 1024 x 1024 at 288 rows 52 -> 25; its gain outweighs the
+# backward's loss on few rows.  Narrow ones do not pay for the pass that forms
+# the parts: 64 x 64 at 73,728 rows 35 -> 46, the gradient's 25 -> 41 (128 x 16:
+# 34 -> 56, 203 x 117: 135 -> 131).
+_FC_SPLIT_ROWS = 2048
+_FC_SPLIT_SWEEP_ROWS = 64
+_FC_SPLIT_WIDTH = 128
 
 
 def _expand_rows(t, B):
@@ -725,6 +765,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         out = [torch.empty(B, n, device=dev) for _ in range(3)]
         call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(rows.alpha), B * n, ptr(out[0]),
              ptr(out[1]), ptr(out[2]), st)
+        if trace is not None:
+            trace.slopes[rows.relu] = out
         return out
 
     def window_conv(rows, p):
@@ -845,10 +887,24 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             p = _op_params(op, dev)
             if rows.relu is not None:
                 L = rows.relu
-                lo, hi = f32(tight[L][0]), f32(tight[L][1])
-                per_domain_acc()
                 M = B * R
                 out = torch.empty(M, p['n_in'], device=dev)
+                parts = None
+                if split and rows.alpha_group is None and not rows.alpha_row:
+                    parts = _fc_split_parts(p, M, st, sweep=trace is not None)
+                if parts is not None:
+                    ls, us, ut = slopes(rows)
+                    work = _fc_split_work(M, p['n_out'], dev)
+                    if trace is not None:
+                        trace.fcs.append(op)
+                    call('vc_backward_fc_split', ptr(rows.ew), M, R, 1 if rows.shared else 0,
+                         p['n_out'], ptr(ls), ptr(us), ptr(ut), ptr(rows.beta),
+                         ptr(parts), ptr(p['b']), p['n_in'], ptr(out), ptr(acc),
+                         ptr(work), st)
+                    put(inp, _Rows(out, False))
+                    continue
+                lo, hi = f32(tight[L][0]), f32(tight[L][1])
+                per_domain_acc()
                 if trace is not None:
                     trace.relus.append((L, rows.ew, rows.shared))
                     trace.fcs.append(op)
@@ -1189,8 +1245,14 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
     # input side: gE_0 = gA W_0^T + b_0, W_0 = fcs[-1]
     f0 = _op_params(fcs[-1], dev)
     g = torch.empty(M, f0['n_out'], device=dev)
-    call('vc_alpha_grad_input', ptr(A), ptr(xl), ptr(xh), M, Q, n_in,
-         ptr(f0['W']), ptr(f0['b']), f0['n_out'], ptr(g), st)
+    parts = _fc_split_parts(f0, M, st, True)
+    if parts is not None:
+        work = _fc_split_work(M, n_in, dev)
+        call('vc_alpha_grad_input_split', ptr(A), ptr(xl), ptr(xh), M, Q, n_in, ptr(parts),
+             ptr(f0['b']), f0['n_out'], ptr(g), ptr(work), st)
+    else:
+        call('vc_alpha_grad_input', ptr(A), ptr(xl), ptr(xh), M, Q, n_in,
+             ptr(f0['W']), ptr(f0['b']), f0['n_out'], ptr(g), st)
     for i in range(len(relus) - 1, -1, -1):
         L, P, p_shared = relus[i]
         lo, hi = f32(sb[L][0]), f32(sb[L][1])
@@ -1222,12 +1284,22 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
             g2 = torch.empty(M, fn['n_out'], device=dev)
             # slopes once per (domain, neuron), then the sweep step without
             # a per-element division
-            ls, us, ut = (torch.empty(B, n, device=dev) for _ in range(3))
-            call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(a), B * n, ptr(ls),
-                 ptr(us), ptr(ut), st)
-            call('vc_alpha_grad_step_slopes', ptr(g), ptr(P), M, Q, n,
-                 ptr(ls), ptr(us), ptr(ut), 1 if p_shared else 0,
-                 ptr(fn['W']), ptr(fn['b']), fn['n_out'], ptr(g2), st)
+            if L in trace.slopes:
+                ls, us, ut = trace.slopes[L]
+            else:
+                ls, us, ut = (torch.empty(B, n, device=dev) for _ in range(3))
+                call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(a), B * n, ptr(ls),
+                     ptr(us), ptr(ut), st)
+            parts = _fc_split_parts(fn, M, st, True)
+            if parts is not None:
+                work = _fc_split_work(M, n, dev)
+                call('vc_alpha_grad_step_split', ptr(g), ptr(P), M, Q, n, ptr(ls), ptr(us),
+                     ptr(ut), 1 if p_shared else 0, ptr(parts), ptr(fn['b']), fn['n_out'],
+                     ptr(g2), ptr(work), st)
+            else:
+                call('vc_alpha_grad_step_slopes', ptr(g), ptr(P), M, Q, n,
+                     ptr(ls), ptr(us), ptr(ut), 1 if p_shared else 0,
+                     ptr(fn['W']), ptr(fn['b']), fn['n_out'], ptr(g2), st)
             g = g2
     return (lb, A) if want_A else lb
 
