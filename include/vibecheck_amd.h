@@ -258,6 +258,30 @@ int vc_alpha_grad_input_split(const float *A, const float *xl, const float *xh, 
                               int R, int n_in, const void *packed_t, const float *bias0, int n1,
                               float *g_out, void *work, vc_stream_t stream);
 
+/* The zonotope relu and the fc after it, taken together.  The relu's slope
+ * scales the generators' rows, and its new generators are one neuron's each, so
+ * through the fc they are scaled columns of W.
+ * vc_zono_relu_lists: lam (B, n) and c_out (B, n) as vc_zono_relu_apply, and
+ *   domain b's new generators in order of their rank, neuron idx[b k_new + j] and
+ *   size mu[b k_new + j].
+ * vc_zono_fc_split: G_out[b][o][j] = sum over k of W[o][k] lam[b][k] G[b][k][j]
+ *   for the K old columns, rows of G_out ld apart, on the bf16 matrix cores
+ *   (packed_t: W's parts, vc_fc_split_pack with trans).  work: any multiple of
+ *   vc_fc_split_pack_bytes(n, K), 16-byte aligned; as many domains at a time.
+ * vc_zono_fc_cols: G_out[b][o][k0 + j] = W[o][idx[b idx_ld + j]] mu[same] for
+ *   j < cnt[b] (NULL: k), zero for the others up to k; mu NULL: the sizes are
+ *   (xh - xl) / 2 of neuron idx (the input's generators).
+ * Replaces verify_zono_bnb.py:3120-3211. */
+int vc_zono_relu_lists(const float *c, const float *lo, const float *hi, const int32_t *rank,
+                       int64_t B, int n, int k_new, float *c_out, float *lam, int32_t *idx,
+                       float *mu, vc_stream_t stream);
+int vc_zono_fc_split(const float *G, const float *lam, int64_t B, int n, int K,
+                     const void *packed_t, int n_out, int64_t ld, float *G_out, void *work,
+                     int64_t work_bytes, vc_stream_t stream);
+int vc_zono_fc_cols(const float *W, int n_out, int n, int64_t B, int k, const int32_t *idx,
+                    int64_t idx_ld, const float *mu, const float *xl, const float *xh,
+                    const int32_t *cnt, int k0, int64_t ld, float *G_out, vc_stream_t stream);
+
 /* relu backward step alone (for a relu that is not fed by an fc):
  * ew_out (M, n) = relaxed rows, acc += neg(ew) . up_t.  Same arguments as
  * the relu part of vc_backward_fc.  Replaces verify_zono_bnb.py:4409-4453. */

@@ -194,11 +194,13 @@ __global__ __launch_bounds__(FNT) void k_fc_rows(RowArgs a) {
 struct GemmArgs {
   const uint4 *Ap, *Bp;
   const float* bias;  // (N) or null
-  float* out;         // (M, N)
-  int64_t M;
-  int N, nkc, ntn, mt16;
+  float* out;         // (M, N); domains: (domains, N, ld), M of its columns
+  int64_t M;          // rows; domains: of each
+  int N, nkc, ntn, mt16;  // mt16: row tiles; domains: of each
   int64_t tiles;
   FastDiv f_ntn;
+  int64_t ld;
+  FastDiv f_dom;  // domains: row blocks of each
 };
 
 // Value j of lane's eight in a packed tile: the sum of its three parts.
@@ -210,9 +212,9 @@ __device__ float part_sum(const uint4* p, int j) {
   return s;
 }
 
-// One output as the plain sum in 64 bits.
-__device__ float plain_sum(const GemmArgs& a, int64_t m, int n) {
-  const uint4* A = a.Ap + (m >> 4) * a.nkc * kTileU + (m & 15);
+// One output, row r of row tile t, as the plain sum in 64 bits.
+__device__ float plain_sum(const GemmArgs& a, int64_t t, int r, int n) {
+  const uint4* A = a.Ap + t * a.nkc * kTileU + r;
   const uint4* B = a.Bp + (int64_t)(n >> 4) * a.nkc * kTileU + (n & 15);
   double s = 0.0;
   for (int kc = 0; kc < a.nkc; ++kc)
@@ -223,7 +225,8 @@ __device__ float plain_sum(const GemmArgs& a, int64_t m, int n) {
   return (float)s;
 }
 
-template <int MT>
+// DOM: the rows are those of many domains, each stored transposed.
+template <int MT, bool DOM>
 __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
   constexpr int AU = MT * 2 * kTileU;       // 16-byte units of a double step's rows
   constexpr int NL = (AU + FNT - 1) / FNT;  // of them per thread
@@ -233,8 +236,11 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t w = vcg::xcd_tile(blockIdx.x, a.tiles);
-  const int tm = (int)a.f_ntn.div((uint32_t)w);
-  const int tn = (int)(w - (int64_t)tm * a.ntn);
+  const int tb = (int)a.f_ntn.div((uint32_t)w);
+  const int tn = (int)(w - (int64_t)tb * a.ntn);
+  const int dom = DOM ? (int)a.f_dom.div((uint32_t)tb) : 0;
+  const int tm = DOM ? tb - dom * (int)a.f_dom.d : tb;
+  const int64_t t0 = DOM ? (int64_t)dom * a.mt16 : 0;  // the domain's first row tile
 
   // this thread's units of each double step's rows (a row tile's two steps lie
   // together); past the last row tile the last one again, not stored
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
   for (int i = 0; i < NL; ++i) {
     const int u = min(tid + i * FNT, AU - 1);
     const int t = min(tm * MT + u / (2 * kTileU), a.mt16 - 1);
-    A[i] = reinterpret_cast<const u4*>(a.Ap) + (int64_t)t * a.nkc * kTileU + u % (2 * kTileU);
+    A[i] = reinterpret_cast<const u4*>(a.Ap) + (t0 + t) * a.nkc * kTileU + u % (2 * kTileU);
   }
   // this wave's two column tiles, likewise
   const int c0 = tn * 8 + wv * 2, nt16 = (a.N + 15) >> 4;
@@ -279,13 +285,12 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < NL; ++i) lds[0][tid + i * FNT] = rn[i];
 
-#pragma unroll 1
-  for (int s = 0; s < steps; ++s) {
+  const auto step = [&](int s, int buf) {
     __syncthreads();  // this step's rows are laid down, the ones before are read
     load_cols(2 * s + 1, b[1]);
     load_rows(s + 1, rn);
     __builtin_amdgcn_sched_barrier(0);  // requested before the products, not where they are used
-    const u4* from = lds[s & 1] + lane;
+    const u4* from = lds[buf] + lane;
     u4 av[2][Q][3];
     const auto read = [&](int t, u4(&v)[Q][3]) {  // half t / NG, row tiles Q (t mod NG) ..
 #pragma unroll
@@ -328,7 +333,15 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < NL; ++i) lds[(s & 1) ^ 1][tid + i * FNT] = rn[i];
+    for (int i = 0; i < NL; ++i) lds[buf ^ 1][tid + i * FNT] = rn[i];
+  };
+  // two at a time: one's sums would be copied back at the loop's end
+#pragma unroll 1
+  for (int s = 0;; s += 2) {
+    step(s, 0);
+    if (s + 1 == steps) break;
+    step(s + 1, 1);
+    if (s + 2 == steps) break;
   }
 
   const int g = lane >> 4, r = lane & 15;
@@ -338,16 +351,124 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
     if (n >= a.N) continue;
     const float b = a.bias ? a.bias[n] : 0.f;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i) {
+      const int64_t m0 = (int64_t)tm * MT * 16 + 16 * i + 4 * g;
+      float v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t m = (int64_t)tm * MT * 16 + 16 * i + 4 * g + q;
-        if (m >= a.M) continue;
-        float v = acc[i][j][q] + small[i][j][q];
+        v[q] = acc[i][j][q] + small[i][j][q];
         // an infinity or NaN among the values: the plain sum
-        if (!finite(v)) v = plain_sum(a, m, n);
-        a.out[m * a.N + n] = a.bias ? v + b : v;
+        if (!finite(v[q]) && m0 + q < a.M)
+          v[q] = plain_sum(a, t0 + tm * MT + i, 4 * g + q, n);
+        if (a.bias) v[q] = v[q] + b;
       }
+      if (DOM) {
+        float* o = a.out + ((int64_t)dom * a.N + n) * a.ld + m0;
+        if (m0 + 4 <= a.M) {
+          typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+          *reinterpret_cast<v4u*>(o) = v4u{v[0], v[1], v[2], v[3]};
+          continue;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (m0 + q < a.M) o[q] = v[q];
+        continue;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (m0 + q < a.M) a.out[(m0 + q) * a.N + n] = v[q];
+    }
+  }
+}
+
+// The zonotope's relu and the fc after it (verify_zono_bnb.py:3120-3211): the
+// relu's slope scales the generators' rows, here in the pass that forms their
+// parts, and its new generators are one neuron's each, so through the fc they
+// are scaled columns of W and need no product.  784-1024x4-10, 512 boxes: the
+// relu's pass over (B, n, K) and the fp32 product of all columns 83 ms, now 37
+// (28 of them k_fc_gemm, at 150 TFLOP/s); 784-256x6-10, 64 boxes, the whole
+// forward 1.76 -> 1.25 ms.
+//
+// Parts of the generators as rows: row = generator column j of domain b, its
+// values G[b][k][j] lam[b][k] over the neurons k.  Four waves take 64 columns,
+// each 16 of them: 256 bytes of a neuron's row at a time.
+__global__ __launch_bounds__(FNT) void k_zono_rows(const float* G, const float* lam, int n, int K,
+                                                   int mt16, int nkc, FastDiv f_blk,
+                                                   uint4* parts) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
+  const int64_t dom = f_blk.div((uint32_t)blockIdx.x);
+  const int t = ((int)(blockIdx.x - dom * f_blk.d)) * 4 + wv;
+  if (t >= mt16) return;
+  const float* x = G + dom * n * (int64_t)K + min(16 * t + r, K - 1);
+  const float* l = lam ? lam + dom * n : nullptr;
+  uint4* out = parts + (dom * mt16 + t) * nkc * kTileU + lane;
+  for (int kc = blockIdx.y; kc < nkc; kc += gridDim.y) {
+    const int k0 = kc * FBK + 8 * g;
+    float e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = min(k0 + j, n - 1);
+      e[j] = x[(int64_t)k * K];
+      if (l) e[j] = e[j] * l[k];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) e[j] = k0 + j < n ? e[j] : 0.f;
+    uint4 h, m, lo;
+    split8_all(e, h, m, lo);
+    uint4* const o = out + (int64_t)kc * kTileU;
+    o[0] = h;
+    o[64] = m;
+    o[128] = lo;
+  }
+}
+
+// A zonotope relu's slope and centre per neuron, and its new generators as a
+// list per domain: neuron and size of each, in order (the operations of
+// vc_zono_relu_apply).
+__global__ void k_zono_lists(const float* c, const float* lo, const float* hi,
+                             const int32_t* rank, int64_t rows, int n, int k_new, float* c_out,
+                             float* lam_out, int32_t* idx, float* mu_out) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < rows;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const float l = lo[i], h = hi[i];
+    const bool ust = l < 0.f && h > 0.f;
+    const float lam = ust ? h / (h - l) : (h <= 0.f ? 0.f : 1.f);
+    const float mu = ust ? (-h * l) / (2.f * (h - l)) : 0.f;
+    lam_out[i] = lam;
+    c_out[i] = lam * c[i] + mu;
+    if (ust) {
+      const int64_t b = i / n, o = b * k_new + rank[i];
+      idx[o] = (int)(i - b * n);
+      mu_out[o] = mu;
+    }
+  }
+}
+
+// Generators that are one neuron's, through an fc: scaled columns of W.
+// G_out[b][o][k0 + j] = W[o][idx[j]] mu[j] for j < cnt[b], else zero.
+constexpr int kColRows = 16;
+__global__ __launch_bounds__(FNT) void k_zono_cols(const float* W, int n_out, int n, int k,
+                                                   const int32_t* idx, int64_t idx_ld,
+                                                   const float* mu, const float* xl,
+                                                   const float* xh, const int32_t* cnt,
+                                                   int64_t blocks, FastDiv f_j, FastDiv f_o,
+                                                   float* out, int64_t ld) {
+  for (int64_t blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+    const uint32_t q = f_j.div((uint32_t)blk);
+    const int64_t b = f_o.div(q);
+    const int j = (int)(blk - (int64_t)q * f_j.d) * FNT + threadIdx.x;
+    const int o0 = (int)(q - b * f_o.d) * kColRows;
+    if (j >= k) continue;
+    int i = 0;
+    float m = 0.f;
+    if (!cnt || j < cnt[b]) {
+      i = idx[b * idx_ld + j];
+      m = mu ? mu[b * idx_ld + j] : (xh[b * n + i] - xl[b * n + i]) / 2.f;
+    }
+    const bool has = !cnt || j < cnt[b];
+    float* o = out + (b * n_out + o0) * ld + j;
+    for (int r = 0; r < kColRows && o0 + r < n_out; ++r)
+      o[r * ld] = has ? W[(int64_t)(o0 + r) * n + i] * m : 0.f;
   }
 }
 
@@ -392,11 +513,14 @@ int launch_fc(RowArgs a, const void* packed, int N, const float* bias, float* ou
   b.mt16 = (int)mt16;
   b.ntn = (N + FBN - 1) / FBN;
   b.f_ntn = FastDiv::make((uint32_t)b.ntn);
-  // the tallest row block that still gives every CU a tile
+  // The tallest row block that gives every CU a tile, or four of them: two fit
+  // a CU, and a third round half empty costs more than the weights read twice
+  // (64 and 32 rows: 4,608 x 1024 x 1024, 576 tiles, 84 and 78 us, 18,432 x 256 x
+  // 256 38 and 34; 18,432 x 1024 x 1024, 2,304 tiles, 251 and 276).
   const int64_t cus = vcm::cu_count();
-  int mt = 4;
-  while (mt > 1 && (mt16 + mt - 1) / mt * b.ntn < cus) mt >>= 1;
-  b.tiles = (mt16 + mt - 1) / mt * b.ntn;
+  const auto blocks = [&](int mt) { return (mt16 + mt - 1) / mt * b.ntn; };
+  const int mt = blocks(4) >= 4 * cus ? 4 : (blocks(2) >= cus ? 2 : 1);
+  b.tiles = blocks(mt);
   if (a.M >= (int64_t(1) << 31) || b.tiles >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
   bool vec = a.K % 4 == 0;
   for (const float* p : {a.x, a.P, a.s0, a.s1, a.s2, a.beta, a.bias}) vec = vec && aligned16(p);
@@ -406,9 +530,9 @@ int launch_fc(RowArgs a, const void* packed, int N, const float* bias, float* ou
     hipLaunchKernelGGL((k_fc_rows<FORM, false>), dim3((unsigned)mt16), dim3(FNT), 0, st, a);
   VC_LAUNCH_CHECK();
   const dim3 grid((unsigned)b.tiles);
-  if (mt == 4) hipLaunchKernelGGL(k_fc_gemm<4>, grid, dim3(FNT), 0, st, b);
-  if (mt == 2) hipLaunchKernelGGL(k_fc_gemm<2>, grid, dim3(FNT), 0, st, b);
-  if (mt == 1) hipLaunchKernelGGL(k_fc_gemm<1>, grid, dim3(FNT), 0, st, b);
+  if (mt == 4) hipLaunchKernelGGL((k_fc_gemm<4, false>), grid, dim3(FNT), 0, st, b);
+  if (mt == 2) hipLaunchKernelGGL((k_fc_gemm<2, false>), grid, dim3(FNT), 0, st, b);
+  if (mt == 1) hipLaunchKernelGGL((k_fc_gemm<1, false>), grid, dim3(FNT), 0, st, b);
   VC_LAUNCH_CHECK();
   return VC_OK;
 }
@@ -495,4 +619,74 @@ extern "C" int vc_alpha_grad_input_split(const float* A, const float* xl, const 
   a.R = R;
   a.K = n_in;
   return launch_fc<kGradInput>(a, packed_t, n1, bias0, g_out, (hipStream_t)stream);
+}
+
+extern "C" int vc_zono_relu_lists(const float* c, const float* lo, const float* hi,
+                                  const int32_t* rank, int64_t B, int n, int k_new, float* c_out,
+                                  float* lam, int32_t* idx, float* mu, vc_stream_t stream) {
+  if (!c || !lo || !hi || !rank || !c_out || !lam || B < 0 || n <= 0 || k_new < 0 ||
+      (k_new > 0 && (!idx || !mu)))
+    return VC_ERR_ARG;
+  if (B == 0) return VC_OK;
+  hipLaunchKernelGGL(k_zono_lists, dim3(vc_blocks(B * n, FNT)), dim3(FNT), 0, (hipStream_t)stream,
+                     c, lo, hi, rank, B * n, n, k_new, c_out, lam, idx, mu);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_zono_fc_cols(const float* W, int n_out, int n, int64_t B, int k,
+                               const int32_t* idx, int64_t idx_ld, const float* mu,
+                               const float* xl, const float* xh, const int32_t* cnt, int k0,
+                               int64_t ld, float* G_out, vc_stream_t stream) {
+  if (B < 0 || n <= 0 || n_out <= 0 || k < 0 || k0 < 0 || ld < (int64_t)k0 + k) return VC_ERR_ARG;
+  if (B == 0 || k == 0) return VC_OK;
+  if (!W || !idx || !G_out || (!mu && (!xl || !xh))) return VC_ERR_ARG;
+  const int nj = (k + FNT - 1) / FNT, no = (n_out + kColRows - 1) / kColRows;
+  const int64_t blocks = B * nj * no;
+  if (blocks >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(k_zono_cols, dim3((unsigned)blocks), dim3(FNT), 0, (hipStream_t)stream, W,
+                     n_out, n, k, idx, idx_ld, mu, xl, xh, cnt, blocks, FastDiv::make(nj),
+                     FastDiv::make(no), G_out + k0, ld);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
+}
+
+extern "C" int vc_zono_fc_split(const float* G, const float* lam, int64_t B, int n, int K,
+                                const void* packed_t, int n_out, int64_t ld, float* G_out,
+                                void* work, int64_t work_bytes, vc_stream_t stream) {
+  if (B < 0 || n <= 0 || n_out <= 0 || K < 0 || ld < K) return VC_ERR_ARG;
+  if (B == 0 || K == 0) return VC_OK;
+  if (!G || !packed_t || !G_out || !work || !aligned16(packed_t) || !aligned16(work))
+    return VC_ERR_ARG;
+  const int64_t per = vc_fc_split_pack_bytes(n, K);
+  const hipStream_t st = (hipStream_t)stream;
+  GemmArgs b{};
+  b.nkc = 2 * ((n + 2 * FBK - 1) / (2 * FBK));
+  b.Ap = (const uint4*)work;
+  b.Bp = (const uint4*)packed_t;
+  b.M = K;
+  b.N = n_out;
+  b.ld = ld;
+  b.mt16 = (K + 15) / 16;
+  b.ntn = (n_out + FBN - 1) / FBN;
+  b.f_ntn = FastDiv::make((uint32_t)b.ntn);
+  const int blk = (b.mt16 + 3) / 4, ny = b.nkc < 4 ? b.nkc : 4;
+  b.f_dom = FastDiv::make((uint32_t)blk);
+  // domains whose parts the buffer holds, and whose tiles a launch counts
+  int64_t step = work_bytes / per;
+  const int64_t most = (((int64_t)1 << 31) - 1) / ((int64_t)blk * b.ntn);
+  if (step > most) step = most;
+  if (step < 1) return VC_ERR_ARG;
+  for (int64_t b0 = 0; b0 < B; b0 += step) {
+    const int64_t cnt = B - b0 < step ? B - b0 : step;
+    hipLaunchKernelGGL(k_zono_rows, dim3((unsigned)(cnt * blk), ny), dim3(FNT), 0, st,
+                       G + b0 * n * K, lam ? lam + b0 * n : nullptr, n, K, b.mt16, b.nkc, b.f_dom,
+                       (uint4*)work);
+    VC_LAUNCH_CHECK();
+    b.out = G_out + b0 * n_out * ld;
+    b.tiles = cnt * blk * b.ntn;
+    hipLaunchKernelGGL((k_fc_gemm<4, true>), dim3((unsigned)b.tiles), dim3(FNT), 0, st, b);
+    VC_LAUNCH_CHECK();
+  }
+  return VC_OK;
 }

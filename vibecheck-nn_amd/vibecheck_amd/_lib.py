@@ -68,6 +68,9 @@ SIGNATURES = {
     'vc_backward_fc_split': [_P, _L, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P],
     'vc_alpha_grad_step_split': [_P, _P, _L, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _P],
     'vc_alpha_grad_input_split': [_P, _P, _P, _L, _I, _I, _P, _P, _I, _P, _P, _P],
+    'vc_zono_relu_lists': [_P, _P, _P, _P, _L, _I, _I, _P, _P, _P, _P, _P],
+    'vc_zono_fc_split': [_P, _P, _L, _I, _I, _P, _I, _L, _P, _P, _L, _P],
+    'vc_zono_fc_cols': [_P, _I, _I, _L, _I, _P, _L, _P, _P, _P, _P, _I, _L, _P, _P],
     'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     'vc_patch_shift': [_P, _I, _I, _I, _I, _I, _P, _P],
     'vc_patch_relax': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P],

@@ -39,7 +39,7 @@ def _zono_sb(gg, xl, xh, device, dtype):
             plan, xl, xh,
             lambda a, b: _forward_zonotope_graph_batched(a, b, gg, device, dtype)[0])
         return sb
-    return _forward_zonotope_graph_batched(xl, xh, gg, device, dtype)[0]
+    return _zono_forward(xl, xh, gg, dtype, True)[0]
 
 
 def _check_dtype(dtype):
@@ -230,6 +230,11 @@ def _fc_split_parts(p, M, st, trans=False, sweep=False):
               and K >= _TWO_PHASE_MIN_WIDTH and max(K, N) >= _FC_SPLIT_WIDTH)
     if not ok or M >= 1 << 31:
         return None
+    return _fc_parts(p, st, trans)
+
+
+def _fc_parts(p, st, trans=False):
+    K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
     key, version = 'WST' if trans else 'WS', p['W']._version  # W may be the caller's own
     if key not in p or p[key][0] != version:
         parts = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, N), dtype=torch.uint8,
@@ -469,6 +474,41 @@ def _forward_zonotope_graph_batched(xl, xh, gg, device, dtype):
     (The (c, G) output needs the layer-wise kernels; bound-only callers use
     the fused kernel through _zono_sb.)
     """
+    sb, out = _zono_forward(xl, xh, gg, dtype, False)
+    _forward_zonotope_graph_batched.last_bilinear_op_bounds = {}
+    return sb, out
+
+
+class _Gens:
+    """Generators whose form a following fc uses: ``lists`` (idx, idx_ld, mu,
+    xl, xh, cnt, k) for columns that are one neuron's, after the columns ``G``
+    (B, n, K) scaled by ``lam`` (B, n); ``dense`` gives the (B, n, K + k) matrix."""
+    __slots__ = ('G', 'lam', 'lists', 'dense')
+
+    def __init__(self, G, lam, lists, dense):
+        self.G, self.lam, self.lists, self.dense = G, lam, lists, dense
+
+
+def _zono_fc(p, g, B, K, st):
+    """(B, n_out, K + k) generators of a _Gens through an fc."""
+    idx, idx_ld, mu, xl, xh, cnt, k = g.lists
+    n, n_out, dev = p['n_in'], p['n_out'], p['W'].device
+    out = torch.empty(B, n_out, K + k, device=dev)
+    if K:
+        parts = _fc_parts(p, st, True)
+        per = _lib.load().vc_fc_split_pack_bytes(n, K)
+        work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)), dtype=torch.uint8,
+                           device=dev)
+        call('vc_zono_fc_split', ptr(g.G), ptr(g.lam), B, n, K, ptr(parts), n_out, K + k,
+             ptr(out), ptr(work), work.numel(), st)
+    call('vc_zono_fc_cols', ptr(p['W']), n_out, n, B, k, ptr(idx), idx_ld, ptr(mu), ptr(xl),
+         ptr(xh), ptr(cnt), K, K + k, ptr(out), st)
+    return out
+
+
+def _zono_forward(xl, xh, gg, dtype, bounds_only):
+    """(sb, (c, G) of the last op); with ``bounds_only`` fc layers above the
+    last relu are left out and the second is None."""
     _check_dtype(dtype)
     xl, xh = f32(xl), f32(xh)
     B, n_in = xl.shape
@@ -479,18 +519,44 @@ def _forward_zonotope_graph_batched(xl, xh, gg, device, dtype):
         torch.zeros(n_in, dtype=torch.bool, device=dev)
     vidx = varying.nonzero(as_tuple=True)[0].to(torch.int32).contiguous()
     K = int(vidx.numel())
+    ops = gg['ops']
+    users = {}
+    for op in ops:
+        for i in op['inputs']:
+            users.setdefault(i, []).append(op)
+    top = max([i for i, op in enumerate(ops) if op['type'] == 'relu' and 'layer_idx' in op],
+              default=len(ops))
+    if not bounds_only or any(op['type'] not in ('fc', 'reshape') for op in ops[top + 1:]):
+        top = len(ops)
+
+    def one_fc(name):
+        """The fc that alone reads a node, in its plain form, or None."""
+        u = users.get(name, [])
+        if len(u) == 1 and u[0]['type'] == 'fc' and _fc_form(u[0], widths[name])[0] == 1:
+            return u[0]
+        return None
+
+    def input_dense():
+        G = torch.empty(B, n_in, K, device=dev)
+        call('vc_zono_input', ptr(xl), ptr(xh), B, n_in, ptr(vidx), K, ptr(c), ptr(G), st)
+        return G
+
     c = torch.empty(B, n_in, device=dev)
-    G = torch.empty(B, n_in, K, device=dev)
-    call('vc_zono_input', ptr(xl), ptr(xh), B, n_in, ptr(vidx), K, ptr(c),
-         ptr(G), st)
+    if one_fc(gg['input_name']) is not None and B > 0:
+        call('vc_zono_input', ptr(xl), ptr(xh), B, n_in, ptr(vidx), 0, ptr(c), None, st)
+        G = _Gens(None, None, (vidx, 0, None, xl, xh, None, K), input_dense)
+    else:
+        G = input_dense()
     state = {gg['input_name']: (c, G)}
     gen_count = {gg['input_name']: K}
     sb = {}
-    for op in gg['ops']:
+    for pos, op in enumerate(ops):
         t = op['type']
         name = op['name']
         c_in, G_in = state[op['inputs'][0]]
-        Kc = G_in.shape[2]
+        Kc = gen_count[op['inputs'][0]]
+        if isinstance(G_in, _Gens) and t != 'fc':
+            G_in = G_in.dense()
         n = c_in.shape[1]
         if t == 'add' and op.get('is_merge'):
             # residual merge: the fork point's generators are shared
@@ -532,6 +598,13 @@ def _forward_zonotope_graph_batched(xl, xh, gg, device, dtype):
             # generators are (B * P, n_in) and (B * P, n_in, K) as they lie
             P, _ = _fc_form(op, widths[op['inputs'][0]])
             c_o = torch.empty(B, P * p['n_out'], device=dev)
+            if isinstance(G_in, _Gens):
+                call('vc_zono_fc', ptr(c_in), None, B, p['n_in'], 0, ptr(p['W']), ptr(p['b']),
+                     p['n_out'], ptr(c_o), None, st)
+                k = G_in.lists[-1]
+                state[name] = (c_o, _zono_fc(p, G_in, B, Kc - k, st))
+                gen_count[name] = Kc
+                continue
             G_o = torch.empty(B, P * p['n_out'], Kc, device=dev)
             call('vc_zono_fc', ptr(c_in), ptr(G_in), B * P, p['n_in'], Kc,
                  ptr(p['W']), ptr(p['b']), p['n_out'], ptr(c_o), ptr(G_o), st)
@@ -553,21 +626,33 @@ def _forward_zonotope_graph_batched(xl, xh, gg, device, dtype):
             cnt = torch.empty(B, dtype=torch.int32, device=dev)
             call('vc_zono_relu_bounds', ptr(c_in), ptr(G_in), B, n, Kc,
                  ptr(lo), ptr(hi), ptr(rank), ptr(cnt), st)
-            k_new = int(cnt.max().item()) if B > 0 else 0
-            c_o = torch.empty(B, n, device=dev)
-            G_o = torch.empty(B, n, Kc + k_new, device=dev)
-            call('vc_zono_relu_apply', ptr(c_in), ptr(G_in), ptr(lo), ptr(hi),
-                 ptr(rank), B, n, Kc, k_new, ptr(c_o), ptr(G_o), st)
-            state[name] = (c_o, G_o)
             if 'layer_idx' in op:
                 sb[op['layer_idx']] = (lo, hi)
+            if pos == top:
+                return sb, None
+            k_new = int(cnt.max().item()) if B > 0 else 0
+            c_o = torch.empty(B, n, device=dev)
+            nxt = one_fc(name)
+            if nxt is not None and B * n * Kc * int(nxt['W'].shape[0]) >= _ZONO_SPLIT_MACS:
+                lam = torch.empty(B, n, device=dev)
+                idx = torch.empty(B, max(k_new, 1), dtype=torch.int32, device=dev)
+                mu = torch.empty(B, max(k_new, 1), device=dev)
+                call('vc_zono_relu_lists', ptr(c_in), ptr(lo), ptr(hi), ptr(rank), B, n, k_new,
+                     ptr(c_o), ptr(lam), ptr(idx), ptr(mu), st)
+                G_o = _Gens(G_in, lam, (idx, k_new, mu, None, None, cnt, k_new), None)
+            else:
+                G_o = torch.empty(B, n, Kc + k_new, device=dev)
+                call('vc_zono_relu_apply', ptr(c_in), ptr(G_in), ptr(lo), ptr(hi),
+                     ptr(rank), B, n, Kc, k_new, ptr(c_o), ptr(G_o), st)
+            state[name] = (c_o, G_o)
+            gen_count[name] = Kc + k_new
+            continue
         elif t == 'reshape':
             state[name] = (c_in, G_in)
         else:
             raise ValueError(f'batched zono forward: unknown op type {t!r}')
         gen_count[name] = state[name][1].shape[2]
-    _forward_zonotope_graph_batched.last_bilinear_op_bounds = {}
-    return sb, state[gg['ops'][-1]['name']]
+    return sb, state[ops[-1]['name']]
 
 
 # --------------------------------------------------------------------------
@@ -612,6 +697,15 @@ class _Window:
         """Windows up to half of the image are carried as such: beyond, the
         part outside the image and the wider steps cost what is saved."""
         return 2 * self.wh * self.ww <= self.H * self.W
+
+
+# A zonotope relu and fc are taken together from this many multiplications up:
+# below, the few more launches cost what the product saves (forwards of three
+# layers, apart and together: 784-256x3-10 of 16 boxes, 0.8e9 in the second
+# layer, 327 and 341 us; of 64 boxes, 3.3e9, 605 and 531).  Parts take so many
+# bytes at a time, which the last-level cache holds.
+_ZONO_SPLIT_MACS = 1.5e9
+_ZONO_WORK_BYTES = 192 << 20
 
 
 class BackwardTrace:
