@@ -282,6 +282,16 @@ int vc_zono_fc_cols(const float *W, int n_out, int n, int64_t B, int k, const in
                     int64_t idx_ld, const float *mu, const float *xl, const float *xh,
                     const int32_t *cnt, int k0, int64_t ld, float *G_out, vc_stream_t stream);
 
+/* vc_ibp_conv on the bf16 matrix cores: packed_t and packed_abs_t are the parts of
+ * the kernel (C_out, C_in kh kw) and of its magnitudes (vc_fc_split_pack with
+ * trans).  work: any multiple of 2 vc_fc_split_pack_bytes(C_in kh kw, H_out
+ * W_out), 16-byte aligned; as many boxes at a time. */
+int vc_ibp_conv_split(const float *l, const float *h, int64_t B, int C_in, int H, int W,
+                      const void *packed_t, const void *packed_abs_t, const float *bias,
+                      int C_out, int kh, int kw, int sh, int sw, int ph, int pw, int H_out,
+                      int W_out, float *lo, float *hi, void *work, int64_t work_bytes,
+                      vc_stream_t stream);
+
 /* relu backward step alone (for a relu that is not fed by an fc):
  * ew_out (M, n) = relaxed rows, acc += neg(ew) . up_t.  Same arguments as
  * the relu part of vc_backward_fc.  Replaces verify_zono_bnb.py:4409-4453. */

@@ -200,8 +200,14 @@ struct GemmArgs {
   int64_t tiles;
   FastDiv f_ntn;
   int64_t ld;
-  FastDiv f_dom;  // domains: row blocks of each
+  FastDiv f_dom;  // domains: row blocks of each; images: pixels
+  float* out2;    // images: the upper bounds
 };
+
+// Where the rows' results go: (M, N); many domains' rows, each stored
+// transposed; the pixels of images, stored by channel, the intervals' centres
+// or, onto those, their radii.
+enum Mode { kRows, kDomains, kCentres, kRadii };
 
 // Value j of lane's eight in a packed tile: the sum of its three parts.
 __device__ float part_sum(const uint4* p, int j) {
@@ -225,8 +231,8 @@ __device__ float plain_sum(const GemmArgs& a, int64_t t, int r, int n) {
   return (float)s;
 }
 
-// DOM: the rows are those of many domains, each stored transposed.
-template <int MT, bool DOM>
+// NJ: column tiles of a wave.
+template <int MT, int MODE, int NJ = 2>
 __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
   constexpr int AU = MT * 2 * kTileU;       // 16-byte units of a double step's rows
   constexpr int NL = (AU + FNT - 1) / FNT;  // of them per thread
@@ -238,9 +244,9 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
   const int64_t w = vcg::xcd_tile(blockIdx.x, a.tiles);
   const int tb = (int)a.f_ntn.div((uint32_t)w);
   const int tn = (int)(w - (int64_t)tb * a.ntn);
-  const int dom = DOM ? (int)a.f_dom.div((uint32_t)tb) : 0;
-  const int tm = DOM ? tb - dom * (int)a.f_dom.d : tb;
-  const int64_t t0 = DOM ? (int64_t)dom * a.mt16 : 0;  // the domain's first row tile
+  const int dom = MODE == kDomains ? (int)a.f_dom.div((uint32_t)tb) : 0;
+  const int tm = MODE == kDomains ? tb - dom * (int)a.f_dom.d : tb;
+  const int64_t t0 = MODE == kDomains ? (int64_t)dom * a.mt16 : 0;  // the domain's first row tile
 
   // this thread's units of each double step's rows (a row tile's two steps lie
   // together); past the last row tile the last one again, not stored
@@ -251,19 +257,19 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
     const int t = min(tm * MT + u / (2 * kTileU), a.mt16 - 1);
     A[i] = reinterpret_cast<const u4*>(a.Ap) + (t0 + t) * a.nkc * kTileU + u % (2 * kTileU);
   }
-  // this wave's two column tiles, likewise
-  const int c0 = tn * 8 + wv * 2, nt16 = (a.N + 15) >> 4;
-  const u4* B[2];
+  // this wave's column tiles, likewise
+  const int c0 = (tn * 4 + wv) * NJ, nt16 = (a.N + 15) >> 4;
+  const u4* B[NJ];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < NJ; ++j)
     B[j] = reinterpret_cast<const u4*>(a.Bp) + (int64_t)min(c0 + j, nt16 - 1) * a.nkc * kTileU +
            lane;
 
-  v4f acc[MT][2], small[MT][2], z[MT][2];
+  v4f acc[MT][NJ], small[MT][NJ], z[MT][NJ];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = small[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = small[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
   // past the last step the last again: no branch, nothing waits for it
   const int steps = a.nkc >> 1;
@@ -272,14 +278,14 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) v[i] = A[i][o];
   };
-  const auto load_cols = [&](int kc, u4(&v)[2][3]) {
+  const auto load_cols = [&](int kc, u4(&v)[NJ][3]) {
     const int64_t o = (int64_t)min(kc, a.nkc - 1) * kTileU;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int p = 0; p < 3; ++p) v[j][p] = B[j][o + 64 * p];
   };
-  u4 rn[NL], b[2][2][3];
+  u4 rn[NL], b[2][NJ][3];
   load_rows(0, rn);
   load_cols(0, b[0]);
 #pragma unroll
@@ -315,7 +321,7 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < Q; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
+          for (int j = 0; j < NJ; ++j) {
             v4f& d = p == 5 ? z[i0 + i][j] : small[i0 + i][j];
             d = mfma_bf16(av[t & 1][i][kPartA[p]], b[hf][j][kPartB[p]],
                           p == 5 && hf == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : d);
@@ -324,7 +330,7 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
 #pragma unroll
         for (int i = i0; i < i0 + Q; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
+          for (int j = 0; j < NJ; ++j) {
             const v4f t2 = acc[i][j] + z[i][j];
             small[i][j] += z[i][j] - (t2 - acc[i][j]);
             acc[i][j] = t2;
@@ -346,7 +352,7 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
 
   const int g = lane >> 4, r = lane & 15;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < NJ; ++j) {
     const int n = (c0 + j) * 16 + r;
     if (n >= a.N) continue;
     const float b = a.bias ? a.bias[n] : 0.f;
@@ -362,10 +368,10 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
           v[q] = plain_sum(a, t0 + tm * MT + i, 4 * g + q, n);
         if (a.bias) v[q] = v[q] + b;
       }
-      if (DOM) {
+      typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+      if (MODE == kDomains) {
         float* o = a.out + ((int64_t)dom * a.N + n) * a.ld + m0;
         if (m0 + 4 <= a.M) {
-          typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
           *reinterpret_cast<v4u*>(o) = v4u{v[0], v[1], v[2], v[3]};
           continue;
         }
@@ -374,10 +380,99 @@ __global__ __launch_bounds__(FNT, 2) void k_fc_gemm(GemmArgs a) {
           if (m0 + q < a.M) o[q] = v[q];
         continue;
       }
+      if (MODE == kCentres || MODE == kRadii) {
+        const uint32_t npx = a.f_dom.d;
+        const int64_t img = a.f_dom.div((uint32_t)m0);
+        const int64_t at = (img * a.N + n) * npx + (m0 - img * npx);
+        if (m0 + 4 <= a.M && m0 - img * npx + 4 <= npx) {
+          v4u* const o = reinterpret_cast<v4u*>(a.out + at);
+          v4u x = v4u{v[0], v[1], v[2], v[3]};
+          if (MODE == kRadii) {
+            const v4u c = *o;
+            *reinterpret_cast<v4u*>(a.out2 + at) = c + x;
+            x = c - x;
+          }
+          *o = x;
+          continue;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (m0 + q >= a.M) continue;
+          const int64_t im = a.f_dom.div((uint32_t)(m0 + q));
+          const int64_t o = (im * a.N + n) * npx + (m0 + q - im * npx);
+          if (MODE == kRadii) {
+            const float c = a.out[o];
+            a.out2[o] = c + v[q];
+            v[q] = c - v[q];
+          }
+          a.out[o] = v[q];
+        }
+        continue;
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (m0 + q < a.M) a.out[(m0 + q) * a.N + n] = v[q];
     }
+  }
+}
+
+// The interval forward of a conv (verify_zono_bnb.py:1114-1123): centres and
+// radii of the pixels it reads, as rows of its products with the kernel and its
+// magnitudes.  Row = output pixel m, value k = (channel, tap) of the kernel.  A
+// wave forms 16 pixels' parts, both kinds from one load of the bounds (HBM
+// bound, by the parts written: 1.2 GB in 385 us).  Three convs of 512 32x32
+// images to 64 channels, the whole forward 1465 -> 1141 us (32 -> 64 and 64 ->
+// 64, 4x4: the gathering product 1017 us, now 680).
+struct ConvRows {
+  const float *l, *h;
+  int C_in, H, W, kh, kw, sh, sw, ph, pw, Wo, K, nkc;
+  int64_t M;
+  FastDiv f_px, f_wo, f_taps, f_kw;
+  uint4 *mid, *rad;
+};
+__global__ __launch_bounds__(FNT) void k_conv_rows(ConvRows a) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
+  const int64_t m0 = (int64_t)blockIdx.x * 16;
+  const uint32_t m = (uint32_t)(m0 + r < a.M ? m0 + r : a.M - 1);
+  const int64_t img = a.f_px.div(m);
+  const int px = (int)(m - img * a.f_px.d);
+  const int oy = (int)a.f_wo.div((uint32_t)px), ox = px - oy * a.Wo;
+  const int y0 = oy * a.sh - a.ph, x0 = ox * a.sw - a.pw;
+  const float* const pl = a.l + img * a.C_in * a.H * a.W;
+  const float* const ph = a.h + img * a.C_in * a.H * a.W;
+  const int64_t out = (int64_t)blockIdx.x * a.nkc * kTileU + lane;
+  for (int kc = wv; kc < a.nkc; kc += 4) {
+    float mid[8], rad[8];
+    int k = kc * FBK + 8 * g;
+    int ci = (int)a.f_taps.div((uint32_t)k), t = k - ci * (int)a.f_taps.d;
+    int ky = (int)a.f_kw.div((uint32_t)t), kx = t - ky * a.kw;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int y = y0 + ky, x = x0 + kx;
+      const bool in = k + j < a.K && (unsigned)y < (unsigned)a.H && (unsigned)x < (unsigned)a.W;
+      const int o = in ? (ci * a.H + y) * a.W + x : 0;
+      const float l = pl[o], h = ph[o];
+      mid[j] = in ? (l + h) / 2.f : 0.f;
+      rad[j] = in ? (h - l) / 2.f : 0.f;
+      // the next tap
+      const bool row = ++kx == a.kw;
+      kx = row ? 0 : kx;
+      ky += row ? 1 : 0;
+      const bool chan = ky == a.kh;
+      ky = chan ? 0 : ky;
+      ci += chan ? 1 : 0;
+    }
+    uint4 p[3];
+    uint4* o = a.mid + out + (int64_t)kc * kTileU;
+    split8_all(mid, p[0], p[1], p[2]);
+    o[0] = p[0];
+    o[64] = p[1];
+    o[128] = p[2];
+    o = a.rad + out + (int64_t)kc * kTileU;
+    split8_all(rad, p[0], p[1], p[2]);
+    o[0] = p[0];
+    o[64] = p[1];
+    o[128] = p[2];
   }
 }
 
@@ -530,9 +625,9 @@ int launch_fc(RowArgs a, const void* packed, int N, const float* bias, float* ou
     hipLaunchKernelGGL((k_fc_rows<FORM, false>), dim3((unsigned)mt16), dim3(FNT), 0, st, a);
   VC_LAUNCH_CHECK();
   const dim3 grid((unsigned)b.tiles);
-  if (mt == 4) hipLaunchKernelGGL((k_fc_gemm<4, false>), grid, dim3(FNT), 0, st, b);
-  if (mt == 2) hipLaunchKernelGGL((k_fc_gemm<2, false>), grid, dim3(FNT), 0, st, b);
-  if (mt == 1) hipLaunchKernelGGL((k_fc_gemm<1, false>), grid, dim3(FNT), 0, st, b);
+  if (mt == 4) hipLaunchKernelGGL((k_fc_gemm<4, kRows>), grid, dim3(FNT), 0, st, b);
+  if (mt == 2) hipLaunchKernelGGL((k_fc_gemm<2, kRows>), grid, dim3(FNT), 0, st, b);
+  if (mt == 1) hipLaunchKernelGGL((k_fc_gemm<1, kRows>), grid, dim3(FNT), 0, st, b);
   VC_LAUNCH_CHECK();
   return VC_OK;
 }
@@ -685,7 +780,79 @@ extern "C" int vc_zono_fc_split(const float* G, const float* lam, int64_t B, int
     VC_LAUNCH_CHECK();
     b.out = G_out + b0 * n_out * ld;
     b.tiles = cnt * blk * b.ntn;
-    hipLaunchKernelGGL((k_fc_gemm<4, true>), dim3((unsigned)b.tiles), dim3(FNT), 0, st, b);
+    hipLaunchKernelGGL((k_fc_gemm<4, kDomains>), dim3((unsigned)b.tiles), dim3(FNT), 0, st, b);
+    VC_LAUNCH_CHECK();
+  }
+  return VC_OK;
+}
+
+extern "C" int vc_ibp_conv_split(const float* l, const float* h, int64_t B, int C_in, int H, int W,
+                                 const void* packed_t, const void* packed_abs_t,
+                                 const float* bias, int C_out, int kh, int kw, int sh, int sw,
+                                 int ph, int pw, int H_out, int W_out, float* lo, float* hi,
+                                 void* work, int64_t work_bytes, vc_stream_t stream) {
+  if (B < 0 || C_in <= 0 || H <= 0 || W <= 0 || C_out <= 0 || kh <= 0 || kw <= 0 || sh <= 0 ||
+      sw <= 0 || ph < 0 || pw < 0 || H_out <= 0 || W_out <= 0)
+    return VC_ERR_ARG;
+  if (B == 0) return VC_OK;
+  if (!l || !h || !packed_t || !packed_abs_t || !lo || !hi || !work || !aligned16(packed_t) ||
+      !aligned16(packed_abs_t) || !aligned16(work))
+    return VC_ERR_ARG;
+  const int64_t npx = (int64_t)H_out * W_out, K = (int64_t)C_in * kh * kw;
+  if (npx >= 1 << 24 || K >= 1 << 24 || (int64_t)H * W >= 1 << 28 ||
+      (int64_t)C_in * H * W >= (int64_t(1) << 31))
+    return VC_ERR_UNSUPPORTED;
+  const hipStream_t st = (hipStream_t)stream;
+  ConvRows a{l, h, C_in, H, W, kh, kw, sh, sw, ph, pw, W_out, (int)K};
+  a.nkc = 2 * (((int)K + 2 * FBK - 1) / (2 * FBK));
+  a.f_px = FastDiv::make((uint32_t)npx);
+  a.f_wo = FastDiv::make((uint32_t)W_out);
+  a.f_taps = FastDiv::make((uint32_t)(kh * kw));
+  a.f_kw = FastDiv::make((uint32_t)kw);
+  // images whose parts the buffer holds, centres and radii, within 32-bit rows
+  const int64_t per = vc_fc_split_pack_bytes(K, npx);
+  int64_t step = work_bytes / (2 * per);
+  const int64_t most = (((int64_t)1 << 31) - 64) / npx;
+  if (step > most) step = most;
+  if (step < 1) return VC_ERR_ARG;
+  // one column tile a wave where two would leave half of the waves without
+  const int nj = C_out <= 64 ? 1 : 2;
+  GemmArgs b{};
+  b.nkc = a.nkc;
+  b.N = C_out;
+  b.ntn = (C_out + 64 * nj - 1) / (64 * nj);
+  b.f_ntn = FastDiv::make((uint32_t)b.ntn);
+  b.f_dom = a.f_px;
+  for (int64_t b0 = 0; b0 < B; b0 += step) {
+    const int64_t cnt = B - b0 < step ? B - b0 : step;
+    a.l = l + b0 * C_in * H * W;
+    a.h = h + b0 * C_in * H * W;
+    a.M = b.M = cnt * npx;
+    b.mt16 = (int)((a.M + 15) / 16);
+    a.mid = (uint4*)work;
+    a.rad = a.mid + (int64_t)b.mt16 * a.nkc * kTileU;
+    hipLaunchKernelGGL(k_conv_rows, dim3((unsigned)b.mt16), dim3(FNT), 0, st, a);
+    VC_LAUNCH_CHECK();
+    b.tiles = (int64_t)((b.mt16 + 3) / 4) * b.ntn;
+    if (b.tiles >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+    const dim3 grid((unsigned)b.tiles);
+    b.out = lo + b0 * C_out * npx;
+    b.out2 = hi + b0 * C_out * npx;
+    b.Ap = a.mid;
+    b.Bp = (const uint4*)packed_t;
+    b.bias = bias;
+    if (nj == 1)
+      hipLaunchKernelGGL((k_fc_gemm<4, kCentres, 1>), grid, dim3(FNT), 0, st, b);
+    else
+      hipLaunchKernelGGL((k_fc_gemm<4, kCentres, 2>), grid, dim3(FNT), 0, st, b);
+    VC_LAUNCH_CHECK();
+    b.Ap = a.rad;
+    b.Bp = (const uint4*)packed_abs_t;
+    b.bias = nullptr;
+    if (nj == 1)
+      hipLaunchKernelGGL((k_fc_gemm<4, kRadii, 1>), grid, dim3(FNT), 0, st, b);
+    else
+      hipLaunchKernelGGL((k_fc_gemm<4, kRadii, 2>), grid, dim3(FNT), 0, st, b);
     VC_LAUNCH_CHECK();
   }
   return VC_OK;

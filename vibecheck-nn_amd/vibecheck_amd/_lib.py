@@ -71,6 +71,8 @@ SIGNATURES = {
     'vc_zono_relu_lists': [_P, _P, _P, _P, _L, _I, _I, _P, _P, _P, _P, _P],
     'vc_zono_fc_split': [_P, _P, _L, _I, _I, _P, _I, _L, _P, _P, _L, _P],
     'vc_zono_fc_cols': [_P, _I, _I, _L, _I, _P, _L, _P, _P, _P, _P, _I, _L, _P, _P],
+    'vc_ibp_conv_split': [_P, _P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I,
+                          _P, _P, _P, _L, _P],
     'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     'vc_patch_shift': [_P, _I, _I, _I, _I, _I, _P, _P],
     'vc_patch_relax': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P],

@@ -244,6 +244,22 @@ def _fc_parts(p, st, trans=False):
     return p[key][1]
 
 
+def _conv_interval_parts(p, K, st):
+    """The parts of a conv's kernel and of its magnitudes for vc_ibp_conv_split,
+    cached with the op's other device tensors."""
+    version = p['K']._version  # the kernel may be the caller's own
+    if 'KI' not in p or p['KI'][0] != version:
+        n = p['K'].shape[0]
+        parts = []
+        for k in (p['K'], p['K'].abs()):
+            out = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, n), dtype=torch.uint8,
+                              device=k.device)
+            call('vc_fc_split_pack', ptr(k), K, n, 1, ptr(out), st)
+            parts.append(out)
+        p['KI'] = (version, parts)
+    return p['KI'][1]
+
+
 def _fc_split_work(M, K, dev):
     """The buffer of M rows' parts that a vc_fc_split product forms first."""
     return torch.empty(_lib.load().vc_fc_split_pack_bytes(K, M), dtype=torch.uint8, device=dev)
@@ -379,9 +395,15 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
     hi = {gg['input_name']: xh}
     sb = {}
     st = stream()
+    # nodes without a relu below them: their intervals are exact, CROWN's first
+    # bounds equal them up to rounding and choose slopes by the larger of the
+    # two, so their sums keep their order
+    raw = {gg['input_name']}
     for op in gg['ops']:
         t = op['type']
         name = op['name']
+        if t != 'relu' and all(i in raw for i in op['inputs']):
+            raw.add(name)
         l, h = lo[op['inputs'][0]], hi[op['inputs'][0]]
         if t == 'fc':
             if _fc_form(op, widths[op['inputs'][0]])[0] > 1:
@@ -401,9 +423,20 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
             C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
             lo_o = torch.empty(B, p['n_out'], device=dev)
             hi_o = torch.empty_like(lo_o)
-            call('vc_ibp_conv', ptr(l), ptr(h), B, C_in, H, W, ptr(p['K']),
-                 ptr(p['b']), C_out, kh, kw, sh, sw, ph, pw, Ho, Wo,
-                 ptr(lo_o), ptr(hi_o), st)
+            K = C_in * kh * kw
+            if (name not in raw and K >= 512 and C_out > 32
+                    and B * p['n_out'] * K >= _IBP_SPLIT_MACS):
+                parts = _conv_interval_parts(p, K, st)
+                per = 2 * _lib.load().vc_fc_split_pack_bytes(K, Ho * Wo)
+                work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)),
+                                   dtype=torch.uint8, device=dev)
+                call('vc_ibp_conv_split', ptr(l), ptr(h), B, C_in, H, W, ptr(parts[0]),
+                     ptr(parts[1]), ptr(p['b']), C_out, kh, kw, sh, sw, ph, pw, Ho, Wo,
+                     ptr(lo_o), ptr(hi_o), ptr(work), work.numel(), st)
+            else:
+                call('vc_ibp_conv', ptr(l), ptr(h), B, C_in, H, W, ptr(p['K']),
+                     ptr(p['b']), C_out, kh, kw, sh, sw, ph, pw, Ho, Wo,
+                     ptr(lo_o), ptr(hi_o), st)
             lo[name], hi[name] = lo_o, hi_o
         elif t == 'relu':
             L = op.get('layer_idx')
@@ -705,6 +738,12 @@ class _Window:
 # layer, 327 and 341 us; of 64 boxes, 3.3e9, 605 and 531).  Parts take so many
 # bytes at a time, which the last-level cache holds.
 _ZONO_SPLIT_MACS = 1.5e9
+# The interval forward of a conv likewise; the pass that forms its parts writes
+# 12 bytes per pixel and tap whatever the channels out, so few of them or few
+# taps stay with the gathering product (whole forwards, it and the parts: 32->64
+# 4x4, 64 boxes 0.5e9 989 and 966 us, 512 boxes 1796 and 1534; 32->32 3x3 of 512
+# 803 and 935, 8->16 5x5 459 and 541).
+_IBP_SPLIT_MACS = 5e8
 _ZONO_WORK_BYTES = 192 << 20
 
 
