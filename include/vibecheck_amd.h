@@ -282,6 +282,14 @@ int vc_zono_fc_cols(const float *W, int n_out, int n, int64_t B, int k, const in
                     int64_t idx_ld, const float *mu, const float *xl, const float *xh,
                     const int32_t *cnt, int k0, int64_t ld, float *G_out, vc_stream_t stream);
 
+/* vc_ibp_fc with K in slices, whose sums (slices, B, n_out, 2) of 64 bits go to
+ * work (16-byte aligned): for long K and few outputs.  vc_ibp_fc_slices: how many
+ * to take, 1 where vc_ibp_fc is to be called. */
+int vc_ibp_fc_slices(int64_t B, int n_in, int n_out);
+int vc_ibp_fc_sliced(const float *l, const float *h, int64_t B, int n_in, const float *W,
+                     const float *bias, int n_out, float *lo, float *hi, int slices, void *work,
+                     vc_stream_t stream);
+
 /* vc_ibp_conv on the bf16 matrix cores: packed_t and packed_abs_t are the parts of
  * the kernel (C_out, C_in kh kw) and of its magnitudes (vc_fc_split_pack with
  * trans).  work: any multiple of 2 vc_fc_split_pack_bytes(C_in kh kw, H_out

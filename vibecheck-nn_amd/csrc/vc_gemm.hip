@@ -106,6 +106,30 @@ struct LoadMidRad {  // A = (mid, rad) of an interval row-block
   }
 };
 
+// Slice bz of a long K: its values from column bz * slice on; past the row's
+// end zero.
+struct LoadMidRadSlice : LoadMidRad {
+  int slice;
+  struct Row {
+    int64_t o;
+    int left;
+  };
+  __device__ Row row(int64_t bz, int64_t m, bool) const {
+    return Row{m * ld + bz * slice, ld - (int)bz * slice};
+  }
+  template <bool VEC>
+  __device__ void fetch(const Row& rw, int k, int n, Raw& x) const {
+    n = min(n, rw.left - k);
+    ld4<VEC>(l + rw.o + k, n, x.l);
+    ld4<VEC>(h + rw.o + k, n, x.h);
+  }
+  template <bool VEC>
+  __device__ void finish(const Row& rw, int k, int n, const Raw& x, float (*v)[4], KSum& s,
+                         bool rows) const {
+    LoadMidRad::finish<VEC>(LoadMidRad::Row{rw.o}, k, n, x, v, s, rows);
+  }
+};
+
 // The group of domain d, read in range: an index outside [0, n_groups)
 // reads group 0 (vc_group_clamp reports such indices to the caller).
 __device__ __forceinline__ int64_t safe_group(const int64_t* group, int64_t n_groups, int64_t d) {
@@ -330,7 +354,32 @@ struct LoadWtAbs {  // B[k][n] = (W[n][k], |W[n][k]|), W (n_out, ld)
   }
 };
 
+struct LoadWtAbsSlice : LoadWtAbs {
+  int slice;
+  struct Col {
+    int64_t o;
+    int left;
+  };
+  __device__ Col col(int64_t bz, int n) const {
+    return Col{(int64_t)n * ld + bz * slice, ld - (int)bz * slice};
+  }
+  template <bool VEC>
+  __device__ void fetch(const Col& c, int k, int cnt, Raw& r) const {
+    ld4<VEC>(W + c.o + k, min(cnt, c.left - k), r.x);
+  }
+};
+
 // ------------------------------------------------------------- epilogues
+struct EpSums {  // a slice's sums in 64 bits
+  typedef double Value;
+  double2* out;
+  int64_t M;
+  int ld;
+  __device__ void operator()(int64_t bz, int64_t m, int n, const double* c) const {
+    out[(bz * M + m) * ld + n] = make_double2(c[0], c[1]);
+  }
+};
+
 struct EpIbp {
   const float* bias;
   float *lo, *hi;
@@ -463,6 +512,69 @@ extern "C" int vc_ibp_fc(const float* l, const float* h, int64_t B, int n_in,
   const bool vec = vec_ok({l, h, W}, {n_in});
   return launch_gemm<2, false>(1, B, n_out, n_in, LoadMidRad{l, h, n_in}, LoadWtAbs{W, n_in},
                                EpIbp{bias, lo, hi, n_out}, nullptr, vec, (hipStream_t)stream);
+}
+
+namespace {
+__global__ __launch_bounds__(NT) void k_ibp_fc_sum(const double2* sums, int slices, int64_t M,
+                                                   int N, EpIbp ep) {
+  const int64_t total = M * N;
+  for (int64_t i = blockIdx.x * (int64_t)NT + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * NT) {
+    double c = 0.0, r = 0.0;
+    for (int s = 0; s < slices; ++s) {
+      const double2 v = sums[s * total + i];
+      c += v.x;
+      r += v.y;
+    }
+    const float o[2] = {(float)c, (float)r};
+    const int64_t m = i / N;
+    ep(0, m, (int)(i - m * N), o);
+  }
+}
+}  // namespace
+
+// Slices of K for the interval fc: where the output has too few tiles to fill
+// the chip and K is long, one workgroup's chain of K-tiles is the whole time.
+// The sums are 64-bit folds of the same 32-deep K-tiles, so slices change their
+// order only, below what a rounding to fp32 shows.  Whole forwards of a CNN
+// with such an fc: 512 images, 4096 -> 512, 1141 -> 991 us; five boxes' CROWN of
+// a small one (28x27 images) 764 -> 739.
+extern "C" int vc_ibp_fc_slices(int64_t B, int n_in, int n_out) {
+  if (B <= 0 || n_in < 512 || n_out <= 0) return 1;
+  const int64_t tiles = (B + 31) / 32 * ((n_out + 63) / 64);
+  int64_t s = (512 + tiles - 1) / tiles;
+  if (s > n_in / 128) s = n_in / 128;
+  return s < 2 ? 1 : (int)(s > 128 ? 128 : s);
+}
+
+extern "C" int vc_ibp_fc_sliced(const float* l, const float* h, int64_t B, int n_in,
+                                const float* W, const float* bias, int n_out, float* lo,
+                                float* hi, int slices, void* work, vc_stream_t stream) {
+  if (!l || !h || !W || !lo || !hi || n_in <= 0 || n_out <= 0 || B < 0 || slices < 1 || !work ||
+      !aligned16(work))
+    return VC_ERR_ARG;
+  if (B == 0) return VC_OK;
+  const int per = ((n_in + slices - 1) / slices + 31) / 32 * 32;
+  slices = (n_in + per - 1) / per;  // rounded up to whole K-tiles: maybe fewer
+  const bool vec = vec_ok({l, h, W}, {n_in});
+  LoadMidRadSlice la;
+  la.l = l;
+  la.h = h;
+  la.ld = n_in;
+  la.slice = per;
+  LoadWtAbsSlice lb;
+  lb.W = W;
+  lb.ld = n_in;
+  lb.slice = per;
+  const int rc = launch_gemm<2, false>(slices, B, n_out, per, la, lb,
+                                       EpSums{(double2*)work, B, n_out}, nullptr, vec,
+                                       (hipStream_t)stream);
+  if (rc != VC_OK) return rc;
+  hipLaunchKernelGGL(k_ibp_fc_sum, dim3(vc_blocks(B * n_out, NT)), dim3(NT), 0,
+                     (hipStream_t)stream, (const double2*)work, slices, B, n_out,
+                     EpIbp{bias, lo, hi, n_out});
+  VC_LAUNCH_CHECK();
+  return VC_OK;
 }
 
 extern "C" int vc_zono_fc(const float* c, const float* G, int64_t B, int n_in, int K,

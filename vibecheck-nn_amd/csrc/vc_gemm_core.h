@@ -93,6 +93,17 @@ struct FastDiv {
   }
 };
 
+// What an epilogue receives: the sums rounded to fp32, or (EP::Value = double)
+// as they are.
+template <class T, class = void>
+struct EpValue {
+  typedef float type;
+};
+template <class T>
+struct EpValue<T, std::void_t<typename T::Value>> {
+  typedef typename T::Value type;
+};
+
 // ---------------------------------------------------------------- core
 // NA: number of A/B operand pairs (1, or 2 for the dual IBP product).
 // ACC_ROWS: the A loader also returns a per-element row contribution,
@@ -286,9 +297,9 @@ __global__ __launch_bounds__(NT) void gemm_kernel(int64_t M, int N, int K, int t
           const int64_t m = m0 + wm * 16 * FM + i * 16 + 4 * g + e;
           const int n = n0 + wn * 16 * FN + j * 16 + r;
           if (m < M && n < N) {
-            float c[NA];
+            typename EpValue<EP>::type c[NA];
 #pragma unroll
-            for (int a = 0; a < NA; ++a) c[a] = (float)acc[a][i][j][e];
+            for (int a = 0; a < NA; ++a) c[a] = (typename EpValue<EP>::type)acc[a][i][j][e];
             ep(bz, m, n, c);
           }
         }

@@ -71,6 +71,8 @@ SIGNATURES = {
     'vc_zono_relu_lists': [_P, _P, _P, _P, _L, _I, _I, _P, _P, _P, _P, _P],
     'vc_zono_fc_split': [_P, _P, _L, _I, _I, _P, _I, _L, _P, _P, _L, _P],
     'vc_zono_fc_cols': [_P, _I, _I, _L, _I, _P, _L, _P, _P, _P, _P, _I, _L, _P, _P],
+    'vc_ibp_fc_slices': [_L, _I, _I],
+    'vc_ibp_fc_sliced': [_P, _P, _L, _I, _P, _P, _I, _P, _P, _I, _P, _P],
     'vc_ibp_conv_split': [_P, _P, _L, _I, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I,
                           _P, _P, _P, _L, _P],
     'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],

@@ -415,8 +415,14 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
             p = _op_params(op, dev)
             lo_o = torch.empty(B, p['n_out'], device=dev)
             hi_o = torch.empty_like(lo_o)
-            call('vc_ibp_fc', ptr(l), ptr(h), B, p['n_in'], ptr(p['W']),
-                 ptr(p['b']), p['n_out'], ptr(lo_o), ptr(hi_o), st)
+            slices = _lib.load().vc_ibp_fc_slices(B, p['n_in'], p['n_out'])
+            if slices > 1:
+                work = torch.empty(slices * B * p['n_out'] * 2, dtype=torch.float64, device=dev)
+                call('vc_ibp_fc_sliced', ptr(l), ptr(h), B, p['n_in'], ptr(p['W']), ptr(p['b']),
+                     p['n_out'], ptr(lo_o), ptr(hi_o), slices, ptr(work), st)
+            else:
+                call('vc_ibp_fc', ptr(l), ptr(h), B, p['n_in'], ptr(p['W']),
+                     ptr(p['b']), p['n_out'], ptr(lo_o), ptr(hi_o), st)
             lo[name], hi[name] = lo_o, hi_o
         elif t == 'conv':
             p = _op_params(op, dev)
