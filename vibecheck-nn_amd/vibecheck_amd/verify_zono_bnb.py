@@ -747,9 +747,9 @@ _ZONO_SPLIT_MACS = 1.5e9
 # The interval forward of a conv likewise; the pass that forms its parts writes
 # 12 bytes per pixel and tap whatever the channels out, so few of them or few
 # taps stay with the gathering product (whole forwards, it and the parts: 32->64
-# 4x4, 64 boxes 0.5e9 989 and 966 us, 512 boxes 1796 and 1534; 32->32 3x3 of 512
+# 4x4, 16 boxes 0.13e9 119 and 108 us, 512 boxes 957 and 697; 32->32 3x3 of 512
 # 803 and 935, 8->16 5x5 459 and 541).
-_IBP_SPLIT_MACS = 5e8
+_IBP_SPLIT_MACS = 1e8
 _ZONO_WORK_BYTES = 192 << 20
 
 
@@ -971,7 +971,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         rows = ew_at.pop(name)
         t = op['type']
         inp = op['inputs'][0]
-        if t not in ('conv', 'relu'):
+        if rows.window is not None and t not in ('conv', 'relu'):
             rows = dense(rows)
         if t in ('add', 'sub', 'mul') and trace is not None:
             trace.other = trace.other or t
@@ -1029,7 +1029,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 M = B * R
                 out = torch.empty(M, p['n_in'], device=dev)
                 parts = None
-                if split and rows.alpha_group is None and not rows.alpha_row:
+                if (split and M >= _FC_SPLIT_SWEEP_ROWS and rows.alpha_group is None
+                        and not rows.alpha_row):
                     parts = _fc_split_parts(p, M, st, sweep=trace is not None)
                 if parts is not None:
                     ls, us, ut = slopes(rows)
