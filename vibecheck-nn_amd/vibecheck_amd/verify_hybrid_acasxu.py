@@ -178,6 +178,7 @@ def _full_freeze(xl, xh, gg, spec_ew, device, dtype, n_iters_per_layer=100,
     if n_iters_spec < 1:
         raise ValueError('vibecheck_amd: the spec loop needs at least one iteration')
     feeds = _relu_feeds(gg)
+    packs = vz._Packs()
     alpha_per_layer = {}
     for L in order:
         if deadline is not None and time.perf_counter() > deadline:
@@ -190,7 +191,8 @@ def _full_freeze(xl, xh, gg, spec_ew, device, dtype, n_iters_per_layer=100,
             ps = _AlphaSet(tight, keys, B, 2 * n, dev)
             best = torch.empty(B, 2 * n, device=dev)
             _optimise(ps, lambda: vz._alpha_backward_and_grad(
-                tight, xl, xh, gg, Wq, bq, ps.alpha, True, ps.galpha, seed_name=feeds[L]),
+                tight, xl, xh, gg, Wq, bq, ps.alpha, True, ps.galpha, seed_name=feeds[L],
+                packs=packs),
                 best, n_iters_per_layer, lr, lr_decay, early_stop_eps)
             if n_iters_per_layer > 0:
                 _tighten_layer(tight, L, best)
@@ -202,7 +204,7 @@ def _full_freeze(xl, xh, gg, spec_ew, device, dtype, n_iters_per_layer=100,
     ps = _AlphaSet(tight, order, B, Q, dev)
     best_spec = torch.empty(B, Q, device=dev)
     _optimise(ps, lambda: vz._alpha_backward_and_grad(
-        tight, xl, xh, gg, Wq, bq, ps.alpha, True, ps.galpha),
+        tight, xl, xh, gg, Wq, bq, ps.alpha, True, ps.galpha, packs=packs),
         best_spec, n_iters_spec, lr, lr_decay, early_stop_eps, deadline)
     alpha_spec = {k: ps.alpha[k].clone() for k in order}
     return tight, alpha_per_layer, alpha_spec, best_spec
@@ -248,6 +250,7 @@ def _replay_batched(xl_b, xh_b, gg, spec_ew, alpha_layer_b, alpha_spec_b,
                         for k, a in alpha_spec_b.items()}
     tight = _zono_tight(xl, xh, gg, device, dtype)
     feeds = _relu_feeds(gg)
+    packs = vz._Packs()
     for L in sorted(tight):
         if not alpha_layer_b.get(L):
             continue
@@ -258,7 +261,7 @@ def _replay_batched(xl_b, xh_b, gg, spec_ew, alpha_layer_b, alpha_spec_b,
         else:
             alpha = {k: _per_leaf(a, B) for k, a in alpha_layer_b[L].items()}
         sl = vz._alpha_backward_and_grad(tight, xl, xh, gg, Wq, bq, alpha, False, None,
-                                         seed_name=feeds[L])
+                                         seed_name=feeds[L], packs=packs)
         _tighten_layer(tight, L, sl)
     Wq, bq = vz._spec_rows(spec_ew, dev)
     Q = Wq.shape[0]
@@ -269,7 +272,7 @@ def _replay_batched(xl_b, xh_b, gg, spec_ew, alpha_layer_b, alpha_spec_b,
     for it in range(n_it):
         last = it == n_it - 1
         lb, A = vz._alpha_backward_and_grad(tight, xl, xh, gg, Wq, bq, ps.alpha, not last,
-                                            ps.galpha, want_A=True)
+                                            ps.galpha, want_A=True, packs=packs)
         call('vc_best_rows_with_A', ptr(best), ptr(lb.contiguous()), ptr(best_A), ptr(A),
              B, Q, n_in, 1 if it == 0 else 0, stream())
         if not last:

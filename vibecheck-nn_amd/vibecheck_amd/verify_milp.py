@@ -18,7 +18,7 @@ import torch
 
 from ._lib import call, f32, ptr, stream
 from .verify_zono_bnb import (_alpha_backward_and_grad, _check_dtype,
-                              _ibp_forward_graph_batched, _spec_rows)
+                              _ibp_forward_graph_batched, _Packs, _spec_rows)
 
 __all__ = ['_split_clamps_batched', '_sb_for_domains', '_ibp_crown_bab_bound']
 
@@ -196,12 +196,13 @@ def _ibp_crown_bab_bound(gg, xl, xh, sb_root, relu_clamps, spec_ew, device,
     n_eval = 0
     step = 0
     n_it = max(1, int(alpha_iters))
+    packs = _Packs()
     for it in range(n_it):
         # the Adam step after the last evaluation is never used: skip its gradient
         last = it == n_it - 1
         lb = _alpha_backward_and_grad(sb, xl_b, xh_b, gg, Wq, bq, alpha, not last,
                                       galpha, beta=beta_s or None,
-                                      gbeta=gbeta or None)
+                                      gbeta=gbeta or None, packs=packs)
         n_eval += 1
         call('vc_best_update', ptr(best), ptr(lb.contiguous()), B * Q,
              1 if it == 0 else 0, ptr(red), st)

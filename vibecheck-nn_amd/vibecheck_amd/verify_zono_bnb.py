@@ -60,7 +60,7 @@ def _op_params(op, device):
     cached = op.get(key)
     if cached is not None and cached['device'] == device:
         return cached
-    p = {'device': device}
+    p = {'device': device, 'name': op['name']}
     if op['type'] == 'fc':
         p['W'] = op['W'].detach().to(device=device, dtype=torch.float32).contiguous()
         b = op.get('bias')
@@ -217,31 +217,41 @@ def _conv_split_parts(p, st):
     return p['KS']
 
 
-def _fc_split_parts(p, M, st, trans=False, sweep=False):
+class _Packs:
+    """The weights in the layouts that one call's products read.  Each is made
+    on first use, on the call's stream, from the weights as they are then, and
+    goes with the call: another thread's call on its own stream packs for
+    itself, and a weight written between two calls (also through ``.data``,
+    which no version counter shows) is seen by the second.  1024 x 1024 weights
+    take about 10 us, of products of 100 us and more."""
+
+    def __init__(self):
+        self._made = {}
+
+    def fc(self, p, st, trans=False):
+        """The bf16 parts of an fc's W, or of its transpose."""
+        out = self._made.get((p['name'], trans))
+        if out is None:
+            K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
+            out = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, N), dtype=torch.uint8,
+                              device=p['W'].device)
+            call('vc_fc_split_pack', ptr(p['W']), K, N, 1 if trans else 0, ptr(out), st)
+            self._made[p['name'], trans] = out
+        return out
+
+
+def _fc_split_parts(packs, p, M, st, trans=False, sweep=False):
     """The fc weights' bf16 parts for M rows' vc_backward_fc_split (``trans``:
-    for the gradient's products with W^T), made on first use and cached with
-    the op's other device tensors; None where the fp32 product is the faster
-    one.  ``sweep``: a gradient sweep follows that uses the backward's slopes."""
+    for the gradient's products with W^T); None where the fp32 product is the
+    faster one.  ``sweep``: a gradient sweep follows that uses the backward's
+    slopes."""
     K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
     if trans:
         ok = M >= _FC_SPLIT_SWEEP_ROWS and min(K, N) >= _FC_SPLIT_WIDTH
     else:
         ok = (M >= (_FC_SPLIT_SWEEP_ROWS if sweep else _FC_SPLIT_ROWS)
               and K >= _TWO_PHASE_MIN_WIDTH and max(K, N) >= _FC_SPLIT_WIDTH)
-    if not ok or M >= 1 << 31:
-        return None
-    return _fc_parts(p, st, trans)
-
-
-def _fc_parts(p, st, trans=False):
-    K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
-    key, version = 'WST' if trans else 'WS', p['W']._version  # W may be the caller's own
-    if key not in p or p[key][0] != version:
-        parts = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, N), dtype=torch.uint8,
-                            device=p['W'].device)
-        call('vc_fc_split_pack', ptr(p['W']), K, N, 1 if trans else 0, ptr(parts), st)
-        p[key] = (version, parts)
-    return p[key][1]
+    return packs.fc(p, st, trans) if ok and M < 1 << 31 else None
 
 
 def _conv_interval_parts(p, K, st):
@@ -528,13 +538,13 @@ class _Gens:
         self.G, self.lam, self.lists, self.dense = G, lam, lists, dense
 
 
-def _zono_fc(p, g, B, K, st):
+def _zono_fc(packs, p, g, B, K, st):
     """(B, n_out, K + k) generators of a _Gens through an fc."""
     idx, idx_ld, mu, xl, xh, cnt, k = g.lists
     n, n_out, dev = p['n_in'], p['n_out'], p['W'].device
     out = torch.empty(B, n_out, K + k, device=dev)
     if K:
-        parts = _fc_parts(p, st, True)
+        parts = packs.fc(p, st, True)
         per = _lib.load().vc_fc_split_pack_bytes(n, K)
         work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)), dtype=torch.uint8,
                            device=dev)
@@ -559,6 +569,7 @@ def _zono_forward(xl, xh, gg, dtype, bounds_only):
     vidx = varying.nonzero(as_tuple=True)[0].to(torch.int32).contiguous()
     K = int(vidx.numel())
     ops = gg['ops']
+    packs = _Packs()
     users = {}
     for op in ops:
         for i in op['inputs']:
@@ -641,7 +652,7 @@ def _zono_forward(xl, xh, gg, dtype, bounds_only):
                 call('vc_zono_fc', ptr(c_in), None, B, p['n_in'], 0, ptr(p['W']), ptr(p['b']),
                      p['n_out'], ptr(c_o), None, st)
                 k = G_in.lists[-1]
-                state[name] = (c_o, _zono_fc(p, G_in, B, Kc - k, st))
+                state[name] = (c_o, _zono_fc(packs, p, G_in, B, Kc - k, st))
                 gen_count[name] = Kc
                 continue
             G_o = torch.empty(B, P * p['n_out'], Kc, device=dev)
@@ -669,10 +680,14 @@ def _zono_forward(xl, xh, gg, dtype, bounds_only):
                 sb[op['layer_idx']] = (lo, hi)
             if pos == top:
                 return sb, None
+            nxt = one_fc(name)
+            together = (nxt is not None
+                        and B * n * Kc * int(nxt['W'].shape[0]) >= _ZONO_SPLIT_MACS)
+            if together and Kc:
+                packs.fc(_op_params(nxt, dev), st, True)  # queued before the host waits
             k_new = int(cnt.max().item()) if B > 0 else 0
             c_o = torch.empty(B, n, device=dev)
-            nxt = one_fc(name)
-            if nxt is not None and B * n * Kc * int(nxt['W'].shape[0]) >= _ZONO_SPLIT_MACS:
+            if together:
                 lam = torch.empty(B, n, device=dev)
                 idx = torch.empty(B, max(k_new, 1), dtype=torch.int32, device=dev)
                 mu = torch.empty(B, max(k_new, 1), device=dev)
@@ -790,16 +805,19 @@ def _expand_rows(t, B):
 
 
 def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
-              alpha_at_layer=None, relu_split_beta=None, trace=None, split=True):
+              alpha_at_layer=None, relu_split_beta=None, trace=None, split=True,
+              packs=None):
     """Walk the ops backward from ``seed_name`` and concretize.
 
     seed: (R, n) rows when ``seed_shared`` else (B*R, n), or a _Rows; acc0:
     (R,) when shared else (B*R,).  split: products may run as bf16 parts on
     the matrix cores; off where the bounds choose slopes, whose step at 1/2
     turns a last-bit change of a bound into another lower slope (on 512 boxes
-    through 1024-wide layers one run in four).  Returns (lb (B, R), A, a_shared, acc (B*R,));
+    through 1024-wide layers one run in four).  packs: the caller's _Packs, where
+    it makes several of these calls.  Returns (lb (B, R), A, a_shared, acc (B*R,));
     A of window rows is None.
     """
+    packs = _Packs() if packs is None else packs
     B, n_in = xl.shape
     dev = xl.device
     st = stream()
@@ -1031,7 +1049,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 parts = None
                 if (split and M >= _FC_SPLIT_SWEEP_ROWS and rows.alpha_group is None
                         and not rows.alpha_row):
-                    parts = _fc_split_parts(p, M, st, sweep=trace is not None)
+                    parts = _fc_split_parts(packs, p, M, st, sweep=trace is not None)
                 if parts is not None:
                     ls, us, ut = slopes(rows)
                     work = _fc_split_work(M, p['n_out'], dev)
@@ -1345,7 +1363,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
 # --------------------------------------------------------------------------
 
 def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
-                             beta=None, gbeta=None, seed_name=None, want_A=False):
+                             beta=None, gbeta=None, seed_name=None, want_A=False, packs=None):
     """One alpha-CROWN evaluation: lb (B, Q); when ``want_grad`` also fills
     ``galpha[L]`` with d(sum lb)/d alpha_L (the autograd of the reference's
     backward, torch clamp subgradients included).  ``beta`` is the signed
@@ -1355,15 +1373,16 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
     shared rows Wq (Q, n) seed, as ``seed_ew_at`` does; an alpha_L of shape
     (B, Q, n_L) is one alpha per row (per-query alpha), and galpha_L then
     has that shape too.  ``want_A``: returns (lb, A) with A (B*Q, n_in) the
-    input linearization of the rows."""
+    input linearization of the rows.  ``packs``: the loop's _Packs."""
     B, n_in = xl.shape
+    packs = _Packs() if packs is None else packs
     Q = Wq.shape[0]
     dev = xl.device
     st = stream()
     trace = BackwardTrace() if want_grad else None
     seed = gg['ops'][-1]['name'] if seed_name is None else seed_name
     lb, A, a_shared, _ = _backward(sb, xl, xh, gg, seed, Wq,
-                                   True, bq, alpha, beta, trace)
+                                   True, bq, alpha, beta, trace, packs=packs)
     if want_A and (A is None or a_shared):
         raise NotImplementedError('vibecheck_amd: per-row linearization needs a relu')
     if not want_grad:
@@ -1385,7 +1404,7 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
     # input side: gE_0 = gA W_0^T + b_0, W_0 = fcs[-1]
     f0 = _op_params(fcs[-1], dev)
     g = torch.empty(M, f0['n_out'], device=dev)
-    parts = _fc_split_parts(f0, M, st, True)
+    parts = _fc_split_parts(packs, f0, M, st, True)
     if parts is not None:
         work = _fc_split_work(M, n_in, dev)
         call('vc_alpha_grad_input_split', ptr(A), ptr(xl), ptr(xh), M, Q, n_in, ptr(parts),
@@ -1430,7 +1449,7 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
                 ls, us, ut = (torch.empty(B, n, device=dev) for _ in range(3))
                 call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(a), B * n, ptr(ls),
                      ptr(us), ptr(ut), st)
-            parts = _fc_split_parts(fn, M, st, True)
+            parts = _fc_split_parts(packs, fn, M, st, True)
             if parts is not None:
                 work = _fc_split_work(M, n, dev)
                 call('vc_alpha_grad_step_split', ptr(g), ptr(P), M, Q, n, ptr(ls), ptr(us),
@@ -1507,9 +1526,10 @@ def _run_alpha_crown_inputsplit_batched(xl, xh, gg, spec_ew, device, dtype,
     n_eval = 0
     step = 0
     cur_lr = float(lr)
+    packs = _Packs()
     for it in range(n_iters):
         lb = _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, True,
-                                      galpha)
+                                      galpha, packs=packs)
         n_eval += 1
         call('vc_best_update', ptr(best), ptr(lb.contiguous()), B * Q,
              1 if it == 0 else 0, ptr(red), st)
