@@ -238,7 +238,8 @@ int vc_relax_slopes(const float *relu_lo, const float *relu_hi,
  * forms the rows' parts in work (vc_fc_split_pack_bytes(K, M) of them, 16-byte
  * aligned).  Slopes (M / R, K) as from vc_relax_slopes; packed: W's parts from
  * vc_fc_split_pack (vc_fc_split_pack_bytes(K, N), 16-byte aligned), of W (K, N)
- * or with trans of W (N, K) whose transpose is meant.  M < 2^31.
+ * or with trans of W (N, K) whose transpose is meant (vc_fc_split_pack_abs: of
+ * W and of |W|, from one pass).  M < 2^31.
  * vc_backward_fc_split: e = pos(x) lo_s + neg(x) up_s [+ beta (M / R, n_out)],
  *   ew_out (M, n_in) = e W, acc[m] += neg(x) . up_t + e . bias, x from row m or,
  *   with ew_shared, row m mod R.  Replaces verify_zono_bnb.py:4379-4453.
@@ -246,6 +247,8 @@ int vc_relax_slopes(const float *relu_lo, const float *relu_hi,
  *   vc_alpha_grad_step_slopes and vc_alpha_grad_input, with the packed transpose. */
 int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N);
 int vc_fc_split_pack(const float *W, int K, int N, int trans, void *out, vc_stream_t stream);
+int vc_fc_split_pack_abs(const float *W, int K, int N, int trans, void *out, void *out_abs,
+                         vc_stream_t stream);
 int vc_backward_fc_split(const float *ew_in, int64_t M, int R, int ew_shared, int n_out,
                          const float *lo_s, const float *up_s, const float *up_t,
                          const float *beta, const void *packed, const float *bias, int n_in,
@@ -291,8 +294,8 @@ int vc_ibp_fc_sliced(const float *l, const float *h, int64_t B, int n_in, const 
                      vc_stream_t stream);
 
 /* vc_ibp_conv on the bf16 matrix cores: packed_t and packed_abs_t are the parts of
- * the kernel (C_out, C_in kh kw) and of its magnitudes (vc_fc_split_pack with
- * trans).  work: any multiple of 2 vc_fc_split_pack_bytes(C_in kh kw, H_out
+ * the kernel (C_out, C_in kh kw) and of its magnitudes (vc_fc_split_pack_abs
+ * with trans).  work: any multiple of 2 vc_fc_split_pack_bytes(C_in kh kw, H_out
  * W_out), 16-byte aligned; as many boxes at a time. */
 int vc_ibp_conv_split(const float *l, const float *h, int64_t B, int C_in, int H, int W,
                       const void *packed_t, const void *packed_abs_t, const float *bias,

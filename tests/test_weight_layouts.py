@@ -10,12 +10,14 @@ import pytest
 import torch
 
 from vibecheck_amd import verify_zono_bnb as vz
+from vibecheck_amd import workloads as wk
 
 F32 = torch.float32
-# entry point: (weight, packed buffer) of a pack, packed operands of a product
-PACKS = {'vc_fc_split_pack': (0, 4)}
+# entry point: weight and packed buffers of a pack; packed operands of a product
+PACKS = {'vc_fc_split_pack': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5])}
 READS = {'vc_backward_fc_split': [9], 'vc_alpha_grad_step_split': [9],
-         'vc_alpha_grad_input_split': [6], 'vc_zono_fc_split': [5]}
+         'vc_alpha_grad_input_split': [6], 'vc_zono_fc_split': [5],
+         'vc_ibp_conv_split': [6, 7]}
 
 
 def _mlp(widths, dtype=F32, dev='cpu'):
@@ -36,10 +38,16 @@ def _mlp(widths, dtype=F32, dev='cpu'):
 MLP = [70, 140, 130, 9]
 
 
+def _cnn(dtype=F32, dev='cpu'):
+    return wk.cnn_gg([(32, 3, 1, 1), (40, 4, 2, 1), (33, 3, 1, 1)], [20, 9], (3, 17, 16), seed=2,
+                     device=dev, dtype=dtype)
+
+
 def _case(path, dtype=F32, dev='cpu'):
     """(gg, call) of a path whose products take packed weights."""
-    gg = _mlp(MLP, dtype, dev)
-    n_in, n_out, n_relu = gg['input_n'], 9, gg['n_relu']
+    cnn = path in ('ibp',)
+    gg = _cnn(dtype, dev) if cnn else _mlp(MLP, dtype, dev)
+    n_in, n_out = gg['input_n'], 9
     B = 256 if path == 'spec' else 16
     g = torch.Generator().manual_seed(3)
     xl = torch.rand(B, n_in, generator=g).to(dev)
@@ -48,8 +56,8 @@ def _case(path, dtype=F32, dev='cpu'):
         eye = torch.eye(n_out, device=dev)
         spec = {q: (eye[0] - eye[q + 1], 0.0) for q in range(n_out - 1)}
     sb = {}
-    for L in range(n_relu):
-        n = gg['ops'][2 * L]['W'].shape[0]
+    widths = vz.validate_gg(gg, n_in)
+    for L, n in enumerate(widths[op['name']] for op in gg['ops'] if op['type'] == 'relu'):
         lo = torch.randn(B, n, generator=g).to(dev) - 0.5
         sb[L] = (lo, lo + 2)
 
@@ -59,12 +67,15 @@ def _case(path, dtype=F32, dev='cpu'):
         if path == 'alpha':
             return [vz._run_alpha_crown_inputsplit_batched(xl, xh, gg, spec, dev, F32, n_iters=3,
                                                            sb=sb)]
+        if path == 'ibp':
+            bounds = vz._ibp_forward_graph_batched(xl, xh, gg, dev, F32)
+            return [t for b in bounds.values() for t in b]
         bounds, (c, G) = vz._forward_zonotope_graph_batched(xl, xh, gg, dev, F32)
         return [c, G] + [t for b in bounds.values() for t in b]
     return gg, run
 
 
-PATHS = ['spec', 'alpha', 'zono']
+PATHS = ['spec', 'alpha', 'zono', 'ibp']
 
 
 def _weights(gg):
@@ -75,6 +86,7 @@ def _weights(gg):
 def small(monkeypatch):
     """Every product from the smallest sizes on by the packed weights."""
     monkeypatch.setattr(vz, '_ZONO_SPLIT_MACS', 0)
+    monkeypatch.setattr(vz, '_IBP_SPLIT_MACS', 0)
 
 
 @pytest.fixture
@@ -84,8 +96,9 @@ def launches(monkeypatch, small):
 
     def call(name, *a):
         if name in PACKS:
-            src, out = (a[i] for i in PACKS[name])
-            rec['packed'][id(out)] = (out, a[-1], src, src.clone())
+            src, outs = PACKS[name]
+            for i in outs:
+                rec['packed'][id(a[i])] = (a[i], a[-1], a[src], a[src].clone())
         for i in READS.get(name, []):
             _, st, src, was = rec['packed'][id(a[i])]
             assert st == a[-1], f'{name} reads weights packed on another stream'

@@ -569,8 +569,9 @@ __global__ __launch_bounds__(FNT) void k_zono_cols(const float* W, int n_out, in
 
 // Wp[column tile][32-deep step][part][lane][8]: part of B[k][n] for
 // k = 32 step + 8 (lane / 16) + j, n = 16 tile + lane % 16; zero past the ends.
+// out_abs (or null): the same of |B|.
 __global__ void k_fc_split_pack(const float* W, int K, int N, int trans, int nkc, int64_t total,
-                                uint4* out) {
+                                uint4* out, uint4* out_abs) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
        t += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(t & 63);
@@ -589,7 +590,25 @@ __global__ void k_fc_split_pack(const float* W, int K, int N, int trans, int nkc
     o[0] = h;
     o[64] = m;
     o[128] = l;
+    if (!out_abs) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = fabsf(v[j]);
+    split8_all(v, h, m, l);
+    o = out_abs + q * kTileU + lane;
+    o[0] = h;
+    o[64] = m;
+    o[128] = l;
   }
+}
+
+int launch_pack(const float* W, int K, int N, int trans, void* out, void* out_abs,
+                hipStream_t st) {
+  const int nkc = 2 * ((K + 2 * FBK - 1) / (2 * FBK));
+  const int64_t total = (int64_t)((N + 15) / 16) * nkc * 64;
+  hipLaunchKernelGGL(k_fc_split_pack, dim3(vc_blocks(total, 256)), dim3(256), 0, st, W, K, N,
+                     trans, nkc, total, (uint4*)out, (uint4*)out_abs);
+  VC_LAUNCH_CHECK();
+  return VC_OK;
 }
 
 template <int FORM>
@@ -647,12 +666,14 @@ extern "C" int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N) {
 extern "C" int vc_fc_split_pack(const float* W, int K, int N, int trans, void* out,
                                 vc_stream_t stream) {
   if (!W || !out || K <= 0 || N <= 0 || !aligned16(out)) return VC_ERR_ARG;
-  const int nkc = 2 * ((K + 2 * FBK - 1) / (2 * FBK));
-  const int64_t total = (int64_t)((N + 15) / 16) * nkc * 64;
-  hipLaunchKernelGGL(k_fc_split_pack, dim3(vc_blocks(total, 256)), dim3(256), 0,
-                     (hipStream_t)stream, W, K, N, trans, nkc, total, (uint4*)out);
-  VC_LAUNCH_CHECK();
-  return VC_OK;
+  return launch_pack(W, K, N, trans, out, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int vc_fc_split_pack_abs(const float* W, int K, int N, int trans, void* out,
+                                    void* out_abs, vc_stream_t stream) {
+  if (!W || !out || !out_abs || K <= 0 || N <= 0 || !aligned16(out) || !aligned16(out_abs))
+    return VC_ERR_ARG;
+  return launch_pack(W, K, N, trans, out, out_abs, (hipStream_t)stream);
 }
 
 extern "C" int vc_backward_fc_split(const float* ew_in, int64_t M, int R, int ew_shared, int n_out,

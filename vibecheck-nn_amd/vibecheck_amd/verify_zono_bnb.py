@@ -239,6 +239,18 @@ class _Packs:
             self._made[p['name'], trans] = out
         return out
 
+    def conv_interval(self, p, K, st):
+        """The parts of a conv's kernel and of its magnitudes for
+        vc_ibp_conv_split."""
+        out = self._made.get((p['name'], 'interval'))
+        if out is None:
+            n = p['K'].shape[0]
+            out = [torch.empty(_lib.load().vc_fc_split_pack_bytes(K, n), dtype=torch.uint8,
+                               device=p['K'].device) for _ in range(2)]
+            call('vc_fc_split_pack_abs', ptr(p['K']), K, n, 1, ptr(out[0]), ptr(out[1]), st)
+            self._made[p['name'], 'interval'] = out
+        return out
+
 
 def _fc_split_parts(packs, p, M, st, trans=False, sweep=False):
     """The fc weights' bf16 parts for M rows' vc_backward_fc_split (``trans``:
@@ -252,22 +264,6 @@ def _fc_split_parts(packs, p, M, st, trans=False, sweep=False):
         ok = (M >= (_FC_SPLIT_SWEEP_ROWS if sweep else _FC_SPLIT_ROWS)
               and K >= _TWO_PHASE_MIN_WIDTH and max(K, N) >= _FC_SPLIT_WIDTH)
     return packs.fc(p, st, trans) if ok and M < 1 << 31 else None
-
-
-def _conv_interval_parts(p, K, st):
-    """The parts of a conv's kernel and of its magnitudes for vc_ibp_conv_split,
-    cached with the op's other device tensors."""
-    version = p['K']._version  # the kernel may be the caller's own
-    if 'KI' not in p or p['KI'][0] != version:
-        n = p['K'].shape[0]
-        parts = []
-        for k in (p['K'], p['K'].abs()):
-            out = torch.empty(_lib.load().vc_fc_split_pack_bytes(K, n), dtype=torch.uint8,
-                              device=k.device)
-            call('vc_fc_split_pack', ptr(k), K, n, 1, ptr(out), st)
-            parts.append(out)
-        p['KI'] = (version, parts)
-    return p['KI'][1]
 
 
 def _fc_split_work(M, K, dev):
@@ -405,6 +401,7 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
     hi = {gg['input_name']: xh}
     sb = {}
     st = stream()
+    packs = _Packs()
     # nodes without a relu below them: their intervals are exact, CROWN's first
     # bounds equal them up to rounding and choose slopes by the larger of the
     # two, so their sums keep their order
@@ -442,7 +439,7 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
             K = C_in * kh * kw
             if (name not in raw and K >= 512 and C_out > 32
                     and B * p['n_out'] * K >= _IBP_SPLIT_MACS):
-                parts = _conv_interval_parts(p, K, st)
+                parts = packs.conv_interval(p, K, st)
                 per = 2 * _lib.load().vc_fc_split_pack_bytes(K, Ho * Wo)
                 work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)),
                                    dtype=torch.uint8, device=dev)
