@@ -14,10 +14,12 @@ from vibecheck_amd import workloads as wk
 
 F32 = torch.float32
 # entry point: weight and packed buffers of a pack; packed operands of a product
-PACKS = {'vc_fc_split_pack': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5])}
+PACKS = {'vc_fc_split_pack': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5]),
+         'vc_conv_split_pack': (0, [7]), 'vc_conv_t_pack': (0, [9])}
 READS = {'vc_backward_fc_split': [9], 'vc_alpha_grad_step_split': [9],
          'vc_alpha_grad_input_split': [6], 'vc_zono_fc_split': [5],
-         'vc_ibp_conv_split': [6, 7]}
+         'vc_ibp_conv_split': [6, 7], 'vc_backward_conv_split': [9],
+         'vc_backward_conv_packed': [3]}
 
 
 def _mlp(widths, dtype=F32, dev='cpu'):
@@ -45,10 +47,10 @@ def _cnn(dtype=F32, dev='cpu'):
 
 def _case(path, dtype=F32, dev='cpu'):
     """(gg, call) of a path whose products take packed weights."""
-    cnn = path in ('ibp',)
+    cnn = path in ('ibp', 'crown_cnn', 'spec_cnn')
     gg = _cnn(dtype, dev) if cnn else _mlp(MLP, dtype, dev)
     n_in, n_out = gg['input_n'], 9
-    B = 256 if path == 'spec' else 16
+    B = 256 if path == 'spec' else 4 if path == 'crown_cnn' else 16
     g = torch.Generator().manual_seed(3)
     xl = torch.rand(B, n_in, generator=g).to(dev)
     xh = xl + 0.1
@@ -62,7 +64,7 @@ def _case(path, dtype=F32, dev='cpu'):
         sb[L] = (lo, lo + 2)
 
     def run():
-        if path == 'spec':
+        if path in ('spec', 'spec_cnn'):
             return [vz._spec_backward_graph_batched(sb, xl, xh, gg, spec, dev, F32)]
         if path == 'alpha':
             return [vz._run_alpha_crown_inputsplit_batched(xl, xh, gg, spec, dev, F32, n_iters=3,
@@ -70,12 +72,15 @@ def _case(path, dtype=F32, dev='cpu'):
         if path == 'ibp':
             bounds = vz._ibp_forward_graph_batched(xl, xh, gg, dev, F32)
             return [t for b in bounds.values() for t in b]
+        if path == 'crown_cnn':
+            bounds = vz._crown_intermediate_batched(gg, xl, xh, dev, F32, chunk=512, sb=sb)
+            return [t for b in bounds.values() for t in b]
         bounds, (c, G) = vz._forward_zonotope_graph_batched(xl, xh, gg, dev, F32)
         return [c, G] + [t for b in bounds.values() for t in b]
     return gg, run
 
 
-PATHS = ['spec', 'alpha', 'zono', 'ibp']
+PATHS = ['spec', 'alpha', 'zono', 'ibp', 'crown_cnn', 'spec_cnn']
 
 
 def _weights(gg):

@@ -180,43 +180,6 @@ def _widths(gg, n_in):
     return w
 
 
-def _conv_t_taps(p, st, window=False):
-    """The conv kernel's transposed taps packed per output-parity class
-    (vc_conv_t_pack), made on first use by a backward pass and cached with
-    the op's other device tensors; ``window``: without the padding, for rows
-    that carry their place in the image."""
-    key = 'KT_window' if window else 'KT'
-    packed = p.get(key)
-    if packed is None:
-        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        n = _lib.load().vc_conv_t_pack_floats(C_out, C_in, kh, kw, sh, sw)
-        if n < 0:
-            raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {p["geom"]}')
-        packed = torch.empty(n, device=p['K'].device)
-        if window:
-            ph = pw = 0
-        call('vc_conv_t_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ph, pw,
-             ptr(packed), st)
-        p[key] = packed
-    return packed
-
-
-def _conv_split_parts(p, st):
-    """The conv kernel's bf16 parts for vc_backward_conv_split, made on first
-    use by a backward pass and cached with the op's other device tensors;
-    None where the geometry is outside that kernel."""
-    if 'KS' not in p:
-        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        p['KS'] = None
-        if _lib.load().vc_backward_conv_split_ok(C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph,
-                                                 pw):
-            n = _lib.load().vc_conv_split_pack_bytes(C_out, C_in, kh, kw, sh, sw)
-            parts = torch.empty(n, dtype=torch.uint8, device=p['K'].device)
-            call('vc_conv_split_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ptr(parts), st)
-            p['KS'] = parts
-    return p['KS']
-
-
 class _Packs:
     """The weights in the layouts that one call's products read.  Each is made
     on first use, on the call's stream, from the weights as they are then, and
@@ -249,6 +212,41 @@ class _Packs:
                                device=p['K'].device) for _ in range(2)]
             call('vc_fc_split_pack_abs', ptr(p['K']), K, n, 1, ptr(out[0]), ptr(out[1]), st)
             self._made[p['name'], 'interval'] = out
+        return out
+
+    def conv_taps(self, p, st, window=False):
+        """A conv kernel's transposed taps by output-parity class
+        (vc_conv_t_pack); ``window``: without the padding, for rows that carry
+        their place in the image."""
+        out = self._made.get((p['name'], 'taps', window))
+        if out is None:
+            C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+            n = _lib.load().vc_conv_t_pack_floats(C_out, C_in, kh, kw, sh, sw)
+            if n < 0:
+                raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {p["geom"]}')
+            out = torch.empty(n, device=p['K'].device)
+            if window:
+                ph = pw = 0
+            call('vc_conv_t_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ph, pw,
+                 ptr(out), st)
+            self._made[p['name'], 'taps', window] = out
+        return out
+
+    def conv_split(self, p, st):
+        """A conv kernel's bf16 parts for vc_backward_conv_split; None where
+        the geometry is outside that kernel."""
+        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+        if 'conv_split_ok' not in p:
+            p['conv_split_ok'] = bool(_lib.load().vc_backward_conv_split_ok(
+                C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw))
+        if not p['conv_split_ok']:
+            return None
+        out = self._made.get((p['name'], 'conv_split'))
+        if out is None:
+            n = _lib.load().vc_conv_split_pack_bytes(C_out, C_in, kh, kw, sh, sw)
+            out = torch.empty(n, dtype=torch.uint8, device=p['K'].device)
+            call('vc_conv_split_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ptr(out), st)
+            self._made[p['name'], 'conv_split'] = out
         return out
 
 
@@ -947,7 +945,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              st)
         out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
                     and rows.relu is None)
-        call('vc_backward_conv_packed', ptr(rel), M, ptr(p['K']), ptr(_conv_t_taps(p, st, True)),
+        call('vc_backward_conv_packed', ptr(rel), M, ptr(p['K']), ptr(packs.conv_taps(p, st, True)),
              ptr(p['b']), C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0, ptr(out.ew),
              ptr(acc), st)
         origin = torch.empty_like(w.origin)
@@ -963,7 +961,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
             return None
         fold = few_channels(p)
-        parts = None if fold or not split else _conv_split_parts(p, st)
+        parts = None if fold or not split else packs.conv_split(p, st)
         if not fold and parts is None:
             return None
         ls, us, ut = slopes(rows)
@@ -1140,7 +1138,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 per_domain_acc()
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
-            parts = None if not split or few_channels(p) else _conv_split_parts(p, st)
+            parts = None if not split or few_channels(p) else packs.conv_split(p, st)
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
                      ptr(p['K']), ptr(parts), ptr(p['b']), C_out, Ho, Wo, C_in, H, W, kh, kw,
@@ -1148,7 +1146,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 put(inp, _Rows(out, rows.shared))
                 continue
             call('vc_backward_conv_packed', ptr(rows.ew), M, ptr(p['K']),
-                 ptr(_conv_t_taps(p, st)), ptr(p['b']), C_out, Ho, Wo, C_in, H, W,
+                 ptr(packs.conv_taps(p, st)), ptr(p['b']), C_out, Ho, Wo, C_in, H, W,
                  kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
             put(inp, _Rows(out, rows.shared))
         elif t == 'reshape':
@@ -1302,6 +1300,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
                  if op['type'] == 'relu' and 'layer_idx' in op}
     B = xl.shape[0]
     st = stream()
+    packs = _Packs()
     ch = max(1, int(chunk))
     for L in sorted(tight):
         if L not in relu_by_L:
@@ -1338,7 +1337,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
                      st)
                 rows.window = _Window(origin, kh, kw, C_in, H, W)
                 sl, _, _, _ = _backward(tight, xl, xh, gg, below, rows, True, acc0,
-                                        split=False)
+                                        split=False, packs=packs)
                 call('vc_crown_intersect', ptr(sl.contiguous()), ptr(cidx), k, B, n,
                      ptr(new_lo), ptr(new_hi), st)
                 continue
@@ -1347,7 +1346,8 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
             seed[ar, cidx.long()] = 1.0
             seed[ar + k, cidx.long()] = -1.0
             acc0 = torch.zeros(2 * k, device=dev)
-            sl, _, _, _ = _backward(tight, xl, xh, gg, feed, seed, True, acc0, split=False)
+            sl, _, _, _ = _backward(tight, xl, xh, gg, feed, seed, True, acc0, split=False,
+                                    packs=packs)
             sl = sl.contiguous()
             call('vc_crown_intersect', ptr(sl), ptr(cidx), k, B, n,
                  ptr(new_lo), ptr(new_hi), st)
