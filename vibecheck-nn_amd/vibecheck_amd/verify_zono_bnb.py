@@ -895,16 +895,32 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              ptr(acc), st)
         return _Rows(out, False)
 
-    def few_channels(p):
-        """Whether the conv is the fold kernel's (vc_backward_relu_conv): a
-        few input channels, the network's first layer."""
-        ok = p.get('relu_conv_ok')
-        if ok is None:
+    def few_channels(p, window=None):
+        """Whether the conv (of windows: (rows' height and width, the result's))
+        is the fold kernel's: a few input channels, the network's first layer."""
+        key = ('fold_ok', window)
+        if key not in p:
             C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-            ok = bool(_lib.load().vc_backward_relu_conv_ok(C_out, Ho, Wo, C_in, H, W, kh, kw,
-                                                           sh, sw, ph, pw))
-            p['relu_conv_ok'] = ok
-        return ok
+            if window is not None:
+                (Ho, Wo, H, W), ph, pw = window, 0, 0
+            p[key] = bool(_lib.load().vc_backward_relu_conv_ok(C_out, Ho, Wo, C_in, H, W, kh, kw,
+                                                               sh, sw, ph, pw))
+        return p[key]
+
+    def conv_fp32(p, ew, M, window, out):
+        """M rows through a conv in fp32, acc += rows . bias; the fold kernel
+        reads the kernel as it lies, the gathering product its packed taps."""
+        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+        if window is not None:
+            (Ho, Wo, H, W), ph, pw = window, 0, 0
+        geom = (C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
+        if few_channels(p, window):
+            call('vc_backward_conv', ptr(ew), M, ptr(p['K']), ptr(p['b']), *geom, ptr(out),
+                 ptr(acc), st)
+        else:
+            call('vc_backward_conv_packed', ptr(ew), M, ptr(p['K']),
+                 ptr(packs.conv_taps(p, st, window is not None)), ptr(p['b']), *geom, ptr(out),
+                 ptr(acc), st)
 
     def slopes(rows):
         """The pending relu's slopes per (domain, neuron) for a conv that
@@ -945,9 +961,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              st)
         out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
                     and rows.relu is None)
-        call('vc_backward_conv_packed', ptr(rel), M, ptr(p['K']), ptr(packs.conv_taps(p, st, True)),
-             ptr(p['b']), C_out, w.wh, w.ww, C_in, oh, ow, kh, kw, sh, sw, 0, 0, ptr(out.ew),
-             ptr(acc), st)
+        conv_fp32(p, rel, M, (w.wh, w.ww, oh, ow), out.ew)
         origin = torch.empty_like(w.origin)
         call('vc_patch_shift', ptr(w.origin), R, sh, sw, ph, pw, ptr(origin), st)
         out.window = _Window(origin, oh, ow, C_in, H, W)
@@ -1145,9 +1159,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                      sh, sw, ph, pw, ptr(out), ptr(acc), st)
                 put(inp, _Rows(out, rows.shared))
                 continue
-            call('vc_backward_conv_packed', ptr(rows.ew), M, ptr(p['K']),
-                 ptr(packs.conv_taps(p, st)), ptr(p['b']), C_out, Ho, Wo, C_in, H, W,
-                 kh, kw, sh, sw, ph, pw, ptr(out), ptr(acc), st)
+            conv_fp32(p, rows.ew, M, None, out)
             put(inp, _Rows(out, rows.shared))
         elif t == 'reshape':
             put(inp, rows)
