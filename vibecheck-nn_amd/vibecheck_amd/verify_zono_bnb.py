@@ -862,6 +862,20 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             call('vc_rows_bias_dot', ptr(rows.ew), B * R, R, n, 1 if rows.shared else 0,
                  ptr(v), v.numel(), sign, ptr(acc), st)
 
+    def bias_acc(rows, p):
+        """The bias and the constant terms that a product of rows without a
+        pending relu adds rows . bias to.  Shared rows add it once, to shared
+        terms; where another branch has given every domain its own by then, it
+        is added to all of them here and the product adds none."""
+        if rows.shared:
+            if not acc_shared:
+                if p['b'] is not None:
+                    bias_dot(rows, p['b'].repeat_interleave(p['n_out'] // p['b'].numel()), 1.0)
+                return None, None
+        else:
+            per_domain_acc()
+        return p['b'], acc
+
     def dense(rows):
         """Window rows as whole images (other rows as they are)."""
         w = rows.window
@@ -907,7 +921,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                                                                sh, sw, ph, pw))
         return p[key]
 
-    def conv_fp32(p, ew, M, window, out):
+    def conv_fp32(p, ew, M, window, out, bias, acc):
         """M rows through a conv in fp32, acc += rows . bias; the fold kernel
         reads the kernel as it lies, the gathering product its packed taps."""
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
@@ -915,11 +929,11 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             (Ho, Wo, H, W), ph, pw = window, 0, 0
         geom = (C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
         if few_channels(p, window):
-            call('vc_backward_conv', ptr(ew), M, ptr(p['K']), ptr(p['b']), *geom, ptr(out),
+            call('vc_backward_conv', ptr(ew), M, ptr(p['K']), ptr(bias), *geom, ptr(out),
                  ptr(acc), st)
         else:
             call('vc_backward_conv_packed', ptr(ew), M, ptr(p['K']),
-                 ptr(packs.conv_taps(p, st, window is not None)), ptr(p['b']), *geom, ptr(out),
+                 ptr(packs.conv_taps(p, st, window is not None)), ptr(bias), *geom, ptr(out),
                  ptr(acc), st)
 
     def slopes(rows):
@@ -946,14 +960,16 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         oh, ow = (w.wh - 1) * sh + kh, (w.ww - 1) * sw + kw
         if (not w.worth() or rows.alpha_group is not None
                 or (rows.alpha is not None and rows.alpha_row)
+                or (rows.shared and rows.relu is None and not acc_shared)
                 or B * R * C_in * oh * ow >= 1 << 31):
             return None
         ls = us = ut = beta = None
         if rows.relu is not None:
             ls, us, ut = slopes(rows)
             beta = rows.beta
-        elif not rows.shared:
-            per_domain_acc()
+            bias, acc_b = p['b'], acc
+        else:
+            bias, acc_b = bias_acc(rows, p)
         M = R if rows.shared and rows.relu is None else B * R
         rel = torch.empty(M, C_out * w.wh * w.ww, device=dev)
         call('vc_patch_relax', ptr(rows.ew), M, R, 1 if rows.shared else 0, ptr(ls), ptr(us),
@@ -961,7 +977,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              st)
         out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
                     and rows.relu is None)
-        conv_fp32(p, rel, M, (w.wh, w.ww, oh, ow), out.ew)
+        conv_fp32(p, rel, M, (w.wh, w.ww, oh, ow), out.ew, bias, acc_b)
         origin = torch.empty_like(w.origin)
         call('vc_patch_shift', ptr(w.origin), R, sh, sw, ph, pw, ptr(origin), st)
         out.window = _Window(origin, oh, ow, C_in, H, W)
@@ -1095,15 +1111,14 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 del rel
                 put(inp, _Rows(out, False))
             else:
-                if not rows.shared:
-                    per_domain_acc()
+                bias, acc_b = bias_acc(rows, p)
                 M = R if rows.shared else B * R
                 out = torch.empty(M, p['n_in'], device=dev)
                 if trace is not None:
                     trace.fcs.append(op)
                 call('vc_backward_fc', ptr(rows.ew), M, R, p['n_out'], None,
-                     None, None, 0, None, ptr(p['W']), ptr(p['b']),
-                     p['n_in'], ptr(out), ptr(acc), None, 0, st)
+                     None, None, 0, None, ptr(p['W']), ptr(bias),
+                     p['n_in'], ptr(out), ptr(acc_b), None, 0, st)
                 put(inp, _Rows(out, rows.shared))
         elif t == 'relu':
             if 'layer_idx' in op:
@@ -1148,18 +1163,17 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                     continue
             rows = materialize(rows)
             C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-            if not rows.shared:
-                per_domain_acc()
+            bias, acc_b = bias_acc(rows, p)
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
             parts = None if not split or few_channels(p) else packs.conv_split(p, st)
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
-                     ptr(p['K']), ptr(parts), ptr(p['b']), C_out, Ho, Wo, C_in, H, W, kh, kw,
-                     sh, sw, ph, pw, ptr(out), ptr(acc), st)
+                     ptr(p['K']), ptr(parts), ptr(bias), C_out, Ho, Wo, C_in, H, W, kh, kw,
+                     sh, sw, ph, pw, ptr(out), ptr(acc_b), st)
                 put(inp, _Rows(out, rows.shared))
                 continue
-            conv_fp32(p, rows.ew, M, None, out)
+            conv_fp32(p, rows.ew, M, None, out, bias, acc_b)
             put(inp, _Rows(out, rows.shared))
         elif t == 'reshape':
             put(inp, rows)
