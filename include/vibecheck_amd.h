@@ -375,14 +375,18 @@ int vc_backward_relu_conv(const float *ew_in, int64_t M, int64_t R, int ew_share
  * packed: the kernel's parts from vc_conv_split_pack (16-byte aligned,
  * vc_conv_split_pack_bytes of them), laid out once per kernel; kernel itself is
  * read where an infinity or NaN among the values asks for the plain sum.
- * vc_backward_conv_split_ok says whether a geometry qualifies, else
- * VC_ERR_UNSUPPORTED.
+ * vc_backward_conv_split_ok says whether a geometry qualifies (for one row),
+ * vc_backward_conv_split_fits whether M of them do (one tile's images, or the R
+ * shared rows, within 32-bit offsets), else VC_ERR_UNSUPPORTED.
  * Replaces verify_zono_bnb.py:4409-4453 followed by 4568-4593. */
 int64_t vc_conv_split_pack_bytes(int C_out, int C_in, int kh, int kw, int sh, int sw);
 int vc_conv_split_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,
                        int sw, void *out, vc_stream_t stream);
 int vc_backward_conv_split_ok(int C_out, int H_out, int W_out, int C_in, int H, int W,
                               int kh, int kw, int sh, int sw, int ph, int pw);
+int vc_backward_conv_split_fits(int64_t M, int64_t R, int ew_shared, int C_out, int H_out,
+                                int W_out, int C_in, int H, int W, int kh, int kw, int sh,
+                                int sw, int ph, int pw);
 int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shared,
                            const float *lo_s, const float *up_s, const float *up_t,
                            const float *beta, const float *kernel, const void *packed,

@@ -522,17 +522,21 @@ const void* pick_kernel(int MT, int gs, bool relu, bool comp) {
   return gs <= 2 ? inst<4, 2>(relu) : (gs <= 4 ? inst<4, 4> : inst<4, 8>)(relu);
 }
 
-int launch_split(SplitArgs& a, hipStream_t st) {
-  const int cus = vcm::cu_count();
-  if (!split_plan(a, a.M, cus)) return VC_ERR_UNSUPPORTED;
+// The plan for the rows at hand; false: outside the kernel's limits.
+bool split_fits(SplitArgs& a) {
+  if (!split_plan(a, a.M, vcm::cu_count())) return false;
   a.TI = CNT / a.G;
   a.n_tiles = (a.M + a.G - 1) / a.G * a.cib;
-  if (a.M >= (int64_t(1) << 31) || a.n_tiles >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+  if (a.M >= (int64_t(1) << 31) || a.n_tiles >= (int64_t(1) << 31)) return false;
   // the loads' byte offsets are 32-bit: one tile's images, or all shared rows
   const int64_t n_e = (int64_t)a.C_out * a.Hs * a.Ws, n_i = (int64_t)a.C_out * a.Hi * a.Wi;
-  if ((a.shared ? a.R : a.G) * n_e * 4 >= 0xf0000000ll || (a.G + 1) * n_i * 4 >= 0xf0000000ll ||
-      (int64_t)a.G * a.MTp * 16 * a.H * a.W * 4 >= 0x7fffffffll)
-    return VC_ERR_UNSUPPORTED;
+  return (a.shared ? a.R : a.G) * n_e * 4 < 0xf0000000ll && (a.G + 1) * n_i * 4 < 0xf0000000ll &&
+         (int64_t)a.G * a.MTp * 16 * a.H * a.W * 4 < 0x7fffffffll;
+}
+
+int launch_split(SplitArgs& a, hipStream_t st) {
+  const int cus = vcm::cu_count();
+  if (!split_fits(a)) return VC_ERR_UNSUPPORTED;
   a.f_cw = FastDiv::make((uint32_t)(a.Hc * a.Wc));
   a.f_wc = FastDiv::make((uint32_t)a.Wc);
   a.f_npx = FastDiv::make((uint32_t)(a.Hb * a.Ws));
@@ -711,6 +715,19 @@ extern "C" int vc_backward_conv_split_ok(int C_out, int H_out, int W_out, int C_
   a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.C_in = C_in, a.H = H, a.W = W;
   a.kh = kh, a.kw = kw, a.sh = sh, a.sw = sw, a.ph = ph, a.pw = pw;
   return split_plan(a, 1, 1) ? 1 : 0;
+}
+
+extern "C" int vc_backward_conv_split_fits(int64_t M, int64_t R, int ew_shared, int C_out,
+                                           int H_out, int W_out, int C_in, int H, int W, int kh,
+                                           int kw, int sh, int sw, int ph, int pw) {
+  if (!geom_ok(C_out, H_out, W_out, C_in, H, W, kh, kw, sh, sw, ph, pw) || M <= 0 || R <= 0)
+    return 0;
+  SplitArgs a{};
+  a.M = M, a.R = R, a.shared = ew_shared ? 1 : 0;
+  a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_out, a.Wi = W_out;
+  a.C_in = C_in, a.H = H, a.W = W;
+  a.kh = kh, a.kw = kw, a.sh = sh, a.sw = sw, a.ph = ph, a.pw = pw;
+  return split_fits(a) ? 1 : 0;
 }
 
 extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, int ew_shared,

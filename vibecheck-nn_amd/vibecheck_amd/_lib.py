@@ -61,6 +61,7 @@ SIGNATURES = {
     'vc_conv_split_pack_bytes': [_I, _I, _I, _I, _I, _I],
     'vc_conv_split_pack': [_P, _I, _I, _I, _I, _I, _I, _P, _P],
     'vc_backward_conv_split_ok': [_I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I],
+    'vc_backward_conv_split_fits': [_L, _L, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I],
     'vc_backward_conv_split': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                _I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
     'vc_fc_split_pack_bytes': [_L, _L],

@@ -232,14 +232,13 @@ class _Packs:
             self._made[p['name'], 'taps', window] = out
         return out
 
-    def conv_split(self, p, st):
-        """A conv kernel's bf16 parts for vc_backward_conv_split; None where
-        the geometry is outside that kernel."""
+    def conv_split(self, p, M, R, shared, st):
+        """A conv kernel's bf16 parts for vc_backward_conv_split of M rows (R a
+        domain, shared by all domains or not); None where the geometry or the
+        rows are outside that kernel."""
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        if 'conv_split_ok' not in p:
-            p['conv_split_ok'] = bool(_lib.load().vc_backward_conv_split_ok(
-                C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw))
-        if not p['conv_split_ok']:
+        if not _lib.load().vc_backward_conv_split_fits(M, R, 1 if shared else 0, C_out, Ho, Wo,
+                                                       C_in, H, W, kh, kw, sh, sw, ph, pw):
             return None
         out = self._made.get((p['name'], 'conv_split'))
         if out is None:
@@ -436,7 +435,9 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
             hi_o = torch.empty_like(lo_o)
             K = C_in * kh * kw
             if (name not in raw and K >= 512 and C_out > 32
-                    and B * p['n_out'] * K >= _IBP_SPLIT_MACS):
+                    and B * p['n_out'] * K >= _IBP_SPLIT_MACS
+                    and Ho * Wo < 1 << 24 and K < 1 << 24 and H * W < 1 << 28
+                    and p['n_in'] < 1 << 31):
                 parts = packs.conv_interval(p, K, st)
                 per = 2 * _lib.load().vc_fc_split_pack_bytes(K, Ho * Wo)
                 work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)),
@@ -991,7 +992,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
             return None
         fold = few_channels(p)
-        parts = None if fold or not split else packs.conv_split(p, st)
+        parts = (None if fold or not split
+                 else packs.conv_split(p, B * R, R, rows.shared, st))
         if not fold and parts is None:
             return None
         ls, us, ut = slopes(rows)
@@ -1166,7 +1168,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             bias, acc_b = bias_acc(rows, p)
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
-            parts = None if not split or few_channels(p) else packs.conv_split(p, st)
+            parts = (None if not split or few_channels(p)
+                     else packs.conv_split(p, M, M, False, st))
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
                      ptr(p['K']), ptr(parts), ptr(bias), C_out, Ho, Wo, C_in, H, W, kh, kw,
