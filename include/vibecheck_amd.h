@@ -269,8 +269,9 @@ int vc_alpha_grad_input_split(const float *A, const float *xl, const float *xh, 
  *   size mu[b k_new + j].
  * vc_zono_fc_split: G_out[b][o][j] = sum over k of W[o][k] lam[b][k] G[b][k][j]
  *   for the K old columns, rows of G_out ld apart, on the bf16 matrix cores
- *   (packed_t: W's parts, vc_fc_split_pack with trans).  work: any multiple of
- *   vc_fc_split_pack_bytes(n, K), 16-byte aligned; as many domains at a time.
+ *   (packed_t: W's parts, vc_fc_split_pack with trans).  work (16-byte aligned):
+ *   as many domains at a time as it holds parts of, vc_fc_split_pack_bytes(n, K)
+ *   each, or 64-column pieces of one; at least vc_fc_split_pack_bytes(n, 64).
  * vc_zono_fc_cols: G_out[b][o][k0 + j] = W[o][idx[b idx_ld + j]] mu[same] for
  *   j < cnt[b] (NULL: k), zero for the others up to k; mu NULL: the sizes are
  *   (xh - xl) / 2 of neuron idx (the input's generators).

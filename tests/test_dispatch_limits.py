@@ -1,5 +1,6 @@
-"""Sizes past a kernel's 32-bit limits go to the kernels that take them.  Host
-logic only: tensors without storage, launches recorded instead of run."""
+"""Sizes past a kernel's 32-bit limits go to the kernels that take them, and the
+part products' scratch stays bounded.  Host logic only: tensors without storage,
+launches recorded instead of run."""
 import pytest
 import torch
 
@@ -52,7 +53,7 @@ def test_shared_rows_past_4_gib(launches, rows, alone):
     assert 'vc_backward_conv_split' in launches
 
 
-@pytest.mark.parametrize('side,entry', [(512, 'vc_ibp_conv_split'), (4097, 'vc_ibp_conv')])
+@pytest.mark.parametrize('side,entry', [(256, 'vc_ibp_conv_split'), (4097, 'vc_ibp_conv')])
 def test_interval_conv_of_many_pixels(launches, monkeypatch, side, entry):
     """2^24 pixels and more."""
     monkeypatch.setattr(vz, '_IBP_SPLIT_MACS', 0)
@@ -74,3 +75,70 @@ def test_split_conv_limits():
     assert not lib.vc_backward_conv_split_fits(2 * (most + 1), most + 1, 1, *geom)
     assert lib.vc_backward_conv_split_fits(2 * (most + 1), most + 1, 0, *geom)
     assert not lib.vc_backward_conv_split_fits(1 << 31, 1, 0, *geom)
+
+
+# argument of the buffer of parts
+WORK = {'vc_backward_fc_split': 14, 'vc_alpha_grad_step_split': 13,
+        'vc_alpha_grad_input_split': 10, 'vc_zono_fc_split': 9, 'vc_ibp_conv_split': 20}
+
+
+@pytest.fixture
+def scratch(monkeypatch, launches):
+    """(name, bytes of parts, rows) of each part product."""
+    rec = []
+
+    def call(name, *a):
+        if name in WORK:
+            rec.append((name, a[WORK[name]].numel(), a[1 if name == 'vc_backward_fc_split' else
+                                                      3 if 'input' in name else 2]))
+        elif name == 'vc_unstable_union':
+            raise AssertionError(name)
+    monkeypatch.setattr(vz, 'call', call)
+    return rec
+
+
+def _mlp(widths):
+    ops, prev = [], 'X'
+    for i, (a, b) in enumerate(zip(widths, widths[1:])):
+        ops.append({'name': f'fc{i}', 'type': 'fc', 'inputs': [prev], 'bias': None,
+                    'W': torch.empty(b, a, device=META)})
+        prev = f'fc{i}'
+        if i + 2 < len(widths):
+            ops.append({'name': f'r{i}', 'type': 'relu', 'inputs': [prev], 'layer_idx': i})
+            prev = f'r{i}'
+    return {'ops': ops, 'input_name': 'X', 'input_n': widths[0], 'fork_points': set(),
+            'input_shape': (1, widths[0]), 'n_relu': len(widths) - 2}
+
+
+@pytest.mark.parametrize('B,Q', [(300000, 9), (3, 700000), (1 << 20, 1)])
+def test_alpha_gradient_scratch(scratch, B, Q):
+    """Rows whose relaxed form takes 10 GB and more: the parts 512 MiB at a time,
+    every row once, and no slopes held past 32 MiB a layer."""
+    gg = _mlp([784, 1000, 1000, 10])
+    x = torch.empty(B, 784, device=META)
+    sb = {L: (torch.empty(B, 1000, device=META),) * 2 for L in (0, 1)}
+    alpha = {L: torch.empty(B, 1000, device=META) for L in (0, 1)}
+    traces = []
+    init = vz.BackwardTrace.__init__
+    vz.BackwardTrace.__init__ = lambda self: (init(self), traces.append(self))[0]
+    try:
+        vz._alpha_backward_and_grad(sb, x, x, gg, torch.empty(Q, 10, device=META),
+                                    torch.empty(Q, device=META), alpha, True, alpha)
+    finally:
+        vz.BackwardTrace.__init__ = init
+    assert max(n for _, n, _ in scratch) <= 512 << 20
+    for name, per in (('vc_backward_fc_split', 2), ('vc_alpha_grad_step_split', 1),
+                      ('vc_alpha_grad_input_split', 1)):
+        assert sum(m for n, _, m in scratch if n == name) == per * B * Q
+    assert sum(t.numel() * 4 for s in traces[0].slopes.values() for t in s) <= 2 * (32 << 20)
+
+
+def test_interval_conv_scratch(scratch, monkeypatch):
+    """One box whose parts would take 7 GB stays with the gathering product."""
+    monkeypatch.setattr(vz, '_IBP_SPLIT_MACS', 0)
+    for side, n in ((64, 1), (1024, 0)):
+        gg = _net(side, [(64, 1), None, (33, 3)])
+        x = torch.empty(2, side * side, device=META)
+        del scratch[:]
+        vz._ibp_forward_graph_batched(x, x, gg, META, torch.float32)
+        assert len(scratch) == n and all(b <= 1 << 30 for _, b, _ in scratch)

@@ -484,17 +484,18 @@ __global__ __launch_bounds__(FNT) void k_conv_rows(ConvRows a) {
 // (28 of them k_fc_gemm, at 150 TFLOP/s); 784-256x6-10, 64 boxes, the whole
 // forward 1.76 -> 1.25 ms.
 //
-// Parts of the generators as rows: row = generator column j of domain b, its
-// values G[b][k][j] lam[b][k] over the neurons k.  Four waves take 64 columns,
-// each 16 of them: 256 bytes of a neuron's row at a time.
+// Parts of the generators as rows: row = generator column j < cols of domain b,
+// its values G[b][k][j] lam[b][k] over the neurons k, K of a neuron's values
+// apart.  Four waves take 64 columns, each 16 of them: 256 bytes of a neuron's
+// row at a time.
 __global__ __launch_bounds__(FNT) void k_zono_rows(const float* G, const float* lam, int n, int K,
-                                                   int mt16, int nkc, FastDiv f_blk,
+                                                   int cols, int mt16, int nkc, FastDiv f_blk,
                                                    uint4* parts) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
   const int64_t dom = f_blk.div((uint32_t)blockIdx.x);
   const int t = ((int)(blockIdx.x - dom * f_blk.d)) * 4 + wv;
   if (t >= mt16) return;
-  const float* x = G + dom * n * (int64_t)K + min(16 * t + r, K - 1);
+  const float* x = G + dom * n * (int64_t)K + min(16 * t + r, cols - 1);
   const float* l = lam ? lam + dom * n : nullptr;
   uint4* out = parts + (dom * mt16 + t) * nkc * kTileU + lane;
   for (int kc = blockIdx.y; kc < nkc; kc += gridDim.y) {
@@ -774,35 +775,44 @@ extern "C" int vc_zono_fc_split(const float* G, const float* lam, int64_t B, int
   if (B == 0 || K == 0) return VC_OK;
   if (!G || !packed_t || !G_out || !work || !aligned16(packed_t) || !aligned16(work))
     return VC_ERR_ARG;
-  const int64_t per = vc_fc_split_pack_bytes(n, K);
   const hipStream_t st = (hipStream_t)stream;
   GemmArgs b{};
   b.nkc = 2 * ((n + 2 * FBK - 1) / (2 * FBK));
   b.Ap = (const uint4*)work;
   b.Bp = (const uint4*)packed_t;
-  b.M = K;
   b.N = n_out;
   b.ld = ld;
-  b.mt16 = (K + 15) / 16;
   b.ntn = (n_out + FBN - 1) / FBN;
   b.f_ntn = FastDiv::make((uint32_t)b.ntn);
-  const int blk = (b.mt16 + 3) / 4, ny = b.nkc < 4 ? b.nkc : 4;
-  b.f_dom = FastDiv::make((uint32_t)blk);
-  // domains whose parts the buffer holds, and whose tiles a launch counts
-  int64_t step = work_bytes / per;
-  const int64_t most = (((int64_t)1 << 31) - 1) / ((int64_t)blk * b.ntn);
-  if (step > most) step = most;
-  if (step < 1) return VC_ERR_ARG;
-  for (int64_t b0 = 0; b0 < B; b0 += step) {
-    const int64_t cnt = B - b0 < step ? B - b0 : step;
-    hipLaunchKernelGGL(k_zono_rows, dim3((unsigned)(cnt * blk), ny), dim3(FNT), 0, st,
-                       G + b0 * n * K, lam ? lam + b0 * n : nullptr, n, K, b.mt16, b.nkc, b.f_dom,
-                       (uint4*)work);
-    VC_LAUNCH_CHECK();
-    b.out = G_out + b0 * n_out * ld;
-    b.tiles = cnt * blk * b.ntn;
-    hipLaunchKernelGGL((k_fc_gemm<4, kDomains>), dim3((unsigned)b.tiles), dim3(FNT), 0, st, b);
-    VC_LAUNCH_CHECK();
+  const int ny = b.nkc < 4 ? b.nkc : 4;
+  // domains whose parts the buffer holds, or columns of one
+  int64_t step = work_bytes / vc_fc_split_pack_bytes(n, K), cols = K;
+  if (step < 1) {
+    step = 1;
+    cols = work_bytes / vc_fc_split_pack_bytes(n, 16) / 4 * 64;
+    if (cols < 64) return VC_ERR_ARG;
+  }
+  for (int64_t j0 = 0; j0 < K; j0 += cols) {
+    const int kc = (int)(K - j0 < cols ? K - j0 : cols);
+    b.M = kc;
+    b.mt16 = (kc + 15) / 16;
+    const int blk = (b.mt16 + 3) / 4;
+    b.f_dom = FastDiv::make((uint32_t)blk);
+    // domains whose tiles a launch counts
+    const int64_t most = (((int64_t)1 << 31) - 1) / ((int64_t)blk * b.ntn);
+    if (most < 1) return VC_ERR_ARG;
+    if (step > most) step = most;
+    for (int64_t b0 = 0; b0 < B; b0 += step) {
+      const int64_t cnt = B - b0 < step ? B - b0 : step;
+      hipLaunchKernelGGL(k_zono_rows, dim3((unsigned)(cnt * blk), ny), dim3(FNT), 0, st,
+                         G + b0 * n * K + j0, lam ? lam + b0 * n : nullptr, n, K, kc, b.mt16,
+                         b.nkc, b.f_dom, (uint4*)work);
+      VC_LAUNCH_CHECK();
+      b.out = G_out + b0 * n_out * ld + j0;
+      b.tiles = cnt * blk * b.ntn;
+      hipLaunchKernelGGL((k_fc_gemm<4, kDomains>), dim3((unsigned)b.tiles), dim3(FNT), 0, st, b);
+      VC_LAUNCH_CHECK();
+    }
   }
   return VC_OK;
 }

@@ -263,9 +263,32 @@ def _fc_split_parts(packs, p, M, st, trans=False, sweep=False):
     return packs.fc(p, st, trans) if ok and M < 1 << 31 else None
 
 
-def _fc_split_work(M, K, dev):
-    """The buffer of M rows' parts that a vc_fc_split product forms first."""
-    return torch.empty(_lib.load().vc_fc_split_pack_bytes(K, M), dtype=torch.uint8, device=dev)
+def _cut(t, rows):
+    return t if t is None or rows is None else t[rows]
+
+
+def _in_slices(B, R, K, dev, launch):
+    """``launch`` a vc_fc_split product of B * R rows of K values, in slices whose
+    parts take up to _FC_WORK_BYTES: whole domains, or rows of one domain.  It
+    gets the slice (for _cut) of a (B, ..), a (B * R, ..) and a shared (R, ..)
+    tensor, its number of rows and of rows a domain, and the buffer of parts."""
+    size = _lib.load().vc_fc_split_pack_bytes
+    most = max(64, _FC_WORK_BYTES // (size(K, 16) // 16))
+    if B * R <= most:
+        launch(None, None, None, B * R, R,
+               torch.empty(size(K, B * R), dtype=torch.uint8, device=dev))
+        return
+    if R <= most:
+        step = -(-B // -(-B // (most // R)))  # the slices alike
+        spans = [(b, min(B, b + step), 0, R) for b in range(0, B, step)]
+    else:
+        step = -(-R // -(-R // most))
+        spans = [(b, b + 1, r, min(R, r + step)) for b in range(B) for r in range(0, R, step)]
+    rows = max((b1 - b0) * (r1 - r0) for b0, b1, r0, r1 in spans)
+    work = torch.empty(size(K, rows), dtype=torch.uint8, device=dev)
+    for b0, b1, r0, r1 in spans:
+        launch(slice(b0, b1), slice(b0 * R + r0, (b1 - 1) * R + r1), slice(r0, r1),
+               (b1 - b0) * (r1 - r0), r1 - r0, work)
 
 
 def _pair(v):
@@ -434,12 +457,11 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
             lo_o = torch.empty(B, p['n_out'], device=dev)
             hi_o = torch.empty_like(lo_o)
             K = C_in * kh * kw
+            per = 2 * _lib.load().vc_fc_split_pack_bytes(K, Ho * Wo)
             if (name not in raw and K >= 512 and C_out > 32
                     and B * p['n_out'] * K >= _IBP_SPLIT_MACS
-                    and Ho * Wo < 1 << 24 and K < 1 << 24 and H * W < 1 << 28
-                    and p['n_in'] < 1 << 31):
+                    and per <= _IBP_BOX_BYTES and H * W < 1 << 28 and p['n_in'] < 1 << 31):
                 parts = packs.conv_interval(p, K, st)
-                per = 2 * _lib.load().vc_fc_split_pack_bytes(K, Ho * Wo)
                 work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)),
                                    dtype=torch.uint8, device=dev)
                 call('vc_ibp_conv_split', ptr(l), ptr(h), B, C_in, H, W, ptr(parts[0]),
@@ -541,9 +563,10 @@ def _zono_fc(packs, p, g, B, K, st):
     out = torch.empty(B, n_out, K + k, device=dev)
     if K:
         parts = packs.fc(p, st, True)
-        per = _lib.load().vc_fc_split_pack_bytes(n, K)
-        work = torch.empty(per * max(1, min(B, _ZONO_WORK_BYTES // per)), dtype=torch.uint8,
-                           device=dev)
+        size = _lib.load().vc_fc_split_pack_bytes
+        per = size(n, K)
+        work = torch.empty(per * min(B, _ZONO_WORK_BYTES // per) if per <= _ZONO_WORK_BYTES
+                           else max(size(n, 64), _ZONO_WORK_BYTES), dtype=torch.uint8, device=dev)
         call('vc_zono_fc_split', ptr(g.G), ptr(g.lam), B, n, K, ptr(parts), n_out, K + k,
              ptr(out), ptr(work), work.numel(), st)
     call('vc_zono_fc_cols', ptr(p['W']), n_out, n, B, k, ptr(idx), idx_ld, ptr(mu), ptr(xl),
@@ -762,13 +785,16 @@ _ZONO_SPLIT_MACS = 1.5e9
 # 803 and 935, 8->16 5x5 459 and 541).
 _IBP_SPLIT_MACS = 1e8
 _ZONO_WORK_BYTES = 192 << 20
+_IBP_BOX_BYTES = 1 << 30  # parts of one box: beyond, the gathering product, which takes none
 
 
 class BackwardTrace:
     """Per-relu stored pre-relaxation rows of one backward, for the alpha
     gradient sweep: entries (L, P, p_shared) in backward order.  ``other``
     names an op the sweep does not replay (add, sub, mul, a fan-in); ``slopes``
-    holds the layers' slopes where the backward had to form them."""
+    holds the layers' slopes where the backward had to form them and they are
+    small (_SLOPES_KEPT_BYTES; for one row a domain they are three times the
+    rows): beyond, the sweep forms them again."""
 
     def __init__(self):
         self.relus = []
@@ -789,6 +815,10 @@ _TWO_PHASE_MIN_WIDTH = 64
 # backward's loss on few rows.  Narrow ones do not pay for the pass that forms
 # the parts: 64 x 64 at 73,728 rows 35 -> 46, the gradient's 25 -> 41 (128 x 16:
 # 34 -> 56, 203 x 117: 135 -> 131).
+_SLOPES_KEPT_BYTES = 32 << 20  # a layer's; forming them takes 10 us at that size
+# Parts of rows take so much at a time, whatever the number of rows.  Slices that the last-level cache holds (192 MiB) are no
+# faster (73,728 rows of 1024 x 1024 977 us whole, 991; of 1024 x 64 286 and 312).
+_FC_WORK_BYTES = 512 << 20
 _FC_SPLIT_ROWS = 2048
 _FC_SPLIT_SWEEP_ROWS = 64
 _FC_SPLIT_WIDTH = 128
@@ -948,7 +978,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         out = [torch.empty(B, n, device=dev) for _ in range(3)]
         call('vc_relax_slopes', ptr(lo), ptr(hi), ptr(rows.alpha), B * n, ptr(out[0]),
              ptr(out[1]), ptr(out[2]), st)
-        if trace is not None:
+        if trace is not None and 12 * B * n <= _SLOPES_KEPT_BYTES:
             trace.slopes[rows.relu] = out
         return out
 
@@ -1079,13 +1109,17 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                     parts = _fc_split_parts(packs, p, M, st, sweep=trace is not None)
                 if parts is not None:
                     ls, us, ut = slopes(rows)
-                    work = _fc_split_work(M, p['n_out'], dev)
                     if trace is not None:
                         trace.fcs.append(op)
-                    call('vc_backward_fc_split', ptr(rows.ew), M, R, 1 if rows.shared else 0,
-                         p['n_out'], ptr(ls), ptr(us), ptr(ut), ptr(rows.beta),
-                         ptr(parts), ptr(p['b']), p['n_in'], ptr(out), ptr(acc),
-                         ptr(work), st)
+
+                    def launch(d, m, r, M, R, work):
+                        call('vc_backward_fc_split',
+                             ptr(_cut(rows.ew, r if rows.shared else m)), M, R,
+                             1 if rows.shared else 0, p['n_out'], ptr(_cut(ls, d)),
+                             ptr(_cut(us, d)), ptr(_cut(ut, d)), ptr(_cut(rows.beta, d)),
+                             ptr(parts), ptr(p['b']), p['n_in'], ptr(_cut(out, m)),
+                             ptr(_cut(acc, m)), ptr(work), st)
+                    _in_slices(B, R, p['n_out'], dev, launch)
                     put(inp, _Rows(out, False))
                     continue
                 lo, hi = f32(tight[L][0]), f32(tight[L][1])
@@ -1432,9 +1466,9 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
     g = torch.empty(M, f0['n_out'], device=dev)
     parts = _fc_split_parts(packs, f0, M, st, True)
     if parts is not None:
-        work = _fc_split_work(M, n_in, dev)
-        call('vc_alpha_grad_input_split', ptr(A), ptr(xl), ptr(xh), M, Q, n_in, ptr(parts),
-             ptr(f0['b']), f0['n_out'], ptr(g), ptr(work), st)
+        _in_slices(B, Q, n_in, dev, lambda d, m, r, M, Q, work: call(
+            'vc_alpha_grad_input_split', ptr(_cut(A, m)), ptr(_cut(xl, d)), ptr(_cut(xh, d)), M,
+            Q, n_in, ptr(parts), ptr(f0['b']), f0['n_out'], ptr(_cut(g, m)), ptr(work), st))
     else:
         call('vc_alpha_grad_input', ptr(A), ptr(xl), ptr(xh), M, Q, n_in,
              ptr(f0['W']), ptr(f0['b']), f0['n_out'], ptr(g), st)
@@ -1477,10 +1511,11 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
                      ptr(us), ptr(ut), st)
             parts = _fc_split_parts(packs, fn, M, st, True)
             if parts is not None:
-                work = _fc_split_work(M, n, dev)
-                call('vc_alpha_grad_step_split', ptr(g), ptr(P), M, Q, n, ptr(ls), ptr(us),
-                     ptr(ut), 1 if p_shared else 0, ptr(parts), ptr(fn['b']), fn['n_out'],
-                     ptr(g2), ptr(work), st)
+                _in_slices(B, Q, n, dev, lambda d, m, r, M, Q, work: call(
+                    'vc_alpha_grad_step_split', ptr(_cut(g, m)),
+                    ptr(_cut(P, r if p_shared else m)), M, Q, n, ptr(_cut(ls, d)),
+                    ptr(_cut(us, d)), ptr(_cut(ut, d)), 1 if p_shared else 0, ptr(parts),
+                    ptr(fn['b']), fn['n_out'], ptr(_cut(g2, m)), ptr(work), st))
             else:
                 call('vc_alpha_grad_step_slopes', ptr(g), ptr(P), M, Q, n,
                      ptr(ls), ptr(us), ptr(ut), 1 if p_shared else 0,
