@@ -111,13 +111,14 @@ def _mlp(widths):
 
 
 @pytest.mark.parametrize('B,Q', [(300000, 9), (3, 700000), (1 << 20, 1)])
-def test_alpha_gradient_scratch(scratch, B, Q):
+def test_alpha_gradient_scratch(scratch, monkeypatch, B, Q):
     """Rows whose relaxed form takes 10 GB and more: the parts 512 MiB at a time,
     every row once, and no slopes held past 32 MiB a layer."""
     gg = _mlp([784, 1000, 1000, 10])
     x = torch.empty(B, 784, device=META)
     sb = {L: (torch.empty(B, 1000, device=META),) * 2 for L in (0, 1)}
     alpha = {L: torch.empty(B, 1000, device=META) for L in (0, 1)}
+    monkeypatch.setattr(vz, '_fc_split_pays', lambda *a: True)
     traces = []
     init = vz.BackwardTrace.__init__
     vz.BackwardTrace.__init__ = lambda self: (init(self), traces.append(self))[0]
@@ -142,3 +143,20 @@ def test_interval_conv_scratch(scratch, monkeypatch):
         del scratch[:]
         vz._ibp_forward_graph_batched(x, x, gg, META, torch.float32)
         assert len(scratch) == n and all(b <= 1 << 30 for _, b, _ in scratch)
+
+
+# rows, values, columns; packed for one pass; a gradient sweep follows: whether
+# the parts were measured the faster, weights packed and slopes formed included
+@pytest.mark.parametrize('M,K,N,once,sweep,pays', [
+    (2304, 64, 128, True, False, False), (4608, 64, 784, False, True, True),
+    (4608, 64, 784, True, False, False), (73728, 64, 128, False, False, False),
+    (2304, 256, 256, True, False, False), (4608, 256, 256, True, False, False),
+    (18432, 256, 256, True, False, True), (73728, 256, 256, False, True, True),
+    (288, 256, 256, False, True, True), (288, 256, 256, False, False, False),
+    (288, 1024, 1024, False, True, False), (576, 784, 128, False, True, False),
+    (4608, 1024, 1024, False, True, True), (4608, 1024, 1024, True, False, True),
+    (18432, 1024, 64, False, True, True), (73728, 1024, 64, False, True, False),
+    (73728, 784, 10, False, False, False), (73728, 300, 5, False, True, True),
+    (73728, 65, 128, False, True, True), (73728, 65, 100, False, True, False)])
+def test_fc_split_rule(M, K, N, once, sweep, pays):
+    assert vz._fc_split_pays(M, K, N, once, sweep) == pays

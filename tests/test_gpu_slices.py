@@ -29,6 +29,7 @@ def _net(gpu, widths):
                                       (600, 1, 200000)])
 @pytest.mark.parametrize('beta', [False, True])
 def test_alpha_gradient_in_slices(gpu, monkeypatch, B, Q, work, beta):
+    monkeypatch.setattr(vz, '_fc_split_pays', lambda *a: True)
     gg = _net(gpu, [130, 150, 190, 140, 7])
     g = torch.Generator(device=gpu).manual_seed(Q)
 

@@ -50,7 +50,7 @@ def _case(path, dtype=F32, dev='cpu'):
     cnn = path in ('ibp', 'crown_cnn', 'spec_cnn')
     gg = _cnn(dtype, dev) if cnn else _mlp(MLP, dtype, dev)
     n_in, n_out = gg['input_n'], 9
-    B = 256 if path == 'spec' else 4 if path == 'crown_cnn' else 16
+    B = 4 if path == 'crown_cnn' else 16
     g = torch.Generator().manual_seed(3)
     xl = torch.rand(B, n_in, generator=g).to(dev)
     xh = xl + 0.1
@@ -92,6 +92,7 @@ def small(monkeypatch):
     """Every product from the smallest sizes on by the packed weights."""
     monkeypatch.setattr(vz, '_ZONO_SPLIT_MACS', 0)
     monkeypatch.setattr(vz, '_IBP_SPLIT_MACS', 0)
+    monkeypatch.setattr(vz, '_fc_split_pays', lambda *a: True)
 
 
 @pytest.fixture

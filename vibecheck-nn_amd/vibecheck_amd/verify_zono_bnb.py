@@ -249,17 +249,29 @@ class _Packs:
         return out
 
 
-def _fc_split_parts(packs, p, M, st, trans=False, sweep=False):
+def _fc_split_pays(M, K, N, once, sweep):
+    """Whether M rows of K values times (K, N) are the faster as parts: ``once``,
+    packed for one pass; ``sweep``, a gradient sweep follows that uses the
+    backward's slopes (the figures stand at _FC_SPLIT_WIDTH)."""
+    if K < _TWO_PHASE_MIN_WIDTH or max(K, N) < _FC_SPLIT_WIDTH:
+        return False
+    # the parts of wide rows for few columns, written and read again, have to
+    # stay in the last-level cache
+    if K > _TWO_PHASE_MIN_WIDTH and (4 * N >= K or 6 * M * K <= 288 << 20):
+        if M >= 8192 or (M >= 4096 if once else M >= 2048) and M * K * N >= (1e9 if once else 4e8):
+            return True
+    return sweep and _FC_SPLIT_SWEEP_ROWS <= M < 8192 and K <= 512
+
+
+def _fc_split_parts(packs, p, M, st, trans=False, once=False, sweep=False):
     """The fc weights' bf16 parts for M rows' vc_backward_fc_split (``trans``:
     for the gradient's products with W^T); None where the fp32 product is the
-    faster one.  ``sweep``: a gradient sweep follows that uses the backward's
-    slopes."""
+    faster one."""
     K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
     if trans:
         ok = M >= _FC_SPLIT_SWEEP_ROWS and min(K, N) >= _FC_SPLIT_WIDTH
     else:
-        ok = (M >= (_FC_SPLIT_SWEEP_ROWS if sweep else _FC_SPLIT_ROWS)
-              and K >= _TWO_PHASE_MIN_WIDTH and max(K, N) >= _FC_SPLIT_WIDTH)
+        ok = _fc_split_pays(M, K, N, once, sweep)
     return packs.fc(p, st, trans) if ok and M < 1 << 31 else None
 
 
@@ -778,11 +790,17 @@ class _Window:
 # layer, 327 and 341 us; of 64 boxes, 3.3e9, 605 and 531).  Parts take so many
 # bytes at a time, which the last-level cache holds.
 _ZONO_SPLIT_MACS = 1.5e9
-# The interval forward of a conv likewise; the pass that forms its parts writes
-# 12 bytes per pixel and tap whatever the channels out, so few of them or few
-# taps stay with the gathering product (whole forwards, it and the parts: 32->64
-# 4x4, 16 boxes 0.13e9 119 and 108 us, 512 boxes 957 and 697; 32->32 3x3 of 512
-# 803 and 935, 8->16 5x5 459 and 541).
+# The interval forward of a conv likewise: the pass that forms its parts writes
+# 12 bytes per pixel and tap whatever the channels out.  The gathering product
+# and the parts, weights packed included, us (values K of a pixel -> channels):
+#   512 -> 33    0.07e9 multiplications 55 and 34, 4.7e9 1,290 and 774
+#   512 -> 128   0.08e9 52 and 37, 1.2e9 216 and 76;  576 -> 64  0.15e9 44 and 34
+#   1600 -> 33   0.05e9 111 and 61, 14e9 3,072 and 2,585
+# and from 512 values and 33 channels on they win everywhere but 1600 -> 64 at
+# 1.7e9 (151 and 154).  Onto 16 channels they lose from
+# 0.3e9 up (576: 1.9 times at 0.6e9, 1024: 1.5 at 5e9).  With fewer values they
+# win from 0.6e9 up only (288 -> 33 0.85, 128 -> 64 0.6 of the time; below, 1.2 to
+# 1.8 times): left with the gathering product.
 _IBP_SPLIT_MACS = 1e8
 _ZONO_WORK_BYTES = 192 << 20
 _IBP_BOX_BYTES = 1 << 30  # parts of one box: beyond, the gathering product, which takes none
@@ -808,20 +826,27 @@ class BackwardTrace:
 # layers than relaxing inside the GEMM's loads).
 _TWO_PHASE_MIN_WIDTH = 64
 
-# Products of bf16 parts, against the fp32 ones (us, slopes included): 256 x 256
-# at 1,152 rows 16 and 16, at 18,432 90 -> 46; 1024 x 1024 at 288 rows 20 -> 32,
-# at 4,608 130 -> 94.  The gradient's, whose fp32 product sums in 64 bits: 256 x
-# 256 at 9 rows 16 -> 9, 1024 x 1024 at 288 rows 52 -> 25; its gain outweighs the
-# backward's loss on few rows.  Narrow ones do not pay for the pass that forms
-# the parts: 64 x 64 at 73,728 rows 35 -> 46, the gradient's 25 -> 41 (128 x 16:
-# 34 -> 56, 203 x 117: 135 -> 131).
-_SLOPES_KEPT_BYTES = 32 << 20  # a layer's; forming them takes 10 us at that size
-# Parts of rows take so much at a time, whatever the number of rows.  Slices that the last-level cache holds (192 MiB) are no
-# faster (73,728 rows of 1024 x 1024 977 us whole, 991; of 1024 x 64 286 and 312).
-_FC_WORK_BYTES = 512 << 20
-_FC_SPLIT_ROWS = 2048
+# Products of bf16 parts against the fp32 ones, both from the rows to the product,
+# us; the parts also take 6 for the slopes and, once a call, 5.5 to pack the
+# weights.  Backward, (values x columns) at rows:
+#   64 x 128      2,304: 14 and 10;  73,728: 30 and 34 (a single tile's width in fp32)
+#   65 x 128     18,432: 44 and 27;  73,728: 107 and 60
+#   128 x 128     4,608: 17 and 11;   9,216: 27 and 15;  73,728: 105 and 48
+#   256 x 256       288: 15 and 10;   4,608: 22 and 18;  13,824: 85 and 29
+#   512 x 512       576: 15 and 14;   2,304: 30 and 25;   4,608: 47 and 32
+#   784 x 128     4,608: 41 and 32;  36,864: 182 and 137; 73,728: 250 and 248
+#   1024 x 784    1,152: 32 and 34;   2,304: 48 and 42;   4,608: 79 and 67
+#   1024 x 1024     288: 20 and 26;   2,304: 75 and 48;  73,728: 1,202 and 991
+# The gradient's, whose fp32 product sums in 64 bits (slopes on both sides):
+#   128 x 128       288: 10 and 9;  256 x 256: 15 and 10;  1024 x 1024: 52 and 25;
+#   128 x 33     18,432: 18 and 18;  64 x 64: 10 and 14.
 _FC_SPLIT_SWEEP_ROWS = 64
 _FC_SPLIT_WIDTH = 128
+_SLOPES_KEPT_BYTES = 32 << 20  # a layer's; forming them takes 10 us at that size
+# Parts of rows take so much at a time, whatever the number of rows.  Slices
+# that the last-level cache holds (192 MiB) are no faster (73,728 rows of 1024 x
+# 1024 977 us whole, 991; of 1024 x 64 286 and 312).
+_FC_WORK_BYTES = 512 << 20
 
 
 def _expand_rows(t, B):
@@ -843,7 +868,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     it makes several of these calls.  Returns (lb (B, R), A, a_shared, acc (B*R,));
     A of window rows is None.
     """
-    packs = _Packs() if packs is None else packs
+    once = packs is None
+    packs = _Packs() if once else packs
     B, n_in = xl.shape
     dev = xl.device
     st = stream()
@@ -1106,7 +1132,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 parts = None
                 if (split and M >= _FC_SPLIT_SWEEP_ROWS and rows.alpha_group is None
                         and not rows.alpha_row):
-                    parts = _fc_split_parts(packs, p, M, st, sweep=trace is not None)
+                    parts = _fc_split_parts(packs, p, M, st, once=once,
+                                            sweep=trace is not None)
                 if parts is not None:
                     ls, us, ut = slopes(rows)
                     if trace is not None:
