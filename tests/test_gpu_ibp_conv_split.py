@@ -17,8 +17,16 @@ CASES = [
 ]
 
 
+# row blocks of 64 pixels, from 384 of them up: one and two column tiles a wave,
+# a last block of 36 pixels, a second slice of boxes with blocks of 32
+CASES_TALL = [
+    (100, 5, 17, 17, 33, 3, 3, 1, 1, 1, 1, 100),
+    (100, 5, 17, 17, 65, 3, 3, 1, 1, 1, 1, 90),
+]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(map(str, c)))
+@pytest.mark.parametrize('case', CASES + CASES_TALL, ids=lambda c: '-'.join(map(str, c)))
 def test_ibp_conv_split_against_fp64(gpu, case):
     B, C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, chunk = case
     Ho, Wo = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1

@@ -652,6 +652,15 @@ int launch_fc(RowArgs a, const void* packed, int N, const float* bias, float* ou
   return VC_OK;
 }
 
+template <int MODE>
+void launch_conv(const GemmArgs& b, int mt, int nj, hipStream_t st) {
+  const dim3 grid((unsigned)b.tiles);
+  if (mt == 4 && nj == 1) hipLaunchKernelGGL((k_fc_gemm<4, MODE, 1>), grid, dim3(FNT), 0, st, b);
+  if (mt == 4 && nj == 2) hipLaunchKernelGGL((k_fc_gemm<4, MODE, 2>), grid, dim3(FNT), 0, st, b);
+  if (mt == 2 && nj == 1) hipLaunchKernelGGL((k_fc_gemm<2, MODE, 1>), grid, dim3(FNT), 0, st, b);
+  if (mt == 2 && nj == 2) hipLaunchKernelGGL((k_fc_gemm<2, MODE, 2>), grid, dim3(FNT), 0, st, b);
+}
+
 bool bad_args(int64_t M, int R, int K, int N, const void* packed, const void* work) {
   return M < 0 || R <= 0 || K <= 0 || N <= 0 || M % R != 0 || !packed || !work ||
          !aligned16(packed) || !aligned16(work);
@@ -848,6 +857,7 @@ extern "C" int vc_ibp_conv_split(const float* l, const float* h, int64_t B, int 
   if (step < 1) return VC_ERR_ARG;
   // one column tile a wave where two would leave half of the waves without
   const int nj = C_out <= 64 ? 1 : 2;
+  const int64_t cus = vcm::cu_count();
   GemmArgs b{};
   b.nkc = a.nkc;
   b.N = C_out;
@@ -864,26 +874,26 @@ extern "C" int vc_ibp_conv_split(const float* l, const float* h, int64_t B, int 
     a.rad = a.mid + (int64_t)b.mt16 * a.nkc * kTileU;
     hipLaunchKernelGGL(k_conv_rows, dim3((unsigned)b.mt16), dim3(FNT), 0, st, a);
     VC_LAUNCH_CHECK();
-    b.tiles = (int64_t)((b.mt16 + 3) / 4) * b.ntn;
+    // 32 pixels a row block where 64 give fewer than three tiles for two CUs
+    // (two fit a CU).  Both kinds of tiles, us: 256 tiles of 64 (16,384 pixels)
+    // of 32 and 64 channels, 5x5, onto 33 170 and 149, onto 64 170 and 154, 3x3
+    // onto 64 58 and 56; 304 of 32, 5x5, onto 128 452 and 407; 448 of 64, 3x3,
+    // onto 128 1,150 and 1,209; a few boxes of any of these 77 and 62.
+    const auto blocks = [&](int mt) { return (int64_t)((b.mt16 + mt - 1) / mt) * b.ntn; };
+    const int mt = 2 * blocks(4) >= 3 * cus ? 4 : 2;
+    b.tiles = blocks(mt);
     if (b.tiles >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)b.tiles);
     b.out = lo + b0 * C_out * npx;
     b.out2 = hi + b0 * C_out * npx;
     b.Ap = a.mid;
     b.Bp = (const uint4*)packed_t;
     b.bias = bias;
-    if (nj == 1)
-      hipLaunchKernelGGL((k_fc_gemm<4, kCentres, 1>), grid, dim3(FNT), 0, st, b);
-    else
-      hipLaunchKernelGGL((k_fc_gemm<4, kCentres, 2>), grid, dim3(FNT), 0, st, b);
+    launch_conv<kCentres>(b, mt, nj, st);
     VC_LAUNCH_CHECK();
     b.Ap = a.rad;
     b.Bp = (const uint4*)packed_abs_t;
     b.bias = nullptr;
-    if (nj == 1)
-      hipLaunchKernelGGL((k_fc_gemm<4, kRadii, 1>), grid, dim3(FNT), 0, st, b);
-    else
-      hipLaunchKernelGGL((k_fc_gemm<4, kRadii, 2>), grid, dim3(FNT), 0, st, b);
+    launch_conv<kRadii>(b, mt, nj, st);
     VC_LAUNCH_CHECK();
   }
   return VC_OK;
