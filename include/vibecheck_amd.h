@@ -406,7 +406,8 @@ int vc_backward_conv_split(const float *ew_in, int64_t M, int64_t R, int ew_shar
  *   rows then "-" rows: rows (2k, C_in kh kw), origin (2k, 2), and acc (2k) =
  *   +- bias.
  * vc_patch_relax: vc_backward_relu of M = B * R window rows (ew_shared: R) by
- *   their images' slopes (B, C H W; null: copied), zero outside the image.
+ *   their images' slopes (B, C H W; null: copied), zero outside the image; a
+ *   beta, which every neuron of the image has, leaves no window.
  *   The conv backward of the relaxed windows is vc_backward_conv(_packed) of
  *   (wh, ww) to ((wh - 1) sh + kh, (ww - 1) sw + kw) without padding.
  * vc_patch_shift: that conv's windows' origin (ph, pw the conv's own padding).
@@ -418,8 +419,7 @@ int vc_patch_seed(const float *kernel, const float *bias, const int32_t *idx, in
 int vc_patch_shift(const int32_t *origin_in, int R, int sh, int sw, int ph, int pw,
                    int32_t *origin_out, vc_stream_t stream);
 int vc_patch_relax(const float *ew_in, int64_t M, int64_t R, int ew_shared, const float *lo_s,
-                   const float *up_s, const float *up_t, const float *beta,
-                   const int32_t *origin, int C, int H, int W, int wh, int ww, float *ew_out,
+                   const float *up_s, const float *up_t, const int32_t *origin, int C, int H, int W, int wh, int ww, float *ew_out,
                    float *acc, vc_stream_t stream);
 int vc_patch_concretize(const float *A, int a_shared, const int32_t *origin, const float *acc,
                         const float *xl, const float *xh, int64_t M, int64_t R, int C, int H,

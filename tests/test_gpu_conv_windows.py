@@ -69,3 +69,35 @@ def test_windows_through_residual_merge(gpu):
     ops[at + 2]['inputs'] = ['merge']
     gg64['fork_points'] = {'relu0'}
     assert _check(gg64, copy.deepcopy(gg64), 4, 2 * 15 * 14, gpu, 2048) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('what', ['beta', 'alpha', 'plain'])
+def test_windows_as_whole_images(gpu, what):
+    """Window rows meet a relu with a beta, whose values outside the window
+    count, or an alpha: as the same rows seeded as whole images."""
+    gg = wk.cnn_gg([(9, 3, 1, 1), (13, 3, 1, 1)], [4], (3, 11, 12), seed=2, device=gpu)
+    B, k = 3, 20
+    xl, xh = (t.to(gpu) for t in wk.linf_boxes(B, 3 * 11 * 12, 0.03, seed=5))
+    sb = vz._ibp_forward_graph_batched(xl, xh, gg, gpu, torch.float32)
+    p = vz._op_params(gg['ops'][2], gpu)
+    C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+    g = torch.Generator().manual_seed(1)
+    idx = torch.randperm(p['n_out'], generator=g)[:k].to(gpu, torch.int32)
+    rows = vz._Rows(torch.empty(2 * k, C_in * kh * kw, device=gpu), True)
+    origin = torch.empty(2 * k, 2, dtype=torch.int32, device=gpu)
+    acc0 = torch.empty(2 * k, device=gpu)
+    vz.call('vc_patch_seed', vz.ptr(p['K']), vz.ptr(p['b']), vz.ptr(idx), k, C_out, Ho, Wo, C_in,
+            kh, kw, sh, sw, ph, pw, vz.ptr(rows.ew), vz.ptr(origin), vz.ptr(acc0), vz.stream())
+    rows.window = vz._Window(origin, kh, kw, C_in, H, W)
+    n = p['n_in']
+    beta = {0: 0.1 * torch.randn(B, n, generator=g).to(gpu)} if what == 'beta' else None
+    alpha = {0: torch.rand(B, n, generator=g).to(gpu)} if what == 'alpha' else None
+    got = vz._backward(sb, xl, xh, gg, 'relu0', rows, True, acc0, alpha, beta, split=False)[0]
+    seed = torch.zeros(2 * k, p['n_out'], device=gpu)
+    seed[torch.arange(k), idx.long()] = 1.0
+    seed[torch.arange(k) + k, idx.long()] = -1.0
+    want = vz._backward(sb, xl, xh, gg, 'conv1', seed, True, torch.zeros(2 * k, device=gpu),
+                        alpha, beta, split=False)[0]
+    # fp32 sums of the same values in another order
+    assert (got.double() - want.double()).norm() <= 2e-6 * want.double().norm()

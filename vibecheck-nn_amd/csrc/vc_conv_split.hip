@@ -595,8 +595,7 @@ __global__ void k_patch_shift(const int* in, int n, int sh, int sw, int ph, int 
 // row, lanes along it: each row is read and written once, coalesced.
 __global__ __launch_bounds__(CNT) void k_patch_relax(const float* x, int shared, const float* ls,
                                                      const float* us, const float* ut,
-                                                     const float* beta, const int* origin,
-                                                     int64_t M, int64_t R, int C, int H, int W,
+                                                     const int* origin, int64_t M, int64_t R, int C, int H, int W,
                                                      int wh, int ww, FastDiv f_ww, FastDiv f_wp,
                                                      float* out, float* acc) {
   const int wp = wh * ww, n = C * wp, lane = threadIdx.x & 63;
@@ -618,7 +617,6 @@ __global__ __launch_bounds__(CNT) void k_patch_relax(const float* x, int shared,
           const float en = e > 0.f ? 0.f : e, ep = e < 0.f ? 0.f : e;
           s += (double)(en * ut[o]);
           e = ep * ls[o] + en * us[o];
-          if (beta) e = e + beta[o];
         }
       }
       out[m * n + i] = e;
@@ -783,19 +781,18 @@ extern "C" int vc_patch_shift(const int32_t* origin_in, int R, int sh, int sw, i
 
 extern "C" int vc_patch_relax(const float* ew_in, int64_t M, int64_t R, int ew_shared,
                               const float* lo_s, const float* up_s, const float* up_t,
-                              const float* beta, const int32_t* origin, int C, int H, int W,
+                              const int32_t* origin, int C, int H, int W,
                               int wh, int ww, float* ew_out, float* acc, vc_stream_t stream) {
   if (!ew_in || !origin || !ew_out || M < 0 || R <= 0 || M % R || C <= 0 || H <= 0 || W <= 0 ||
       wh <= 0 || ww <= 0)
     return VC_ERR_ARG;
   if ((lo_s == nullptr) != (up_s == nullptr) || (lo_s == nullptr) != (up_t == nullptr) ||
-      (beta && !lo_s) || (lo_s && !acc))
+      (lo_s && !acc))
     return VC_ERR_ARG;
   if ((int64_t)C * wh * ww > (1 << 30) || (int64_t)C * H * W > (1 << 30)) return VC_ERR_UNSUPPORTED;
   if (M == 0) return VC_OK;
   hipLaunchKernelGGL(k_patch_relax, dim3(vc_blocks(64 * M, CNT)), dim3(CNT), 0,
-                     (hipStream_t)stream, ew_in, ew_shared ? 1 : 0, lo_s, up_s, up_t, beta, origin,
-                     M, R, C, H, W, wh, ww, FastDiv::make((uint32_t)ww),
+                     (hipStream_t)stream, ew_in, ew_shared ? 1 : 0, lo_s, up_s, up_t, origin, M, R, C, H, W, wh, ww, FastDiv::make((uint32_t)ww),
                      FastDiv::make((uint32_t)(wh * ww)), ew_out, acc);
   VC_LAUNCH_CHECK();
   return VC_OK;

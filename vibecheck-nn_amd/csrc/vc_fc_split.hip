@@ -44,11 +44,6 @@ constexpr int kTileU = 3 * 64;  // 16-byte units of 16 rows x 32 values, three p
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ v4f mfma_bf16(u4 a, u4 b, v4f acc) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a),
-                                                 __builtin_bit_cast(v8bf, b), acc, 0, 0, 0);
-}
-
 enum Form { kRelax, kGradStep, kGradInput };
 
 struct RowArgs {

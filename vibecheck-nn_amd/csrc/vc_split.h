@@ -46,7 +46,8 @@ __device__ __forceinline__ void split8(const float* x, uint4& h, uint4& m, uint4
 // One 16x16x32 step.  Operand layout for lane l, g = l / 16, r = l % 16:
 //   a[j] = A[row r][k 8 g + j], b[j] = B[k 8 g + j][col r],
 //   acc[i] = D[row 4 g + i][col r].
-__device__ __forceinline__ v4f mfma_bf16(const uint4& a, const uint4& b, v4f acc) {
+template <class Operand>  // sixteen bytes
+__device__ __forceinline__ v4f mfma_bf16(Operand a, Operand b, v4f acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a),
                                                  __builtin_bit_cast(v8bf, b), acc, 0, 0, 0);
 }
@@ -68,10 +69,6 @@ __device__ __forceinline__ Buf buffer(const float* p, int64_t bytes) {
 __device__ __forceinline__ float ldb(Buf b, uint32_t off, int soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, off, soff, 0));
 }
-__device__ __forceinline__ v4f ldb4(Buf b, uint32_t off) {
-  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
-}
-
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 
 }  // namespace vcs

@@ -79,7 +79,7 @@ SIGNATURES = {
                           _P, _P, _P, _L, _P],
     'vc_patch_seed': [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     'vc_patch_shift': [_P, _I, _I, _I, _I, _I, _P, _P],
-    'vc_patch_relax': [_P, _L, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P],
+    'vc_patch_relax': [_P, _L, _L, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P],
     'vc_patch_concretize': [_P, _I, _P, _P, _P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
     'vc_patch_dense': [_P, _P, _L, _L, _I, _I, _I, _I, _I, _P, _P],
     'vc_concretize': [_P, _P, _P, _P, _L, _I, _I, _I, _P, _P],

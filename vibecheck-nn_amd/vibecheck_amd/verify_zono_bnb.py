@@ -1011,27 +1011,26 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     def window_conv(rows, p):
         """Window rows through a conv: the pending relu relaxed at their
         places in the image, then the conv of the windows alone; None where
-        the window is no longer worth it or the alpha's form is another."""
+        the window is no longer worth it, or where the relu has an alpha or a
+        beta (which gives every neuron of the image a value)."""
         w = rows.window
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
         oh, ow = (w.wh - 1) * sh + kh, (w.ww - 1) * sw + kw
-        if (not w.worth() or rows.alpha_group is not None
-                or (rows.alpha is not None and rows.alpha_row)
+        if (not w.worth() or trace is not None or rows.alpha is not None
+                or rows.beta is not None
                 or (rows.shared and rows.relu is None and not acc_shared)
                 or B * R * C_in * oh * ow >= 1 << 31):
             return None
-        ls = us = ut = beta = None
+        ls = us = ut = None
         if rows.relu is not None:
             ls, us, ut = slopes(rows)
-            beta = rows.beta
             bias, acc_b = p['b'], acc
         else:
             bias, acc_b = bias_acc(rows, p)
         M = R if rows.shared and rows.relu is None else B * R
         rel = torch.empty(M, C_out * w.wh * w.ww, device=dev)
         call('vc_patch_relax', ptr(rows.ew), M, R, 1 if rows.shared else 0, ptr(ls), ptr(us),
-             ptr(ut), ptr(beta), ptr(w.origin), C_out, w.H, w.W, w.wh, w.ww, ptr(rel), ptr(acc),
-             st)
+             ptr(ut), ptr(w.origin), C_out, w.H, w.W, w.wh, w.ww, ptr(rel), ptr(acc), st)
         out = _Rows(torch.empty(M, C_in * oh * ow, device=dev), M == R and rows.shared
                     and rows.relu is None)
         conv_fp32(p, rel, M, (w.wh, w.ww, oh, ow), out.ew, bias, acc_b)
