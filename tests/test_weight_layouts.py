@@ -48,7 +48,7 @@ def _cnn(dtype=F32, dev='cpu'):
 def _case(path, dtype=F32, dev='cpu'):
     """(gg, call) of a path whose products take packed weights."""
     cnn = path in ('ibp', 'crown_cnn', 'spec_cnn')
-    gg = _cnn(dtype, dev) if cnn else _mlp(MLP, dtype, dev)
+    gg = _cnn(dtype, dev) if cnn else _mlp([5, 50, 50, 9] if path == 'narrow' else MLP, dtype, dev)
     n_in, n_out = gg['input_n'], 9
     B = 4 if path == 'crown_cnn' else 16
     g = torch.Generator().manual_seed(3)
@@ -69,6 +69,8 @@ def _case(path, dtype=F32, dev='cpu'):
         if path == 'alpha':
             return [vz._run_alpha_crown_inputsplit_batched(xl, xh, gg, spec, dev, F32, n_iters=3,
                                                            sb=sb)]
+        if path == 'narrow':
+            return [t for b in vz._zono_sb(gg, xl, xh, dev, F32).values() for t in b]
         if path == 'ibp':
             bounds = vz._ibp_forward_graph_batched(xl, xh, gg, dev, F32)
             return [t for b in bounds.values() for t in b]
@@ -153,6 +155,39 @@ def test_inference_mode_weights(launches, path):
     assert launches['read'] >= 2
 
 
+def test_copies_are_kept_when_ready(monkeypatch):
+    """Copies of weights (another type or device) and the narrow networks' plan
+    are kept on the graph only after the stream that makes them has been waited
+    for, and not under capture; the caller's own fp32 tensors as they are."""
+    from vibecheck_amd import mlp_fused
+    waits = []
+    ready = [False]
+
+    def settled(dev):
+        waits.append(('_vc_amd_params' in op, mlp_fused.PLAN_KEY in narrow))
+        return ready[0]
+    monkeypatch.setattr(vz._lib, 'settled', settled)
+    monkeypatch.setattr(mlp_fused, 'call', lambda *a: None)
+    monkeypatch.setattr(mlp_fused, 'ptr', lambda t: t.data_ptr())
+    monkeypatch.setattr(mlp_fused, 'stream', lambda: 0)
+    narrow = _mlp([5, 50, 50, 5])
+    op = _mlp(MLP)['ops'][0]
+    cpu = torch.device('cpu')
+    p = vz._op_params(op, cpu)
+    assert not waits and vz._op_params(op, cpu) is p
+    op = _mlp(MLP, torch.float64)['ops'][0]
+    for ready[0] in (False, True):
+        del waits[:]
+        p = vz._op_params(op, cpu)
+        assert len(waits) == 1 and not waits[0][0]
+        q = mlp_fused.plan_for(narrow, cpu)
+        assert len(waits) == 2 and not waits[1][1]
+        if not ready[0]:
+            assert '_vc_amd_params' not in op and mlp_fused.PLAN_KEY not in narrow
+            continue
+        assert vz._op_params(op, cpu) is p and mlp_fused.plan_for(narrow, cpu) is q
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('path', PATHS)
 def test_changed_weights_gpu(gpu, small, path):
@@ -173,12 +208,13 @@ def test_changed_weights_gpu(gpu, small, path):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('path', PATHS)
-def test_two_streams_gpu(gpu, small, path):
+@pytest.mark.parametrize('path,dtype', [(p, F32) for p in PATHS]
+                         + [('zono', torch.float64), ('narrow', F32)])
+def test_two_streams_gpu(gpu, small, path, dtype):
     """A first call that waits behind other work on its stream, and a second one
     on another stream before it has run."""
-    _, run = _case(path, dev=gpu)
-    _, ref = _case(path, dev=gpu)
+    _, run = _case(path, dtype, dev=gpu)
+    _, ref = _case(path, dtype, dev=gpu)
     want = ref()
     torch.cuda.synchronize()
     a, b = torch.cuda.Stream(), torch.cuda.Stream()

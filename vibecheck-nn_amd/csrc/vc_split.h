@@ -69,6 +69,7 @@ __device__ __forceinline__ Buf buffer(const float* p, int64_t bytes) {
 __device__ __forceinline__ float ldb(Buf b, uint32_t off, int soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, off, soff, 0));
 }
+
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 
 }  // namespace vcs

@@ -356,3 +356,15 @@ def f32(t):
 def stream():
     """The current HIP stream of the current device (raw handle)."""
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def settled(device):
+    """Whether what was just made on the current stream may be kept for later
+    calls, on whatever streams those are: the stream is waited for, once.  What
+    is made under graph capture belongs to the graph and is not kept."""
+    if torch.device(device).type != 'cuda':
+        return True
+    if torch.cuda.is_current_stream_capturing():
+        return False
+    torch.cuda.current_stream(device).synchronize()
+    return True

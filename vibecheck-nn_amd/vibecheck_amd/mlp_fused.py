@@ -97,7 +97,8 @@ def plan_for(gg, device):
         gg[PLAN_KEY] = 'no'
         return None
     plan = MlpPlan(gg, device)
-    gg[PLAN_KEY] = plan
+    if _lib.settled(device):
+        gg[PLAN_KEY] = plan
     return plan
 
 

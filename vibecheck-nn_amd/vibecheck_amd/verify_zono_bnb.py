@@ -85,7 +85,14 @@ def _op_params(op, device):
         p['geom'] = (C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo)
         p['n_in'] = C_in * H * W
         p['n_out'] = C_out * Ho * Wo
-    op[key] = p
+    # the caller's own fp32 tensors are as ready as the caller has them; copies
+    # are ready for every stream before they are kept
+    given = (op.get('W', op.get('kernel')), op.get('bias'))
+    made = [p.get('W', p.get('K')), p.get('b')]
+    own = all(t is None or torch.is_tensor(g) and g.data_ptr() == t.data_ptr()
+              for t, g in zip(made, given))
+    if own or _lib.settled(device):
+        op[key] = p
     return p
 
 
@@ -1112,10 +1119,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             p = _op_params(op, dev)
             rows = materialize(rows)
             if p['b'] is not None:
-                key = ('b_rep', P)
-                if key not in p:
-                    p[key] = p['b'].repeat(P).contiguous()
-                bias_dot(rows, p[key], 1.0)
+                bias_dot(rows, p['b'].repeat(P), 1.0)
             M = rows.ew.shape[0]
             out = torch.empty(M, P * p['n_in'], device=dev)
             call('vc_backward_fc', ptr(rows.ew), M * P, R * P, p['n_out'], None,
