@@ -63,6 +63,12 @@ def test_interval_conv_of_many_pixels(launches, monkeypatch, side, entry):
     assert launches.count(entry) == (2 if entry == 'vc_ibp_conv' else 1)
 
 
+def test_window_limits():
+    """Images of more than 2^30 values are carried whole."""
+    assert vz._Window(None, 3, 3, 4, 1 << 14, 1 << 14).worth()
+    assert not vz._Window(None, 3, 3, 5, 1 << 14, 1 << 14).worth()
+
+
 def test_split_conv_limits():
     """vc_backward_conv_split_fits follows the rows; the geometry alone is
     vc_backward_conv_split_ok's."""

@@ -787,8 +787,10 @@ class _Window:
 
     def worth(self):
         """Windows up to half of the image are carried as such: beyond, the
-        part outside the image and the wider steps cost what is saved."""
-        return 2 * self.wh * self.ww <= self.H * self.W
+        part outside the image and the wider steps cost what is saved.  Images
+        of more than 2^30 values are past the window kernels' offsets."""
+        return (2 * self.wh * self.ww <= self.H * self.W
+                and self.C * self.H * self.W <= 1 << 30)
 
 
 # A zonotope relu and fc are taken together from this many multiplications up:
@@ -1413,7 +1415,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
         if feed_op['type'] == 'conv':
             p = _op_params(feed_op, dev)
             C_in, H, W, _, kh, kw = p['geom'][:6]
-            if _Window(None, kh, kw, C_in, H, W).worth():
+            if p['n_out'] <= 1 << 30 and _Window(None, kh, kw, C_in, H, W).worth():
                 window, below = p, feed_op['inputs'][0]
         for c0 in range(0, m, ch):
             cidx = idx[c0:c0 + ch].contiguous()
