@@ -101,3 +101,49 @@ def test_windows_as_whole_images(gpu, what):
                         alpha, beta, split=False)[0]
     # fp32 sums of the same values in another order
     assert (got.double() - want.double()).norm() <= 2e-6 * want.double().norm()
+
+
+@pytest.mark.gpu
+def test_window_steps_infinities(gpu):
+    """vc_patch_relax and vc_patch_concretize on windows partly outside their
+    images, with infinities and NaN inside: the values of the plain formula;
+    what lies outside the image or the window enters nothing."""
+    B, R, C, H, W, wh, ww = 3, 5, 2, 9, 8, 4, 3
+    g = torch.Generator().manual_seed(0)
+    rows = torch.randn(B * R, C, wh, ww, generator=g)
+    rows[1, 0, 2, 1], rows[7, 1, 3, 2], rows[12, 0, 0, 0] = float('inf'), float('-inf'), float('nan')
+    origin = torch.tensor([[-2, -1], [7, 6], [0, 0], [3, 2], [5, 5]], dtype=torch.int32)
+    ls, us, ut = (torch.rand(B, C, H, W, generator=g) for _ in range(3))
+    us[0, 0, 4, 3] = float('inf')
+    ut[1, 1, 1, 1] = float('inf')
+    acc = torch.randn(B * R, generator=g)
+    xl = torch.randn(B, C, H, W, generator=g)
+    xh = xl + torch.rand(B, C, H, W, generator=g)
+    xh[2, 1, 6, 6] = float('inf')
+    want, wacc, wlb = torch.zeros(B * R, C, wh, ww, dtype=torch.float64), [], []
+    for m in range(B * R):
+        b, (oy, ox) = m // R, origin[m % R].tolist()
+        a, lb = acc[m].double(), acc[m].double()
+        for c in range(C):
+            for dy in range(wh):
+                for dx in range(ww):
+                    y, x = oy + dy, ox + dx
+                    if 0 <= y < H and 0 <= x < W:
+                        e = rows[m, c, dy, dx].double()
+                        en, ep = e.clamp(max=0), e.clamp(min=0)
+                        a = a + en * ut[b, c, y, x].double()
+                        want[m, c, dy, dx] = ep * ls[b, c, y, x].double() + en * us[b, c, y, x].double()
+                        lb = lb + e * (xh if e < 0 else xl)[b, c, y, x].double()
+        wacc.append(a)
+        wlb.append(lb)
+    d = [t.to(gpu) for t in (rows, origin, ls, us, ut, acc, xl, xh)]
+    out, a2, lb2 = torch.empty_like(d[0]), d[5].clone(), torch.empty_like(d[5])
+    p, st = vz.ptr, vz.stream()
+    vz.call('vc_patch_relax', p(d[0]), B * R, R, 0, p(d[2]), p(d[3]), p(d[4]), p(d[1]), C, H, W,
+            wh, ww, p(out), p(a2), st)
+    vz.call('vc_patch_concretize', p(d[0]), 0, p(d[1]), p(d[5]), p(d[6]), p(d[7]), B * R, R, C, H,
+            W, wh, ww, p(lb2), st)
+    # one or two roundings of fp32 terms
+    for got, ref in ((out, want), (a2, torch.stack(wacc)), (lb2, torch.stack(wlb))):
+        torch.testing.assert_close(got.cpu().double(), ref, rtol=1e-6, atol=1e-6, equal_nan=True)
+    assert out.isfinite().logical_not().sum() >= 3 and a2.isfinite().any() and lb2.isfinite().any()

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from vibecheck_amd import _lib
+from vibecheck_amd import verify_zono_bnb as vz
 from vibecheck_amd._lib import call, ptr, stream
 
 # B, R, shared, beta, K, N
@@ -114,3 +115,82 @@ def test_fc_split_infinities(gpu):
     ok = want.isfinite()
     rows = [r for r in range(45) if r not in (3, 17)]
     assert _rel(out[rows][ok[rows]], (e @ t['W'].double())[rows][ok[rows]]) < 2 * TOL
+
+
+def _mlp(gpu, widths):
+    g = torch.Generator(device=gpu).manual_seed(sum(widths))
+    ops, prev = [], 'X'
+    for i, (a, b) in enumerate(zip(widths, widths[1:])):
+        ops.append({'name': f'fc{i}', 'type': 'fc', 'inputs': [prev],
+                    'W': torch.randn(b, a, generator=g, device=gpu) * (2.0 / a) ** 0.5,
+                    'bias': torch.randn(b, generator=g, device=gpu) * 0.1})
+        prev = f'fc{i}'
+        if i + 2 < len(widths):
+            ops.append({'name': f'r{i}', 'type': 'relu', 'inputs': [prev], 'layer_idx': i})
+            prev = f'r{i}'
+    return {'ops': ops, 'input_name': 'X', 'input_n': widths[0], 'fork_points': set(),
+            'input_shape': (1, widths[0]), 'n_relu': len(widths) - 2}
+
+
+# boxes on both sides of the rule's lines: 8,192 rows; 1e9 and 4e8 products; 64
+# rows with a sweep
+@pytest.mark.gpu
+@pytest.mark.parametrize('widths,boxes', [([70, 128, 130, 5], (2047, 2048)),
+                                          ([70, 500, 510, 5], (1024, 1030)),
+                                          ([40, 150, 512, 5], (15, 16)),
+                                          ([784, 520, 260, 5], (505, 920))])
+def test_backward_with_and_without_parts(gpu, monkeypatch, widths, boxes):
+    """The whole backward and its alpha gradient, products as parts and not, each
+    against 64 bits: the parts are no further off."""
+    gg, Q, F32 = _mlp(gpu, widths), 4, torch.float32
+    for B in boxes:
+        g = torch.Generator(device=gpu).manual_seed(B)
+
+        def rand(*shape):
+            return torch.randn(*shape, generator=g, device=gpu)
+        xl = rand(B, widths[0])
+        xh = xl + 0.1
+        sb, alpha, ga = {}, {}, {}
+        for L, n in enumerate(widths[1:-1]):
+            lo = rand(B, n) - 0.5
+            sb[L] = (lo, lo + 2)
+            alpha[L] = torch.rand(B, n, generator=g, device=gpu)
+            ga[L] = torch.empty(B, n, device=gpu)
+        Wq, bq = rand(Q, widths[-1]), rand(Q)
+        a64 = {L: a.double().requires_grad_() for L, a in alpha.items()}
+        e = Wq.double().unsqueeze(0).expand(B, Q, -1)
+        acc = bq.double().expand(B, Q)
+        for op in reversed(gg['ops']):
+            if op['type'] == 'fc':
+                acc = acc + e @ op['bias'].double()
+                e = e @ op['W'].double()
+                continue
+            lo, hi = (t.double() for t in sb[op['layer_idx']])
+            act, dead = lo >= 0, hi <= 0
+            un = ~act & ~dead
+            us = torch.where(un, hi / (hi - lo), act.double())
+            ut = torch.where(un, -lo * us, torch.zeros_like(lo))
+            ls = act + un * a64[op['layer_idx']]
+            en = e.clamp(max=0)
+            acc = acc + (en * ut.unsqueeze(1)).sum(2)
+            e = e.clamp(min=0) * ls.unsqueeze(1) + en * us.unsqueeze(1)
+        lb64 = acc + (e.clamp(min=0) * xl.double().unsqueeze(1)
+                      + e.clamp(max=0) * xh.double().unsqueeze(1)).sum(2)
+        g64 = dict(zip(a64, torch.autograd.grad(lb64.sum(), list(a64.values()))))
+        err = {}
+        rule = _fc_rule
+        for how, pays in (('rule', rule), ('parts', lambda *a: True), ('fp32', lambda *a: False)):
+            monkeypatch.setattr(vz, '_fc_split_pays', pays)
+            monkeypatch.setattr(vz, '_FC_SPLIT_SWEEP_ROWS', 64 if how == 'rule' else
+                                1 if how == 'parts' else 1 << 30)
+            lb, A = vz._alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, True, ga,
+                                                want_A=True)
+            err[how] = [_rel(lb, lb64.detach()), _rel(A.view(B, Q, -1), e.detach())] + \
+                [_rel(ga[L], g64[L]) for L in ga]
+        for k in ('rule', 'parts'):
+            # three layers of fp32 sums; no further off than the fp32 products but
+            # for what their last roundings differ by
+            assert all(x <= max(1e-6, 1.5 * y) for x, y in zip(err[k], err['fp32'])), (k, err)
+
+
+_fc_rule = vz._fc_split_pays

@@ -52,3 +52,50 @@ def test_ibp_conv_split_against_fp64(gpu, case):
     for got, want in ((lo, c - r), (hi, c + r)):
         # the centres' and radii's own rounding and the sums': 2^-24 each of |c| + |r|
         assert float((got.double() - want).norm() / (c.abs() + r).norm()) < 2e-7
+
+
+@pytest.mark.gpu
+def test_ibp_conv_split_infinities(gpu):
+    """Bounds that are infinite, NaN or round to infinity in bf16: what the
+    gathering product gives, in the pixels that read them only."""
+    B, C_in, H, W, C_out, k = 3, 9, 8, 7, 20, 3
+    g = torch.Generator(device=gpu).manual_seed(2)
+    K = torch.randn(C_out, C_in, k, k, generator=g, device=gpu)
+    b = torch.randn(C_out, generator=g, device=gpu)
+    l = torch.randn(B, C_in, H, W, generator=g, device=gpu)
+    h = l + torch.rand(B, C_in, H, W, generator=g, device=gpu)
+    h[0, 2, 0, 0] = float('inf')
+    l[0, 5, 7, 6] = float('-inf')
+    l[1, 0, 3, 3] = h[1, 0, 3, 3] = float('nan')
+    l[2, 8, 1, 1], h[2, 8, 1, 1] = 3.39e38, 3.395e38  # the sum of both is infinite
+    n = C_in * k * k
+    size = _lib.load().vc_fc_split_pack_bytes
+    parts = [torch.empty(size(n, C_out), dtype=torch.uint8, device=gpu) for _ in range(2)]
+    call('vc_fc_split_pack_abs', ptr(K), n, C_out, 1, ptr(parts[0]), ptr(parts[1]), stream())
+    work = torch.empty(2 * B * size(n, H * W), dtype=torch.uint8, device=gpu)
+    got, want = ([torch.empty(B, C_out, H, W, device=gpu) for _ in range(2)] for _ in range(2))
+    geom = (C_out, k, k, 1, 1, 1, 1, H, W)
+    call('vc_ibp_conv_split', ptr(l), ptr(h), B, C_in, H, W, ptr(parts[0]), ptr(parts[1]), ptr(b),
+         *geom, ptr(got[0]), ptr(got[1]), ptr(work), work.numel(), stream())
+    call('vc_ibp_conv', ptr(l), ptr(h), B, C_in, H, W, ptr(K), ptr(b), *geom, ptr(want[0]),
+         ptr(want[1]), stream())
+    for x, y in zip(got, want):
+        assert torch.equal(x.isnan(), y.isnan())
+        assert torch.equal(x[y.isinf()], y[y.isinf()])
+        ok = y.isfinite()
+        assert 0 < int(ok.sum()) < y.numel()
+        # both within 2e-7 of the sums' terms
+        assert float((x - y)[ok].norm() / y[ok].norm()) < 4e-7
+
+
+@pytest.mark.gpu
+def test_pack_abs_is_two_packs(gpu):
+    g = torch.Generator(device=gpu).manual_seed(3)
+    W = torch.randn(37, 75, generator=g, device=gpu)
+    out = [torch.empty(_lib.load().vc_fc_split_pack_bytes(75, 37), dtype=torch.uint8, device=gpu)
+           for _ in range(4)]
+    call('vc_fc_split_pack_abs', ptr(W), 75, 37, 1, ptr(out[0]), ptr(out[1]), stream())
+    Wa = W.abs()
+    for w, o in ((W, out[2]), (Wa, out[3])):
+        call('vc_fc_split_pack', ptr(w), 75, 37, 1, ptr(o), stream())
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])

@@ -30,3 +30,26 @@ def test_ibp_fc_slices(gpu, B, n_in, n_out):
             # straddle, one value in 1e6, is one step of its terms' size
             assert int((x != y).sum()) <= 1 + B * n_out // 100000
             assert float((x - y).abs().max()) <= 2 ** -22 * float(y.abs().max())
+
+
+@pytest.mark.gpu
+def test_ibp_fc_slices_infinities(gpu):
+    """Infinities and NaN in a slice reach the outputs of their own rows, as in
+    one sum."""
+    B, n_in, n_out = 6, 700, 12
+    g = torch.Generator(device=gpu).manual_seed(1)
+    W = torch.randn(n_out, n_in, generator=g, device=gpu)
+    l = torch.randn(B, n_in, generator=g, device=gpu)
+    h = l + torch.rand(B, n_in, generator=g, device=gpu)
+    h[0, 3], l[1, 699], l[2, 350], h[3, 223] = (float(v) for v in ('inf', '-inf', 'nan', '3.4e38'))
+    want, got = ([torch.empty(B, n_out, device=gpu) for _ in range(2)] for _ in range(2))
+    call('vc_ibp_fc', ptr(l), ptr(h), B, n_in, ptr(W), None, n_out, ptr(want[0]), ptr(want[1]),
+         stream())
+    work = torch.empty(4 * B * n_out * 2, dtype=torch.float64, device=gpu)
+    call('vc_ibp_fc_sliced', ptr(l), ptr(h), B, n_in, ptr(W), None, n_out, ptr(got[0]),
+         ptr(got[1]), 4, ptr(work), stream())
+    for x, y in zip(got, want):
+        assert torch.equal(x.isnan(), y.isnan())
+        ok = ~y.isnan()
+        assert torch.equal(x[ok].isinf(), y[ok].isinf()) and y[4:].isfinite().all()
+        assert float((x - y)[4:].abs().max()) <= 2 ** -22 * float(y[4:].abs().max())

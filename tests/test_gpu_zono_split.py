@@ -4,6 +4,7 @@ that do not vary, and against the forward that takes them one by one."""
 import pytest
 import torch
 
+from vibecheck_amd import _lib
 from vibecheck_amd import verify_zono_bnb as vz
 
 # boxes, widths, inputs held fixed, bytes of parts at a time
@@ -90,3 +91,33 @@ def test_zono_fc_split(gpu, case, monkeypatch):
     # the first layer's generators are single products: the same bits
     for a, b in zip(out[0][0], out[1e30][0]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_zono_fc_split_infinities(gpu):
+    """Generators that are infinite, NaN or round to infinity in bf16, some under
+    a zero slope: what the plain sum gives, in their own columns only."""
+    B, n, K, n_out = 2, 70, 90, 33
+    g = torch.Generator(device=gpu).manual_seed(5)
+    G = torch.randn(B, n, K, generator=g, device=gpu)
+    lam = torch.rand(B, n, generator=g, device=gpu)
+    W = torch.randn(n_out, n, generator=g, device=gpu) * 0.1
+    G[0, 3, 5], G[0, 69, 89], G[1, 20, 64] = float('inf'), float('-inf'), float('nan')
+    G[1, 40, 7], G[1, 41, 8] = 3.4e38, float('inf')
+    lam[1, 40], lam[1, 41] = 1.0, 0.0
+    size = _lib.load().vc_fc_split_pack_bytes
+    parts = torch.empty(size(n, n_out), dtype=torch.uint8, device=gpu)
+    _lib.call('vc_fc_split_pack', _lib.ptr(W), n, n_out, 1, _lib.ptr(parts), _lib.stream())
+    work = torch.empty(size(n, K) * B, dtype=torch.uint8, device=gpu)
+    out = torch.empty(B, n_out, K, device=gpu)
+    _lib.call('vc_zono_fc_split', _lib.ptr(G), _lib.ptr(lam), B, n, K, _lib.ptr(parts), n_out, K,
+              _lib.ptr(out), _lib.ptr(work), work.numel(), _lib.stream())
+    want = W.double() @ (G * lam.unsqueeze(2)).double()
+    f = want.float()
+    assert torch.equal(out.isnan(), f.isnan())
+    assert torch.equal(out[f.isinf()], f[f.isinf()])
+    big = f.isfinite() & (f.abs() > 1e30)  # sums rounded at their largest term's size
+    ok = f.isfinite() & ~big
+    assert int((~f.isfinite()).sum()) >= 4 * n_out - 4 and int(big.sum()) > 0
+    assert _rel(out[ok], want[ok]) < 2e-7  # as test_fc_split_against_fp64
+    assert ((out[big].double() - want[big]).abs() <= 1e-6 * want[big].abs()).all()

@@ -2,7 +2,11 @@
 // parts, each the rounding of what the parts before it leave,
 //   x = h + m + l,  |m| <= 2^-9 |x|,  |l| <= 2^-17 |x|,
 // exact for every x whose parts neither overflow nor fall below the smallest
-// normal (the three hold 24 bits).  Of the nine products of two such sums the
+// normal (the three hold 24 bits).  The matrix core takes smaller parts as
+// zero: products of rows or weights that are all below 2^-112 lose accuracy
+// (relative to 64 bits 5.2e-8 down to 2^-108, 1.5e-7 at 2^-112, 2.2e-6 at
+// 2^-116; the fp32 product 2.9e-7 throughout), smaller values beside larger
+// ones nothing that their sum shows.  Of the nine products of two such sums the
 // six largest are formed, each exact in fp32 and summed by the matrix core:
 //   a b = ah bh + ah bm + am bh + am bm + ah bl + al bh  (+ < 2^-24 |a b|).
 // gfx950 does 16x16x32 bf16 in 16 cycles against 32 for 16x16x4 fp32, so six
