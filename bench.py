@@ -786,17 +786,32 @@ LAYERWISE_MFMA = {
     'vc_zono_conv': lambda a: 2.0 * a[2] * (a[3] + 1) * a[9] * a[16] * a[17] * a[4] * a[10] * a[11],
     # 4 B (C_out H_out W_out)(C_in kh kw)
     'vc_ibp_conv': lambda a: 4.0 * a[2] * a[8] * a[15] * a[16] * a[3] * a[9] * a[10],
+    'vc_ibp_fc_sliced': lambda a: 4.0 * a[2] * a[3] * a[6],
+    # 2 M n_in n1
+    'vc_alpha_grad_input': lambda a: 2.0 * a[3] * a[5] * a[8],
 }
+# The same products as six bf16 part products each, from one call with the pass
+# that forms the rows' parts.
+LAYERWISE_PARTS = {
+    'vc_backward_fc_split': lambda a: 2.0 * a[1] * a[4] * a[11],
+    'vc_backward_conv_split': lambda a: 2.0 * a[1] * a[11] * a[12] * a[13] * a[14] * a[17] * a[18],
+    'vc_alpha_grad_step_split': lambda a: 2.0 * a[2] * a[4] * a[11],
+    'vc_alpha_grad_input_split': lambda a: 2.0 * a[3] * a[5] * a[8],
+    'vc_zono_fc_split': lambda a: 2.0 * a[2] * a[3] * a[4] * a[6],
+    'vc_ibp_conv_split': lambda a: 4.0 * a[2] * a[9] * a[16] * a[17] * a[3] * a[10] * a[11],
+}
+PARTS_PEAK = 2500.0 / 6  # dense bf16, six part products for one
 
 
 def layerwise_roofline(step, reps):
     """Run ``step`` with HIP events around every layer-wise MFMA entry
     point: per entry its time per step, algorithmic TFLOP/s and fraction of
-    the fp32 MFMA peak; the roofline is the entry with the most time."""
+    the fp32 MFMA peak (of a sixth of the dense bf16 peak for the products of
+    parts); the roofline is the entry with the most time."""
     from vibecheck_amd import _lib
-    for name, f in LAYERWISE_MFMA.items():
-        _lib._FLOPS[name] = f
-    _lib.timing_begin(list(LAYERWISE_MFMA))
+    entries = {**LAYERWISE_MFMA, **LAYERWISE_PARTS}
+    _lib._FLOPS.update(entries)
+    _lib.timing_begin(list(entries))
     for _ in range(reps):
         step()
     kt = _lib.timing_end()
@@ -804,9 +819,10 @@ def layerwise_roofline(step, reps):
     for name, k in kt.items():
         if k['launches'] and k['seconds'] > 0:
             ach = k['flops'] / k['seconds'] / 1e12
+            peak = PARTS_PEAK if name in LAYERWISE_PARTS else FP32_MFMA_PEAK
             rows.append({'entry': name, 'ms_per_step': 1e3 * k['seconds'] / reps,
                          'launches_per_step': k['launches'] / reps, 'achieved': ach,
-                         'frac': ach / FP32_MFMA_PEAK})
+                         'peak': peak, 'frac': ach / peak})
     rows.sort(key=lambda r: -r['ms_per_step'])
     return rows
 
@@ -1007,10 +1023,11 @@ def run_config(cfg, steps, warmup, cpu):
         rows = layerwise_roofline(step, steps)
         top = rows[0]
         how = {'vc_backward_fc': 'relaxation pass + rocBLAS sgemm',
-               'vc_zono_fc': 'rocBLAS strided-batched sgemm for the generators'}.get(
+               'vc_zono_fc': 'rocBLAS strided-batched sgemm for the generators',
+               **{k: 'products of bf16 parts' for k in LAYERWISE_PARTS}}.get(
                    top['entry'], 'MFMA GEMM core')
         line['roofline'] = {'kernel': f'{top["entry"]} ({how})', 'bound': 'mfma',
-                            'achieved': top['achieved'], 'peak': FP32_MFMA_PEAK,
+                            'achieved': top['achieved'], 'peak': top['peak'],
                             'unit': 'TFLOP/s', 'frac': top['frac'], 'traffic': None,
                             'share_of_step': top['ms_per_step'] / (1e3 * per_step)}
         line['mfma_entries'] = rows
