@@ -590,38 +590,43 @@ __global__ void k_patch_shift(const int* in, int n, int sh, int sw, int ph, int 
 }
 
 // Rows of windows relaxed by their domains' slopes at the windows' places in
-// the image (ls null: copied), zero outside the image, and the intercepts
-// added to acc in 64 bits: the separate relu step on windows.  One wave per
-// row, lanes along it: each row is read and written once, coalesced.
+// the image (RELU 0: copied), zero outside the image, and the intercepts added
+// to acc in 64 bits: the separate relu step on windows.  One wave per row, lanes
+// along it: each row is read and written once, coalesced; a lane's four loads
+// go out together, outside the image from its first pixel, not used.
+template <bool RELU>
 __global__ __launch_bounds__(CNT) void k_patch_relax(const float* x, int shared, const float* ls,
                                                      const float* us, const float* ut,
-                                                     const int* origin, int64_t M, int64_t R, int C, int H, int W,
-                                                     int wh, int ww, FastDiv f_ww, FastDiv f_wp,
-                                                     float* out, float* acc) {
+                                                     const int* origin, int64_t M, int64_t R,
+                                                     int C, int H, int W, int wh, int ww,
+                                                     FastDiv f_ww, FastDiv f_wp, float* out,
+                                                     float* acc) {
   const int wp = wh * ww, n = C * wp, lane = threadIdx.x & 63;
-  for (int64_t m = (int64_t)blockIdx.x * (CNT / 64) + (threadIdx.x >> 6); m < M;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t m = (int64_t)blockIdx.x * (CNT / 64) + wv; m < M;
        m += (int64_t)gridDim.x * (CNT / 64)) {
     const int64_t d = m / R, row = m - d * R, img = d * C * H * W;
     const float* a = x + (shared ? row : m) * n;
+    const float *lm = ls + img, *um = us + img, *tm = ut + img;
+    float* const om = out + m * n;
     const int oy = origin[2 * row], ox = origin[2 * row + 1];
     double s = 0.0;
     for (int i = lane; i < n; i += 64) {
       const int c = (int)f_wp.div((uint32_t)i), p = i - c * wp;
       const int dy = (int)f_ww.div((uint32_t)p), dx = p - dy * ww;
       const int y = oy + dy, xx = ox + dx;
-      float e = 0.f;
-      if ((unsigned)y < (unsigned)H && (unsigned)xx < (unsigned)W) {
-        e = a[i];
-        if (ls) {
-          const int64_t o = img + (c * H + y) * W + xx;
-          const float en = e > 0.f ? 0.f : e, ep = e < 0.f ? 0.f : e;
-          s += (double)(en * ut[o]);
-          e = ep * ls[o] + en * us[o];
-        }
+      const bool in = (unsigned)y < (unsigned)H && (unsigned)xx < (unsigned)W;
+      float e = a[(uint32_t)i];
+      if (RELU) {
+        const uint32_t o = in ? (c * H + y) * W + xx : 0;
+        const float l = lm[o], u = um[o], t = tm[o];
+        const float en = e > 0.f ? 0.f : e, ep = e < 0.f ? 0.f : e;
+        s += in ? (double)(en * t) : 0.0;
+        e = ep * l + en * u;
       }
-      out[m * n + i] = e;
+      om[(uint32_t)i] = in ? e : 0.f;
     }
-    if (ls) {
+    if (RELU) {
       s = wave_sum_f64(s);
       if (lane == 0) acc[m] = (float)((double)acc[m] + s);
     }
@@ -791,9 +796,10 @@ extern "C" int vc_patch_relax(const float* ew_in, int64_t M, int64_t R, int ew_s
     return VC_ERR_ARG;
   if ((int64_t)C * wh * ww > (1 << 30) || (int64_t)C * H * W > (1 << 30)) return VC_ERR_UNSUPPORTED;
   if (M == 0) return VC_OK;
-  hipLaunchKernelGGL(k_patch_relax, dim3(vc_blocks(64 * M, CNT)), dim3(CNT), 0,
-                     (hipStream_t)stream, ew_in, ew_shared ? 1 : 0, lo_s, up_s, up_t, origin, M, R, C, H, W, wh, ww, FastDiv::make((uint32_t)ww),
-                     FastDiv::make((uint32_t)(wh * ww)), ew_out, acc);
+  hipLaunchKernelGGL(lo_s ? k_patch_relax<true> : k_patch_relax<false>,
+                     dim3(vc_blocks(64 * M, CNT)), dim3(CNT), 0, (hipStream_t)stream, ew_in,
+                     ew_shared ? 1 : 0, lo_s, up_s, up_t, origin, M, R, C, H, W, wh, ww,
+                     FastDiv::make((uint32_t)ww), FastDiv::make((uint32_t)(wh * ww)), ew_out, acc);
   VC_LAUNCH_CHECK();
   return VC_OK;
 }
