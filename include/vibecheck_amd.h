@@ -321,14 +321,12 @@ int vc_backward_conv(const float *ew_in, int64_t M, const float *kernel,
                      int ph, int pw, float *ew_out, float *acc,
                      vc_stream_t stream);
 
-/* The taps of the transposed convolution packed once per kernel for
+/* The taps of the transposed convolution packed for
  * vc_backward_conv_packed: for each of the sh * sw output-parity classes,
  * C_in rows of C_out * ceil(kh / sh) * ceil(kw / sw) taps (zero past the
  * kernel), rows padded to a multiple of 4 floats; vc_conv_t_pack_floats
  * gives the size.  The reference has no counterpart (it calls
- * conv_transpose2d, verify_zono_bnb.py:4568-4593): the packing is this
- * build's weight cache, like the reference's cached op tensors
- * (verify_zono_bnb.py:4482-4486). */
+ * conv_transpose2d, verify_zono_bnb.py:4568-4593). */
 int64_t vc_conv_t_pack_floats(int C_out, int C_in, int kh, int kw, int sh, int sw);
 int vc_conv_t_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,
                    int sw, int ph, int pw, float *out, vc_stream_t stream);
@@ -374,7 +372,7 @@ int vc_backward_relu_conv(const float *ew_in, int64_t M, int64_t R, int ew_share
  * for M = B * R rows, x from input row m or, with ew_shared, row m mod R of the
  * R rows every domain shares.  Slopes and beta as in vc_backward_relu_conv.
  * packed: the kernel's parts from vc_conv_split_pack (16-byte aligned,
- * vc_conv_split_pack_bytes of them), laid out once per kernel; kernel itself is
+ * vc_conv_split_pack_bytes of them); kernel itself is
  * read where an infinity or NaN among the values asks for the plain sum.
  * vc_backward_conv_split_ok says whether a geometry qualifies (for one row),
  * vc_backward_conv_split_fits whether M of them do (one tile's images, or the R
