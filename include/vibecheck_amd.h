@@ -376,7 +376,8 @@ int vc_backward_relu_conv(const float *ew_in, int64_t M, int64_t R, int ew_share
  * read where an infinity or NaN among the values asks for the plain sum.
  * vc_backward_conv_split_ok says whether a geometry qualifies (for one row),
  * vc_backward_conv_split_fits whether M of them do (one tile's images, or the R
- * shared rows, within 32-bit offsets), else VC_ERR_UNSUPPORTED.
+ * shared rows, within 32-bit offsets), else VC_ERR_UNSUPPORTED, and in how many
+ * bands one workgroup takes an image.
  * Replaces verify_zono_bnb.py:4409-4453 followed by 4568-4593. */
 int64_t vc_conv_split_pack_bytes(int C_out, int C_in, int kh, int kw, int sh, int sw);
 int vc_conv_split_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,

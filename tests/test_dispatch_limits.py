@@ -63,6 +63,23 @@ def test_interval_conv_of_many_pixels(launches, monkeypatch, side, entry):
     assert launches.count(entry) == (2 if entry == 'vc_ibp_conv' else 1)
 
 
+# rows; channels in and out, side, kernel, stride, padding; whether the split conv
+# was measured the faster, weights packed and the relu before it included
+@pytest.mark.parametrize('M,geom,split', [
+    (6, (16, 8, 28, 3, 1, 1), False), (60, (16, 8, 28, 3, 1, 1), False),
+    (300, (16, 8, 28, 3, 1, 1), True), (6, (33, 17, 20, 3, 1, 1), False),
+    (120, (33, 17, 20, 3, 1, 1), False), (300, (33, 17, 20, 3, 1, 1), True),
+    (6, (64, 64, 32, 3, 1, 1), False), (12, (64, 64, 32, 3, 1, 1), False),
+    (30, (64, 64, 32, 3, 1, 1), True), (6, (13, 8, 14, 3, 1, 0), True),
+    (12, (64, 32, 32, 4, 2, 1), True), (6, (32, 16, 28, 5, 2, 2), True)])
+def test_split_conv_rule(launches, M, geom, split):
+    co, ci, side, k, s, pad = geom
+    out = (side + 2 * pad - k) // s + 1
+    p = {'name': 'c', 'geom': (ci, side, side, co, k, k, s, s, pad, pad, out, out),
+         'K': torch.empty(co, ci, k, k, device=META), 'n_out': co * out * out}
+    assert (vz._Packs().conv_split(p, M, M, False, 0) is not None) == split
+
+
 def test_window_limits():
     """Images of more than 2^30 values are carried whole."""
     assert vz._Window(None, 3, 3, 4, 1 << 14, 1 << 14).worth()

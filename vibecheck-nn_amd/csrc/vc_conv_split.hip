@@ -730,7 +730,7 @@ extern "C" int vc_backward_conv_split_fits(int64_t M, int64_t R, int ew_shared, 
   a.C_out = C_out, a.Hs = H_out, a.Ws = W_out, a.Hi = H_out, a.Wi = W_out;
   a.C_in = C_in, a.H = H, a.W = W;
   a.kh = kh, a.kw = kw, a.sh = sh, a.sw = sw, a.ph = ph, a.pw = pw;
-  return split_fits(a) ? 1 : 0;
+  return split_fits(a) ? a.NB : 0;
 }
 
 extern "C" int vc_backward_conv_split(const float* ew_in, int64_t M, int64_t R, int ew_shared,

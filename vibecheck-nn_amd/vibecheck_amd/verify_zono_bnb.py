@@ -221,6 +221,9 @@ class _Packs:
             self._made[p['name'], 'interval'] = out
         return out
 
+    def has_taps(self, p, window):
+        return (p['name'], 'taps', window) in self._made
+
     def conv_taps(self, p, st, window=False):
         """A conv kernel's transposed taps by output-parity class
         (vc_conv_t_pack); ``window``: without the padding, for rows that carry
@@ -242,10 +245,12 @@ class _Packs:
     def conv_split(self, p, M, R, shared, st):
         """A conv kernel's bf16 parts for vc_backward_conv_split of M rows (R a
         domain, shared by all domains or not); None where the geometry or the
-        rows are outside that kernel."""
+        rows are outside that kernel, or the fp32 product is the faster one."""
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        if not _lib.load().vc_backward_conv_split_fits(M, R, 1 if shared else 0, C_out, Ho, Wo,
-                                                       C_in, H, W, kh, kw, sh, sw, ph, pw):
+        bands = _lib.load().vc_backward_conv_split_fits(
+            M, R, 1 if shared else 0, C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
+        if bands == 0 or (bands > 1 and M < _CONV_SPLIT_ROWS
+                          and M * p['n_out'] * C_in * kh * kw < _CONV_SPLIT_MACS):
             return None
         out = self._made.get((p['name'], 'conv_split'))
         if out is None:
@@ -851,6 +856,21 @@ _TWO_PHASE_MIN_WIDTH = 64
 #   128 x 33     18,432: 18 and 18;  64 x 64: 10 and 14.
 _FC_SPLIT_SWEEP_ROWS = 64
 _FC_SPLIT_WIDTH = 128
+# The split conv takes a large image band by band in one workgroup, a few rows of
+# them on as many CUs, while the gathering product spreads their pixels.  Both
+# from the rows to the product, weights packed, us (split; relu and fp32 conv):
+#   16 -> 8, 3x3, 28x28    6 rows 65 and 37;  60: 65 and 56;  120: 65 and 70
+#   33 -> 17, 3x3, 20x20   6: 76 and 47;     120: 78 and 71;  300: 97 and 112
+#   64 -> 64, 3x3, 32x32   6 (0.23e9 multiplications): 210 and 153;  12: 212 and
+#                          195;  30 (1.1e9): 213 and 239
+# An image in one band is as fast or faster at any number of rows (13 -> 8, 14x14,
+# 6: 22 and 25; 64 -> 32, 4x4 stride 2 onto 32x32, 6: 51 and 48, 12: 52 and 57).
+_CONV_SPLIT_ROWS = 128
+_CONV_SPLIT_MACS = 5e8
+# Below, packing the taps costs what it saves (with it and without: 16 -> 8,
+# 28x28, 60 rows 57 and 56, 300 rows 110 and 123; 64 -> 64 onto 16x16, 12 rows 32
+# and 31) and is a launch more.
+_CONV_TAPS_MACS = 5e7
 _SLOPES_KEPT_BYTES = 32 << 20  # a layer's; forming them takes 10 us at that size
 # Parts of rows take so much at a time, whatever the number of rows.  Slices
 # that the last-level cache holds (192 MiB) are no faster (73,728 rows of 1024 x
@@ -989,12 +1009,14 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
 
     def conv_fp32(p, ew, M, window, out, bias, acc):
         """M rows through a conv in fp32, acc += rows . bias; the fold kernel
-        reads the kernel as it lies, the gathering product its packed taps."""
+        reads the kernel as it lies, the gathering product its packed taps, or
+        for few rows their kernel (the same bits)."""
         C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
         if window is not None:
             (Ho, Wo, H, W), ph, pw = window, 0, 0
         geom = (C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
-        if few_channels(p, window):
+        if few_channels(p, window) or (M * C_out * Ho * Wo * C_in * kh * kw < _CONV_TAPS_MACS
+                                       and not packs.has_taps(p, window is not None)):
             call('vc_backward_conv', ptr(ew), M, ptr(p['K']), ptr(bias), *geom, ptr(out),
                  ptr(acc), st)
         else:
