@@ -239,7 +239,8 @@ int vc_relax_slopes(const float *relu_lo, const float *relu_hi,
  * aligned).  Slopes (M / R, K) as from vc_relax_slopes; packed: W's parts from
  * vc_fc_split_pack (vc_fc_split_pack_bytes(K, N), 16-byte aligned), of W (K, N)
  * or with trans of W (N, K) whose transpose is meant (vc_fc_split_pack_abs: of
- * W and of |W|, from one pass).  M < 2^31.
+ * W and of |W|, from one pass; vc_fc_split_pack_many: of count matrices, host
+ * arrays of their pointers and sizes, sixteen a launch).  M < 2^31.
  * vc_backward_fc_split: e = pos(x) lo_s + neg(x) up_s [+ beta (M / R, n_out)],
  *   ew_out (M, n_in) = e W, acc[m] += neg(x) . up_t + e . bias, x from row m or,
  *   with ew_shared, row m mod R.  Replaces verify_zono_bnb.py:4379-4453.
@@ -249,6 +250,8 @@ int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N);
 int vc_fc_split_pack(const float *W, int K, int N, int trans, void *out, vc_stream_t stream);
 int vc_fc_split_pack_abs(const float *W, int K, int N, int trans, void *out, void *out_abs,
                          vc_stream_t stream);
+int vc_fc_split_pack_many(const float *const *W, const int32_t *K, const int32_t *N, int trans,
+                          void *const *out, int count, vc_stream_t stream);
 int vc_backward_fc_split(const float *ew_in, int64_t M, int R, int ew_shared, int n_out,
                          const float *lo_s, const float *up_s, const float *up_t,
                          const float *beta, const void *packed, const float *bias, int n_in,

@@ -1,5 +1,7 @@
 """vc_ibp_conv_split (the interval forward of a conv as products of bf16 parts)
 against 64-bit sums, at the edges of its pixel tiles, chunks and column tiles."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -105,3 +107,28 @@ def test_pack_abs_is_two_packs(gpu):
     for w, o in ((W, out[2]), (Wa, out[3])):
         call('vc_fc_split_pack', ptr(w), 75, 37, 1, ptr(o), stream())
     assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('trans', [0, 1])
+def test_pack_many_is_each_pack(gpu, trans):
+    """Nineteen matrices, more than a launch takes, of one to eight workgroups."""
+    g = torch.Generator(device=gpu).manual_seed(4)
+    size = _lib.load().vc_fc_split_pack_bytes
+    KN = [(1 + 37 * i, 1 + 11 * (18 - i)) for i in range(19)]
+    W = [torch.randn(*((N, K) if trans else (K, N)), generator=g, device=gpu) for K, N in KN]
+    many = [torch.empty(size(K, N), dtype=torch.uint8, device=gpu) for K, N in KN]
+    arrays = [_lib.host_array(ctypes.c_void_p, [ptr(w) for w in W]),
+              _lib.host_array(ctypes.c_int32, [K for K, _ in KN]),
+              _lib.host_array(ctypes.c_int32, [N for _, N in KN]),
+              _lib.host_array(ctypes.c_void_p, [ptr(m) for m in many])]
+    call('vc_fc_split_pack_many', *(p for _, p in arrays[:3]), trans, arrays[3][1], 19, stream())
+    for (K, N), w, m in zip(KN, W, many):
+        one = torch.empty_like(m)
+        call('vc_fc_split_pack', ptr(w), K, N, trans, ptr(one), stream())
+        assert torch.equal(m, one)
+        # the parts' sum is the value (bf16 in operand order)
+        p = one.view(torch.bfloat16).view((N + 15) // 16, -1, 3, 4, 16, 8).double().sum(2)
+        B = p.permute(1, 2, 4, 0, 3).reshape(64 * -(-K // 64), -1)
+        assert torch.equal(B[:K, :N], (w.T if trans else w).double())
+        assert not B[K:].any() and not B[:, N:].any()

@@ -37,7 +37,7 @@ def _mlp(widths, dtype=F32, dev='cpu'):
             'input_shape': (1, widths[0]), 'n_relu': len(widths) - 2}
 
 
-MLP = [70, 140, 130, 9]
+MLP = [70, 140, 130, 150, 9]
 
 
 def _cnn(dtype=F32, dev='cpu'):
@@ -107,6 +107,9 @@ def launches(monkeypatch, small):
             src, outs = PACKS[name]
             for i in outs:
                 rec['packed'][id(a[i])] = (a[i], a[-1], a[src], a[src].clone())
+        if name == 'vc_fc_split_pack_many':
+            for w, out in zip(a[0], a[4]):
+                rec['packed'][id(out)] = (out, a[-1], w, w.clone())
         for i in READS.get(name, []):
             _, st, src, was = rec['packed'][id(a[i])]
             assert st == a[-1], f'{name} reads weights packed on another stream'
@@ -122,6 +125,7 @@ def launches(monkeypatch, small):
 
     monkeypatch.setattr(vz, 'call', call)
     monkeypatch.setattr(vz, 'ptr', lambda t: t)
+    monkeypatch.setattr(vz, 'host_array', lambda ctype, values: (values, values))
     monkeypatch.setattr(vz, 'f32', lambda t: t.contiguous())
     monkeypatch.setattr(vz, 'stream', lambda: rec['stream'])
     return rec

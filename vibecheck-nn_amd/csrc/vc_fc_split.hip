@@ -563,46 +563,66 @@ __global__ __launch_bounds__(FNT) void k_zono_cols(const float* W, int n_out, in
   }
 }
 
-// Wp[column tile][32-deep step][part][lane][8]: part of B[k][n] for
+// One matrix' parts; and as many as a launch's arguments hold.
+struct Pack {
+  const float* W;
+  uint4 *out, *out_abs;
+  int K, N, trans, nkc;
+  uint32_t block0;  // its first workgroup
+};
+constexpr int kPacks = 16;
+struct Packs {
+  Pack p[kPacks];
+  int count;
+};
+
+// out[column tile][32-deep step][part][lane][8]: part of B[k][n] for
 // k = 32 step + 8 (lane / 16) + j, n = 16 tile + lane % 16; zero past the ends.
-// out_abs (or null): the same of |B|.
-__global__ void k_fc_split_pack(const float* W, int K, int N, int trans, int nkc, int64_t total,
-                                uint4* out, uint4* out_abs) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int lane = (int)(t & 63);
-    const int64_t q = t >> 6;
-    const int kc = (int)(q % nkc), n = (int)(q / nkc) * 16 + (lane & 15);
-    const int k0 = kc * FBK + 8 * (lane >> 4);
-    float v[8];
+// out_abs (or null): the same of |B|.  A launch takes 5 us whatever it packs up
+// to a million weights, so a call's matrices go together (five of 256 x 256: 22
+// us apart, 6 together).
+__global__ __launch_bounds__(256) void k_fc_split_pack(Packs a) {
+  int i = 0;
+  while (i + 1 < a.count && blockIdx.x >= a.p[i + 1].block0) ++i;
+  const Pack& m = a.p[i];
+  const int64_t t = (int64_t)(blockIdx.x - m.block0) * 256 + threadIdx.x;
+  const int64_t q = t >> 6;
+  if (q >= (int64_t)((m.N + 15) >> 4) * m.nkc) return;
+  const int lane = (int)(t & 63);
+  const int kc = (int)(q % m.nkc), n = (int)(q / m.nkc) * 16 + (lane & 15);
+  const int k0 = kc * FBK + 8 * (lane >> 4);
+  float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = n < N && k0 + j < K
-                 ? (trans ? W[(int64_t)n * K + k0 + j] : W[(int64_t)(k0 + j) * N + n])
-                 : 0.f;
-    uint4 h, m, l;
-    split8_all(v, h, m, l);
-    uint4* o = out + q * kTileU + lane;
-    o[0] = h;
-    o[64] = m;
-    o[128] = l;
-    if (!out_abs) continue;
+  for (int j = 0; j < 8; ++j)
+    v[j] = n < m.N && k0 + j < m.K
+               ? (m.trans ? m.W[(int64_t)n * m.K + k0 + j] : m.W[(int64_t)(k0 + j) * m.N + n])
+               : 0.f;
+  uint4 h, md, l;
+  split8_all(v, h, md, l);
+  uint4* o = m.out + q * kTileU + lane;
+  o[0] = h;
+  o[64] = md;
+  o[128] = l;
+  if (!m.out_abs) return;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = fabsf(v[j]);
-    split8_all(v, h, m, l);
-    o = out_abs + q * kTileU + lane;
-    o[0] = h;
-    o[64] = m;
-    o[128] = l;
-  }
+  for (int j = 0; j < 8; ++j) v[j] = fabsf(v[j]);
+  split8_all(v, h, md, l);
+  o = m.out_abs + q * kTileU + lane;
+  o[0] = h;
+  o[64] = md;
+  o[128] = l;
 }
 
-int launch_pack(const float* W, int K, int N, int trans, void* out, void* out_abs,
-                hipStream_t st) {
-  const int nkc = 2 * ((K + 2 * FBK - 1) / (2 * FBK));
-  const int64_t total = (int64_t)((N + 15) / 16) * nkc * 64;
-  hipLaunchKernelGGL(k_fc_split_pack, dim3(vc_blocks(total, 256)), dim3(256), 0, st, W, K, N,
-                     trans, nkc, total, (uint4*)out, (uint4*)out_abs);
+int launch_pack(Packs& a, hipStream_t st) {
+  int64_t blocks = 0;
+  for (int i = 0; i < a.count; ++i) {
+    Pack& m = a.p[i];
+    m.nkc = 2 * ((m.K + 2 * FBK - 1) / (2 * FBK));
+    m.block0 = (uint32_t)blocks;
+    blocks += ((int64_t)((m.N + 15) / 16) * m.nkc * 64 + 255) / 256;
+    if (blocks >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+  }
+  hipLaunchKernelGGL(k_fc_split_pack, dim3((unsigned)blocks), dim3(256), 0, st, a);
   VC_LAUNCH_CHECK();
   return VC_OK;
 }
@@ -671,14 +691,33 @@ extern "C" int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N) {
 extern "C" int vc_fc_split_pack(const float* W, int K, int N, int trans, void* out,
                                 vc_stream_t stream) {
   if (!W || !out || K <= 0 || N <= 0 || !aligned16(out)) return VC_ERR_ARG;
-  return launch_pack(W, K, N, trans, out, nullptr, (hipStream_t)stream);
+  Packs a{{{W, (uint4*)out, nullptr, K, N, trans}}, 1};
+  return launch_pack(a, (hipStream_t)stream);
 }
 
 extern "C" int vc_fc_split_pack_abs(const float* W, int K, int N, int trans, void* out,
                                     void* out_abs, vc_stream_t stream) {
   if (!W || !out || !out_abs || K <= 0 || N <= 0 || !aligned16(out) || !aligned16(out_abs))
     return VC_ERR_ARG;
-  return launch_pack(W, K, N, trans, out, out_abs, (hipStream_t)stream);
+  Packs a{{{W, (uint4*)out, (uint4*)out_abs, K, N, trans}}, 1};
+  return launch_pack(a, (hipStream_t)stream);
+}
+
+extern "C" int vc_fc_split_pack_many(const float* const* W, const int32_t* K, const int32_t* N,
+                                     int trans, void* const* out, int count,
+                                     vc_stream_t stream) {
+  if (count < 0 || (count > 0 && (!W || !K || !N || !out))) return VC_ERR_ARG;
+  for (int i = 0; i < count; ++i)
+    if (!W[i] || !out[i] || K[i] <= 0 || N[i] <= 0 || !aligned16(out[i])) return VC_ERR_ARG;
+  for (int i0 = 0; i0 < count; i0 += kPacks) {
+    Packs a{};
+    a.count = count - i0 < kPacks ? count - i0 : kPacks;
+    for (int i = 0; i < a.count; ++i)
+      a.p[i] = Pack{W[i0 + i], (uint4*)out[i0 + i], nullptr, K[i0 + i], N[i0 + i], trans};
+    const int rc = launch_pack(a, (hipStream_t)stream);
+    if (rc != VC_OK) return rc;
+  }
+  return VC_OK;
 }
 
 extern "C" int vc_backward_fc_split(const float* ew_in, int64_t M, int R, int ew_shared, int n_out,
