@@ -79,3 +79,26 @@ def test_shortcut_before_main_branch(gpu, kind, split):
                                          torch.float32, seed_ew_at={'merge': s})
     ref = ref[0] if isinstance(ref, tuple) else ref
     assert (lb.cpu().double() - ref).norm() <= 2e-6 * ref.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B', [1, 3])
+@pytest.mark.parametrize('bias', [False, True])
+def test_callers_constant_terms_stay(gpu, B, bias):
+    """The shared rows' constant terms are the caller's: a call leaves them as
+    they are, also for one domain, whose own terms would be the same memory."""
+    gg, n_in = _net('conv8')
+    for op in gg['ops']:
+        if op['type'] == 'fc':
+            op['bias'] = op['bias'] if bias else None
+    xl, xh = (t.to(gpu) for t in wk.linf_boxes(B, n_in, 0.05, seed=5))
+    sb = vz._ibp_forward_graph_batched(xl, xh, gg, gpu, torch.float32)
+    W, b = torch.randn(4, 5, device=gpu), torch.randn(4, device=gpu)
+    keep = b.clone()
+    out = [vz._backward(sb, xl, xh, gg, 'head', W, True, b) for _ in range(2)]
+    assert torch.equal(b, keep)
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][3], out[1][3])
+    spec = {0: (W[0], 1.5)}
+    lb = [vz._spec_backward_graph_batched(sb, xl, xh, gg, spec, gpu, torch.float32)
+          for _ in range(2)]
+    assert torch.equal(lb[0], lb[1])

@@ -908,7 +908,7 @@ def _expand_rows(t, B):
 
 def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
               alpha_at_layer=None, relu_split_beta=None, trace=None, split=True,
-              packs=None):
+              packs=None, fresh=False):
     """Walk the ops backward from ``seed_name`` and concretize.
 
     seed: (R, n) rows when ``seed_shared`` else (B*R, n), or a _Rows; acc0:
@@ -916,7 +916,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     the matrix cores; off where the bounds choose slopes, whose step at 1/2
     turns a last-bit change of a bound into another lower slope (on 512 boxes
     through 1024-wide layers one run in four).  packs: the caller's _Packs, where
-    it makes several of these calls.  Returns (lb (B, R), A, a_shared, acc (B*R,));
+    it makes several of these calls; fresh: acc0 is this call's to write to.
+    Returns (lb (B, R), A, a_shared, acc (B*R,));
     A of window rows is None.
     """
     once = packs is None
@@ -927,16 +928,24 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     widths = _widths(gg, n_in)
     rows = seed if isinstance(seed, _Rows) else _Rows(seed, seed_shared)
     R = rows.ew.shape[0] if seed_shared else rows.ew.shape[0] // max(B, 1)
-    acc = acc0.clone()
+    acc, acc_own = (acc0, fresh) if seed_shared else (acc0.clone(), True)
     acc_shared = seed_shared
     ew_at = {seed_name: rows}
     ops = gg['ops']
 
     def per_domain_acc():
-        nonlocal acc, acc_shared
+        nonlocal acc, acc_own, acc_shared
         if acc_shared:
+            if B == 1:  # the expansion is the same memory
+                own_acc()
             acc = acc.unsqueeze(0).expand(B, R).reshape(B * R).contiguous()
-            acc_shared = False
+            acc_own, acc_shared = True, False
+
+    def own_acc():
+        """Before a write to shared constant terms: acc0 stays as it is."""
+        nonlocal acc, acc_own
+        if not acc_own:
+            acc, acc_own = acc.clone(), True
 
     def combine(a, b):
         """Rows reaching one node from two consumers, summed (ew_at[inp] +
@@ -963,6 +972,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         """acc += sign * rows . v (the constant of an add or sub)."""
         n = rows.ew.shape[1]
         if rows.shared and acc_shared:
+            own_acc()
             call('vc_rows_bias_dot', ptr(rows.ew), R, R, n, 1, ptr(v), v.numel(), sign,
                  ptr(acc), st)
         else:
@@ -980,6 +990,8 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
                 if p['b'] is not None:
                     bias_dot(rows, p['b'].repeat_interleave(p['n_out'] // p['b'].numel()), 1.0)
                 return None, None
+            if p['b'] is not None:
+                own_acc()
         else:
             per_domain_acc()
         return p['b'], acc
@@ -1476,7 +1488,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
                      st)
                 rows.window = _Window(origin, kh, kw, C_in, H, W)
                 sl, _, _, _ = _backward(tight, xl, xh, gg, below, rows, True, acc0,
-                                        split=False, packs=packs)
+                                        split=False, packs=packs, fresh=True)
                 call('vc_crown_intersect', ptr(sl.contiguous()), ptr(cidx), k, B, n,
                      ptr(new_lo), ptr(new_hi), st)
                 continue
@@ -1486,7 +1498,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
             seed[ar + k, cidx.long()] = -1.0
             acc0 = torch.zeros(2 * k, device=dev)
             sl, _, _, _ = _backward(tight, xl, xh, gg, feed, seed, True, acc0, split=False,
-                                    packs=packs)
+                                    packs=packs, fresh=True)
             sl = sl.contiguous()
             call('vc_crown_intersect', ptr(sl), ptr(cidx), k, B, n,
                  ptr(new_lo), ptr(new_hi), st)
