@@ -239,8 +239,8 @@ int vc_relax_slopes(const float *relu_lo, const float *relu_hi,
  * aligned).  Slopes (M / R, K) as from vc_relax_slopes; packed: W's parts from
  * vc_fc_split_pack (vc_fc_split_pack_bytes(K, N), 16-byte aligned), of W (K, N)
  * or with trans of W (N, K) whose transpose is meant (vc_fc_split_pack_abs: of
- * W and of |W|, from one pass; vc_fc_split_pack_many: of count matrices, host
- * arrays of their pointers and sizes, sixteen a launch).  M < 2^31.
+ * W and of |W|, from one pass; vc_fc_split_pack_many: of count matrices, from
+ * host arrays of their pointers, sizes and forms, sixteen a launch).  M < 2^31.
  * vc_backward_fc_split: e = pos(x) lo_s + neg(x) up_s [+ beta (M / R, n_out)],
  *   ew_out (M, n_in) = e W, acc[m] += neg(x) . up_t + e . bias, x from row m or,
  *   with ew_shared, row m mod R.  Replaces verify_zono_bnb.py:4379-4453.
@@ -250,8 +250,9 @@ int64_t vc_fc_split_pack_bytes(int64_t K, int64_t N);
 int vc_fc_split_pack(const float *W, int K, int N, int trans, void *out, vc_stream_t stream);
 int vc_fc_split_pack_abs(const float *W, int K, int N, int trans, void *out, void *out_abs,
                          vc_stream_t stream);
-int vc_fc_split_pack_many(const float *const *W, const int32_t *K, const int32_t *N, int trans,
-                          void *const *out, int count, vc_stream_t stream);
+int vc_fc_split_pack_many(const float *const *W, const int32_t *K, const int32_t *N,
+                          const int32_t *trans, void *const *out, int count,
+                          vc_stream_t stream);
 int vc_backward_fc_split(const float *ew_in, int64_t M, int R, int ew_shared, int n_out,
                          const float *lo_s, const float *up_s, const float *up_t,
                          const float *beta, const void *packed, const float *bias, int n_in,
@@ -333,6 +334,10 @@ int vc_backward_conv(const float *ew_in, int64_t M, const float *kernel,
 int64_t vc_conv_t_pack_floats(int C_out, int C_in, int kh, int kw, int sh, int sw);
 int vc_conv_t_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,
                    int sw, int ph, int pw, float *out, vc_stream_t stream);
+/* Of count kernels, sixteen a launch; geom: (C_out, C_in, kh, kw, sh, sw, ph, pw)
+ * of each.  All three arrays are the host's. */
+int vc_conv_t_pack_many(const float *const *kernel, const int32_t *geom, float *const *out,
+                        int count, vc_stream_t stream);
 
 /* vc_backward_conv reading the packed taps (16-byte aligned, from
  * vc_conv_t_pack of the same kernel and geometry) instead of deriving each
@@ -385,6 +390,10 @@ int vc_backward_relu_conv(const float *ew_in, int64_t M, int64_t R, int ew_share
 int64_t vc_conv_split_pack_bytes(int C_out, int C_in, int kh, int kw, int sh, int sw);
 int vc_conv_split_pack(const float *kernel, int C_out, int C_in, int kh, int kw, int sh,
                        int sw, void *out, vc_stream_t stream);
+/* Of count kernels, sixteen a launch; geom: (C_out, C_in, kh, kw, sh, sw) of each.
+ * All three arrays are the host's. */
+int vc_conv_split_pack_many(const float *const *kernel, const int32_t *geom, void *const *out,
+                            int count, vc_stream_t stream);
 int vc_backward_conv_split_ok(int C_out, int H_out, int W_out, int C_in, int H, int W,
                               int kh, int kw, int sh, int sw, int ph, int pw);
 int vc_backward_conv_split_fits(int64_t M, int64_t R, int ew_shared, int C_out, int H_out,

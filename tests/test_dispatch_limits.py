@@ -15,6 +15,7 @@ def launches(monkeypatch):
     names = []
     monkeypatch.setattr(vz, 'call', lambda name, *a: names.append(name))
     monkeypatch.setattr(vz, 'ptr', lambda t: t)
+    monkeypatch.setattr(vz, 'host_array', lambda ctype, values: (values, values))
     monkeypatch.setattr(vz, 'f32', lambda t: t.contiguous())
     monkeypatch.setattr(vz, 'stream', lambda: 0)
     return names
@@ -76,8 +77,9 @@ def test_split_conv_rule(launches, M, geom, split):
     co, ci, side, k, s, pad = geom
     out = (side + 2 * pad - k) // s + 1
     p = {'name': 'c', 'geom': (ci, side, side, co, k, k, s, s, pad, pad, out, out),
-         'K': torch.empty(co, ci, k, k, device=META), 'n_out': co * out * out}
-    assert (vz._Packs().conv_split(p, M, M, False, 0) is not None) == split
+         'K': torch.empty(co, ci, k, k, device=META), 'n_out': co * out * out,
+         'n_in': ci * side * side}
+    assert (vz._Packs({'ops': []}, META).conv_split(p, M, M, False, 0) is not None) == split
 
 
 def test_window_limits():
@@ -177,6 +179,7 @@ def test_interval_conv_scratch(scratch, monkeypatch):
     (18432, 256, 256, True, False, True), (73728, 256, 256, False, True, True),
     (288, 256, 256, False, True, True), (288, 256, 256, False, False, False),
     (288, 1024, 1024, False, True, False), (576, 784, 128, False, True, False),
+    (2304, 784, 128, False, True, True), (2304, 1024, 64, False, False, False),
     (4608, 1024, 1024, False, True, True), (4608, 1024, 1024, True, False, True),
     (18432, 1024, 64, False, True, True), (73728, 1024, 64, False, True, False),
     (73728, 784, 10, False, False, False), (73728, 300, 5, False, True, True),

@@ -1,6 +1,8 @@
 """vc_backward_conv_split (the conv backward on the bf16 matrix cores, relu
 relaxation fused) against 64-bit sums, at the edges of its image groups, bands,
 channel chunks, output tiles and parity classes."""
+import ctypes
+
 import pytest
 import torch
 
@@ -112,3 +114,39 @@ def test_conv_split_infinities(gpu):
     assert (got - ref)[ok & ~big].norm() <= 1.3e-7 * ref[ok & ~big].norm()
     assert ((got - ref).abs() <= 1e-6 * ref.abs())[ok & big].all()
     assert (~ok).sum() > 0 and big.sum() > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('which', ['vc_conv_split_pack', 'vc_conv_t_pack'])
+def test_conv_pack_many_is_each_pack(gpu, which):
+    """Eighteen kernels, more than a launch takes, of one to a few workgroups."""
+    lib, taps = _lib.load(), which == 'vc_conv_t_pack'
+    g = torch.Generator(device=gpu).manual_seed(6)
+    geom = [(1 + 5 * i, 1 + 7 * (17 - i), 1 + i % 5, 1 + (i + 2) % 4, 1 + i % 3, 1 + (i + 1) % 2,
+             i % 3, i % 2) for i in range(18)]
+    K = [torch.randn(*q[:4], generator=g, device=gpu) for q in geom]
+
+    def out(q):
+        if taps:
+            return torch.full((lib.vc_conv_t_pack_floats(*q[:6]),), float('nan'), device=gpu)
+        return torch.full((lib.vc_conv_split_pack_bytes(*q[:6]),), 255, dtype=torch.uint8,
+                          device=gpu)
+    many, n = [out(q) for q in geom], 8 if taps else 6
+    arrays = [_lib.host_array(ctypes.c_void_p, [ptr(k) for k in K]),
+              _lib.host_array(ctypes.c_int32, [v for q in geom for v in q[:n]]),
+              _lib.host_array(ctypes.c_void_p, [ptr(m) for m in many])]
+    call(which + '_many', *(p for _, p in arrays), 18, stream())
+    for q, k, m in zip(geom, K, many):
+        co, ci, kh, kw, sh, sw, ph, pw = q
+        one = out(q)
+        call(which, ptr(k), *q[:n], ptr(one), stream())
+        assert torch.equal(m, one)
+        if not taps:
+            # the parts' sum, by class, chunk of 32 channels, tap, 16-channel tile
+            Ty, Tx, nch = -(-kh // sh), -(-kw // sw), -(-co // 32)
+            v = one.view(torch.bfloat16).view(sh, sw, nch, Ty, Tx, -1, 3, 4, 16, 8).double().sum(6)
+            # co = 32 chunk + 8 g + j, ci = 16 tile + r, ky = class + sh tap
+            v = v.permute(2, 6, 8, 5, 7, 3, 0, 4, 1).reshape(nch * 32, -1, Ty * sh, Tx * sw)
+            want = torch.zeros_like(v)
+            want[:co, :ci, :kh, :kw] = k
+            assert torch.equal(v, want)

@@ -121,8 +121,9 @@ def test_pack_many_is_each_pack(gpu, trans):
     arrays = [_lib.host_array(ctypes.c_void_p, [ptr(w) for w in W]),
               _lib.host_array(ctypes.c_int32, [K for K, _ in KN]),
               _lib.host_array(ctypes.c_int32, [N for _, N in KN]),
+              _lib.host_array(ctypes.c_int32, [trans] * 19),
               _lib.host_array(ctypes.c_void_p, [ptr(m) for m in many])]
-    call('vc_fc_split_pack_many', *(p for _, p in arrays[:3]), trans, arrays[3][1], 19, stream())
+    call('vc_fc_split_pack_many', *(p for _, p in arrays), 19, stream())
     for (K, N), w, m in zip(KN, W, many):
         one = torch.empty_like(m)
         call('vc_fc_split_pack', ptr(w), K, N, trans, ptr(one), stream())

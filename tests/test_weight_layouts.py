@@ -13,9 +13,9 @@ from vibecheck_amd import verify_zono_bnb as vz
 from vibecheck_amd import workloads as wk
 
 F32 = torch.float32
-# entry point: weight and packed buffers of a pack; packed operands of a product
-PACKS = {'vc_fc_split_pack': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5]),
-         'vc_conv_split_pack': (0, [7]), 'vc_conv_t_pack': (0, [9])}
+# entry point: weights and packed buffers of a pack; packed operands of a product
+PACKS = {'vc_fc_split_pack_many': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5]),
+         'vc_conv_split_pack_many': (0, [2]), 'vc_conv_t_pack_many': (0, [2])}
 READS = {'vc_backward_fc_split': [9], 'vc_alpha_grad_step_split': [9],
          'vc_alpha_grad_input_split': [6], 'vc_zono_fc_split': [5],
          'vc_ibp_conv_split': [6, 7], 'vc_backward_conv_split': [9],
@@ -100,16 +100,16 @@ def small(monkeypatch):
 @pytest.fixture
 def launches(monkeypatch, small):
     """Records launches on the CPU; the dict's 'stream' is the current one."""
-    rec = {'stream': 1, 'packed': {}, 'read': 0}
+    rec = {'stream': 1, 'packed': {}, 'read': 0, 'packs': 0}
 
     def call(name, *a):
         if name in PACKS:
             src, outs = PACKS[name]
             for i in outs:
-                rec['packed'][id(a[i])] = (a[i], a[-1], a[src], a[src].clone())
-        if name == 'vc_fc_split_pack_many':
-            for w, out in zip(a[0], a[4]):
-                rec['packed'][id(out)] = (out, a[-1], w, w.clone())
+                many = name.endswith('_many')
+                for w, out in zip(a[src], a[i]) if many else [(a[src], a[i])]:
+                    rec['packed'][id(out)] = (out, a[-1], w, w.clone())
+            rec['packs'] += 1
         for i in READS.get(name, []):
             _, st, src, was = rec['packed'][id(a[i])]
             assert st == a[-1], f'{name} reads weights packed on another stream'
@@ -148,6 +148,16 @@ def test_changed_weights_are_packed_again(launches, path):
         w.data.mul_(1.5)
     run()
     assert launches['read'] >= 2
+
+
+@pytest.mark.parametrize('path,most', [('spec', 1), ('alpha', 1), ('zono', 1), ('ibp', 1),
+                                       ('crown_cnn', 2), ('spec_cnn', 2)])
+def test_a_layout_is_one_launch(launches, path, most):
+    """The layers' weights go together: one launch for each kind of parts, one
+    for each form of the taps."""
+    gg, run = _case(path)
+    run()
+    assert 1 <= launches['packs'] <= most
 
 
 @pytest.mark.parametrize('path', PATHS)

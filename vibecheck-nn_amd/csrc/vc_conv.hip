@@ -273,30 +273,42 @@ struct LoadPackedT {
   }
 };
 
+// Kernels whose taps one launch packs.
+struct TapPack {
+  const float* K;
+  float* out;
+  int C_out, C_in, kh, kw, sh, sw, ph, pw, ld;
+  uint32_t block0;  // its first workgroup
+};
+constexpr int kTapPacks = 16;
+struct TapPacks {
+  TapPack p[kTapPacks];
+  int count;
+};
+
 // A[bz][ci][(co, ty, tx)] = K[co][ci][ky0 + sh ty][kx0 + sw tx] for every
 // parity class bz (LoadKernelT's values), zero past the kernel and in the
 // row padding.
-__global__ void k_conv_t_pack(const float* __restrict__ K, ConvGeom g, int Ty, int Tx, int ld,
-                              float* __restrict__ out) {
-  const int classes = g.sh * g.sw;
-  const int64_t total = (int64_t)classes * g.C_in * ld;
-  const int Kd = g.C_out * Ty * Tx;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int k = (int)(t % ld);
-    const int64_t rest = t / ld;
-    const int ci = (int)(rest % g.C_in);
-    const int bz = (int)(rest / g.C_in);
-    float v = 0.f;
-    if (k < Kd) {
-      const int co = k / (Ty * Tx), tt = k % (Ty * Tx);
-      const int ty = tt / Tx, tx = tt % Tx;
-      const int ky = tap_class(bz / g.sw, g.ph, g.sh).k0 + g.sh * ty;
-      const int kx = tap_class(bz % g.sw, g.pw, g.sw).k0 + g.sw * tx;
-      if (ky < g.kh && kx < g.kw) v = K[(((int64_t)co * g.C_in + ci) * g.kh + ky) * g.kw + kx];
-    }
-    out[t] = v;
+__global__ __launch_bounds__(NT) void k_conv_t_pack(TapPacks list) {
+  int i = 0;
+  while (i + 1 < list.count && blockIdx.x >= list.p[i + 1].block0) ++i;
+  const TapPack& g = list.p[i];
+  const int64_t t = (int64_t)(blockIdx.x - g.block0) * NT + threadIdx.x;
+  if (t >= (int64_t)g.sh * g.sw * g.C_in * g.ld) return;
+  const int Ty = (g.kh + g.sh - 1) / g.sh, Tx = (g.kw + g.sw - 1) / g.sw;
+  const int k = (int)(t % g.ld);
+  const int64_t rest = t / g.ld;
+  const int ci = (int)(rest % g.C_in);
+  const int bz = (int)(rest / g.C_in);
+  float v = 0.f;
+  if (k < g.C_out * Ty * Tx) {
+    const int co = k / (Ty * Tx), tt = k % (Ty * Tx);
+    const int ty = tt / Tx, tx = tt % Tx;
+    const int ky = tap_class(bz / g.sw, g.ph, g.sh).k0 + g.sh * ty;
+    const int kx = tap_class(bz % g.sw, g.pw, g.sw).k0 + g.sw * tx;
+    if (ky < g.kh && kx < g.kw) v = g.K[(((int64_t)co * g.C_in + ci) * g.kh + ky) * g.kw + kx];
   }
+  g.out[t] = v;
 }
 
 // ------------------------------------------------------------ epilogues
@@ -1046,19 +1058,36 @@ extern "C" int64_t vc_conv_t_pack_floats(int C_out, int C_in, int kh, int kw, in
   return (int64_t)sh * sw * C_in * conv_t_ld(C_out, kh, kw, sh, sw);
 }
 
+extern "C" int vc_conv_t_pack_many(const float* const* kernel, const int32_t* geom,
+                                   float* const* out, int count, vc_stream_t stream) {
+  if (count < 0 || (count > 0 && (!kernel || !geom || !out))) return VC_ERR_ARG;
+  for (int i = 0; i < count; ++i) {
+    const int32_t* g = geom + 8 * i;
+    if (!kernel[i] || !out[i] || g[6] < 0 || g[7] < 0 ||
+        vc_conv_t_pack_floats(g[0], g[1], g[2], g[3], g[4], g[5]) < 0)
+      return VC_ERR_ARG;
+  }
+  for (int i0 = 0; i0 < count; i0 += kTapPacks) {
+    TapPacks a{};
+    a.count = count - i0 < kTapPacks ? count - i0 : kTapPacks;
+    int64_t blocks = 0;
+    for (int i = 0; i < a.count; ++i) {
+      const int32_t* g = geom + 8 * (i0 + i);
+      a.p[i] = TapPack{kernel[i0 + i], out[i0 + i], g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7],
+                       conv_t_ld(g[0], g[2], g[3], g[4], g[5]), (uint32_t)blocks};
+      blocks += (vc_conv_t_pack_floats(g[0], g[1], g[2], g[3], g[4], g[5]) + NT - 1) / NT;
+      if (blocks >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(k_conv_t_pack, dim3((unsigned)blocks), dim3(NT), 0, (hipStream_t)stream, a);
+    VC_LAUNCH_CHECK();
+  }
+  return VC_OK;
+}
+
 extern "C" int vc_conv_t_pack(const float* kernel, int C_out, int C_in, int kh, int kw, int sh,
                               int sw, int ph, int pw, float* out, vc_stream_t stream) {
-  if (!kernel || !out || C_out <= 0 || C_in <= 0 || kh <= 0 || kw <= 0 || sh <= 0 || sw <= 0 ||
-      ph < 0 || pw < 0)
-    return VC_ERR_ARG;
-  ConvGeom g{C_in, 1, 1, C_out, kh, kw, sh, sw, ph, pw, 1, 1};
-  const int Ty = (kh + sh - 1) / sh, Tx = (kw + sw - 1) / sw;
-  const int ld = conv_t_ld(C_out, kh, kw, sh, sw);
-  const int64_t total = (int64_t)sh * sw * C_in * ld;
-  hipLaunchKernelGGL(k_conv_t_pack, dim3(vc_blocks(total, NT)), dim3(NT), 0, (hipStream_t)stream,
-                     kernel, g, Ty, Tx, ld, out);
-  VC_LAUNCH_CHECK();
-  return VC_OK;
+  const int32_t geom[8] = {C_out, C_in, kh, kw, sh, sw, ph, pw};
+  return vc_conv_t_pack_many(&kernel, geom, &out, 1, stream);
 }
 
 extern "C" int vc_backward_conv_packed(const float* ew_in, int64_t M, const float* kernel,

@@ -391,37 +391,50 @@ __global__ __launch_bounds__(CNT, 2) void k_conv_split(SplitArgs a) {
   }
 }
 
+// Kernels whose parts one launch makes (5 us whatever their size).
+struct PackArgs {
+  const float* K;
+  uint4* out;
+  int C_out, C_in, kh, kw, sh, sw, Ty, Tx, nchunk, MTp;
+  uint32_t block0;  // its first workgroup
+};
+constexpr int kPacks = 16;
+struct PackList {
+  PackArgs p[kPacks];
+  int count;
+};
+
 // A[class][chunk][tap][mt][part][lane][8]: part of K[co][ci][k0y + sh ty][k0x
 // + sw tx] with ci = 16 mt + lane % 16, co = 32 chunk + 8 (lane / 16) + j;
 // zero past the kernel and the channels.  class = k0y sw + k0x.
-__global__ void k_conv_split_pack(const float* K, int C_out, int C_in, int kh, int kw, int sh,
-                                  int sw, int Ty, int Tx, int nchunk, int MTp, uint4* out) {
-  const int T = Ty * Tx;
-  const int64_t total = (int64_t)sh * sw * nchunk * T * MTp * 64;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int lane = (int)(t & 63);
-    int64_t q = t >> 6;
-    const int mt = (int)(q % MTp);
-    q /= MTp;
-    const int tap = (int)(q % T);
-    q /= T;
-    const int ch = (int)(q % nchunk), cls = (int)(q / nchunk);
-    const int ky = cls / sw + sh * (tap / Tx), kx = cls % sw + sw * (tap % Tx);
-    const int ci = 16 * mt + (lane & 15), co0 = CK * ch + 8 * (lane >> 4);
-    float v[8];
+__global__ __launch_bounds__(CNT) void k_conv_split_pack(PackList list) {
+  int i = 0;
+  while (i + 1 < list.count && blockIdx.x >= list.p[i + 1].block0) ++i;
+  const PackArgs& a = list.p[i];
+  const int T = a.Ty * a.Tx;
+  const int64_t t = (int64_t)(blockIdx.x - a.block0) * CNT + threadIdx.x;
+  if (t >= (int64_t)a.sh * a.sw * a.nchunk * T * a.MTp * 64) return;
+  const int lane = (int)(t & 63);
+  int64_t q = t >> 6;
+  const int mt = (int)(q % a.MTp);
+  q /= a.MTp;
+  const int tap = (int)(q % T);
+  q /= T;
+  const int ch = (int)(q % a.nchunk), cls = (int)(q / a.nchunk);
+  const int ky = cls / a.sw + a.sh * (tap / a.Tx), kx = cls % a.sw + a.sw * (tap % a.Tx);
+  const int ci = 16 * mt + (lane & 15), co0 = CK * ch + 8 * (lane >> 4);
+  float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = (ci < C_in && co0 + j < C_out && ky < kh && kx < kw)
-                 ? K[(((int64_t)(co0 + j) * C_in + ci) * kh + ky) * kw + kx]
-                 : 0.f;
-    uint4 h, m, l;
-    split8(v, h, m, l);
-    uint4* o = out + ((t >> 6) * 3) * 64 + lane;
-    o[0] = h;
-    o[64] = m;
-    o[128] = l;
-  }
+  for (int j = 0; j < 8; ++j)
+    v[j] = (ci < a.C_in && co0 + j < a.C_out && ky < a.kh && kx < a.kw)
+               ? a.K[(((int64_t)(co0 + j) * a.C_in + ci) * a.kh + ky) * a.kw + kx]
+               : 0.f;
+  uint4 h, m, l;
+  split8(v, h, m, l);
+  uint4* o = a.out + ((t >> 6) * 3) * 64 + lane;
+  o[0] = h;
+  o[64] = m;
+  o[128] = l;
 }
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
@@ -700,15 +713,38 @@ extern "C" int64_t vc_conv_split_pack_bytes(int C_out, int C_in, int kh, int kw,
          split_mtp(C_in) * 3 * 64 * 16;
 }
 
+extern "C" int vc_conv_split_pack_many(const float* const* kernel, const int32_t* geom,
+                                       void* const* out, int count, vc_stream_t stream) {
+  if (count < 0 || (count > 0 && (!kernel || !geom || !out))) return VC_ERR_ARG;
+  for (int i = 0; i < count; ++i) {
+    const int32_t* g = geom + 6 * i;
+    if (!kernel[i] || !out[i] || !aligned16(out[i]) ||
+        vc_conv_split_pack_bytes(g[0], g[1], g[2], g[3], g[4], g[5]) < 0)
+      return VC_ERR_ARG;
+  }
+  for (int i0 = 0; i0 < count; i0 += kPacks) {
+    PackList a{};
+    a.count = count - i0 < kPacks ? count - i0 : kPacks;
+    int64_t blocks = 0;
+    for (int i = 0; i < a.count; ++i) {
+      const int32_t* g = geom + 6 * (i0 + i);
+      a.p[i] = PackArgs{kernel[i0 + i], (uint4*)out[i0 + i], g[0], g[1], g[2], g[3], g[4], g[5],
+                        ceil_div(g[2], g[4]), ceil_div(g[3], g[5]), ceil_div(g[0], CK),
+                        split_mtp(g[1]), (uint32_t)blocks};
+      blocks += (vc_conv_split_pack_bytes(g[0], g[1], g[2], g[3], g[4], g[5]) / 48 + CNT - 1) / CNT;
+      if (blocks >= (int64_t(1) << 31)) return VC_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(k_conv_split_pack, dim3((unsigned)blocks), dim3(CNT), 0,
+                       (hipStream_t)stream, a);
+    VC_LAUNCH_CHECK();
+  }
+  return VC_OK;
+}
+
 extern "C" int vc_conv_split_pack(const float* kernel, int C_out, int C_in, int kh, int kw, int sh,
                                   int sw, void* out, vc_stream_t stream) {
-  const int64_t bytes = vc_conv_split_pack_bytes(C_out, C_in, kh, kw, sh, sw);
-  if (!kernel || !out || bytes < 0 || !aligned16(out)) return VC_ERR_ARG;
-  hipLaunchKernelGGL(k_conv_split_pack, dim3(vc_blocks(bytes / 48, CNT)), dim3(CNT), 0,
-                     (hipStream_t)stream, kernel, C_out, C_in, kh, kw, sh, sw, ceil_div(kh, sh),
-                     ceil_div(kw, sw), ceil_div(C_out, CK), split_mtp(C_in), (uint4*)out);
-  VC_LAUNCH_CHECK();
-  return VC_OK;
+  const int32_t geom[6] = {C_out, C_in, kh, kw, sh, sw};
+  return vc_conv_split_pack_many(&kernel, geom, &out, 1, stream);
 }
 
 extern "C" int vc_backward_conv_split_ok(int C_out, int H_out, int W_out, int C_in, int H, int W,

@@ -704,16 +704,17 @@ extern "C" int vc_fc_split_pack_abs(const float* W, int K, int N, int trans, voi
 }
 
 extern "C" int vc_fc_split_pack_many(const float* const* W, const int32_t* K, const int32_t* N,
-                                     int trans, void* const* out, int count,
+                                     const int32_t* trans, void* const* out, int count,
                                      vc_stream_t stream) {
-  if (count < 0 || (count > 0 && (!W || !K || !N || !out))) return VC_ERR_ARG;
+  if (count < 0 || (count > 0 && (!W || !K || !N || !trans || !out))) return VC_ERR_ARG;
   for (int i = 0; i < count; ++i)
     if (!W[i] || !out[i] || K[i] <= 0 || N[i] <= 0 || !aligned16(out[i])) return VC_ERR_ARG;
   for (int i0 = 0; i0 < count; i0 += kPacks) {
     Packs a{};
     a.count = count - i0 < kPacks ? count - i0 : kPacks;
     for (int i = 0; i < a.count; ++i)
-      a.p[i] = Pack{W[i0 + i], (uint4*)out[i0 + i], nullptr, K[i0 + i], N[i0 + i], trans};
+      a.p[i] =
+          Pack{W[i0 + i], (uint4*)out[i0 + i], nullptr, K[i0 + i], N[i0 + i], trans[i0 + i]};
     const int rc = launch_pack(a, (hipStream_t)stream);
     if (rc != VC_OK) return rc;
   }

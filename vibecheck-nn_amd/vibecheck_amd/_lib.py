@@ -67,7 +67,9 @@ SIGNATURES = {
     'vc_fc_split_pack_bytes': [_L, _L],
     'vc_fc_split_pack': [_P, _I, _I, _I, _P, _P],
     'vc_fc_split_pack_abs': [_P, _I, _I, _I, _P, _P, _P],
-    'vc_fc_split_pack_many': [_P, _P, _P, _I, _P, _I, _P],
+    'vc_fc_split_pack_many': [_P, _P, _P, _P, _P, _I, _P],
+    'vc_conv_split_pack_many': [_P, _P, _P, _I, _P],
+    'vc_conv_t_pack_many': [_P, _P, _P, _I, _P],
     'vc_backward_fc_split': [_P, _L, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P],
     'vc_alpha_grad_step_split': [_P, _P, _L, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _P],
     'vc_alpha_grad_input_split': [_P, _P, _P, _L, _I, _I, _P, _P, _I, _P, _P, _P],

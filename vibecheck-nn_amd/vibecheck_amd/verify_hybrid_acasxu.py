@@ -178,7 +178,7 @@ def _full_freeze(xl, xh, gg, spec_ew, device, dtype, n_iters_per_layer=100,
     if n_iters_spec < 1:
         raise ValueError('vibecheck_amd: the spec loop needs at least one iteration')
     feeds = _relu_feeds(gg)
-    packs = vz._Packs()
+    packs = vz._Packs(gg, dev)
     alpha_per_layer = {}
     for L in order:
         if deadline is not None and time.perf_counter() > deadline:
@@ -250,7 +250,7 @@ def _replay_batched(xl_b, xh_b, gg, spec_ew, alpha_layer_b, alpha_spec_b,
                         for k, a in alpha_spec_b.items()}
     tight = _zono_tight(xl, xh, gg, device, dtype)
     feeds = _relu_feeds(gg)
-    packs = vz._Packs()
+    packs = vz._Packs(gg, dev)
     for L in sorted(tight):
         if not alpha_layer_b.get(L):
             continue

@@ -196,7 +196,7 @@ def _ibp_crown_bab_bound(gg, xl, xh, sb_root, relu_clamps, spec_ew, device,
     n_eval = 0
     step = 0
     n_it = max(1, int(alpha_iters))
-    packs = _Packs()
+    packs = _Packs(gg, dev)
     for it in range(n_it):
         # the Adam step after the last evaluation is never used: skip its gradient
         last = it == n_it - 1

@@ -195,35 +195,48 @@ class _Packs:
     goes with the call: another thread's call on its own stream packs for
     itself, and a weight written between two calls (also through ``.data``,
     which no version counter shows) is seen by the second.  1024 x 1024 weights
-    take 6 us, of products of 100 us and more."""
+    take 6 us, of products of 100 us and more; a launch takes 5 whatever it
+    packs, so the first need of a layout makes it of every layer of the network
+    that the same rule takes."""
 
-    def __init__(self):
-        self._made = {}
+    def __init__(self, gg, dev):
+        self.gg, self.dev, self._made = gg, dev, {}
 
-    def fc(self, p, st, trans=False):
-        """The bf16 parts of an fc's W, or of its transpose."""
-        self.fcs([p], st, trans)
+    def _params(self, kind):
+        return [_op_params(op, self.dev) for op in self.gg['ops'] if op['type'] == kind]
+
+    def _make(self, entry, keys, params, describe, dtype, st):
+        """One launch: the weights of ``params`` into buffers under ``keys``;
+        ``describe`` gives their sizes and the host arrays of the layers' shapes,
+        which the graph keeps by those shapes."""
+        shapes = self.gg.setdefault('_vc_amd_packs', {})
+        at = (entry, *keys, *[q.get('geom', (q['n_in'], q['n_out'])) for q in params])
+        if at not in shapes:
+            sizes, rows = describe()
+            shapes[at] = sizes, sum(sizes), [host_array(ctypes.c_int32, r) for r in rows]
+        sizes, total, arrays = shapes[at]
+        outs = torch.empty(total, dtype=dtype, device=self.dev).split(sizes)
+        src, src_p = host_array(ctypes.c_void_p,
+                                [ptr(q['W'] if 'W' in q else q['K']) for q in params])
+        dst, dst_p = host_array(ctypes.c_void_p, [ptr(o) for o in outs])
+        call(entry, src_p, *[p for _, p in arrays], dst_p, len(keys), st)
+        self._made.update(zip(keys, outs))
+
+    def fc(self, p, st, trans=False, others=()):
+        """The bf16 parts of an fc's W, or of its transpose; ``others``: (params,
+        transposed) that the call will need as well."""
+        if (p['name'], trans) not in self._made:
+            want = [(p, trans)] + [q for q in others if q[0] is not p or q[1] != trans]
+            want = [(q, t) for q, t in want if (q['name'], t) not in self._made]
+
+            def describe():
+                KN = [(q['n_in'], q['n_out']) if t else (q['n_out'], q['n_in']) for q, t in want]
+                size = _lib.load().vc_fc_split_pack_bytes
+                return ([size(K, N) for K, N in KN],
+                        [[K for K, _ in KN], [N for _, N in KN], [int(t) for _, t in want]])
+            self._make('vc_fc_split_pack_many', [(q['name'], t) for q, t in want],
+                       [q for q, _ in want], describe, torch.uint8, st)
         return self._made[p['name'], trans]
-
-    def fcs(self, ps, st, trans):
-        """Makes those of several, together."""
-        ps = [p for p in ps if (p['name'], trans) not in self._made]
-        if not ps:
-            return
-        size = _lib.load().vc_fc_split_pack_bytes
-        KN = [(p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in']) for p in ps]
-        sizes = [size(K, N) for K, N in KN]  # multiples of 16 bytes
-        outs = torch.empty(sum(sizes), dtype=torch.uint8, device=ps[0]['W'].device).split(sizes)
-        if len(ps) == 1:
-            call('vc_fc_split_pack', ptr(ps[0]['W']), *KN[0], 1 if trans else 0, ptr(outs[0]), st)
-        else:
-            W, W_p = host_array(ctypes.c_void_p, [ptr(p['W']) for p in ps])
-            out, out_p = host_array(ctypes.c_void_p, [ptr(o) for o in outs])
-            k, k_p = host_array(ctypes.c_int32, [K for K, _ in KN])
-            n, n_p = host_array(ctypes.c_int32, [N for _, N in KN])
-            call('vc_fc_split_pack_many', W_p, k_p, n_p, 1 if trans else 0, out_p, len(ps), st)
-        for p, o in zip(ps, outs):
-            self._made[p['name'], trans] = o
 
     def conv_interval(self, p, K, st):
         """The parts of a conv's kernel and of its magnitudes for
@@ -244,37 +257,70 @@ class _Packs:
         """A conv kernel's transposed taps by output-parity class
         (vc_conv_t_pack); ``window``: without the padding, for rows that carry
         their place in the image."""
-        out = self._made.get((p['name'], 'taps', window))
-        if out is None:
+        key = (p['name'], 'taps', window)
+        if key not in self._made:
+            # the fold kernel's convs, of up to four channels, take none
+            want = [p] + [q for q in self._params('conv')
+                          if q is not p and q['geom'][0] > 4 and not self.has_taps(q, window)]
+
+            def describe():
+                geom, sizes = [], []
+                for q in want:
+                    C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = q['geom']
+                    geom += [C_out, C_in, kh, kw, sh, sw] + ([0, 0] if window else [ph, pw])
+                    sizes.append(_lib.load().vc_conv_t_pack_floats(C_out, C_in, kh, kw, sh, sw))
+                    if sizes[-1] < 0:
+                        raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {q["geom"]}')
+                return sizes, [geom]
+            # rows of four floats: every buffer starts on 16 bytes
+            self._make('vc_conv_t_pack_many', [(q['name'], 'taps', window) for q in want], want,
+                       describe, torch.float32, st)
+        return self._made[key]
+
+    def _conv_split_pays(self, p, M, R, shared):
+        last = p.get('split_pays')  # of the rows asked for last
+        if last is None or last[0] != (M, R, shared):
             C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-            n = _lib.load().vc_conv_t_pack_floats(C_out, C_in, kh, kw, sh, sw)
-            if n < 0:
-                raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {p["geom"]}')
-            out = torch.empty(n, device=p['K'].device)
-            if window:
-                ph = pw = 0
-            call('vc_conv_t_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ph, pw,
-                 ptr(out), st)
-            self._made[p['name'], 'taps', window] = out
-        return out
+            bands = 0 if _few_channels(p) else _lib.load().vc_backward_conv_split_fits(
+                M, R, 1 if shared else 0, C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
+            last = (M, R, shared), (
+                bands == 1 or bands > 1 and (M >= _CONV_SPLIT_ROWS or M * p['n_out'] * C_in * kh
+                                             * kw >= _CONV_SPLIT_MACS))
+            p['split_pays'] = last
+        return last[1]
 
     def conv_split(self, p, M, R, shared, st):
         """A conv kernel's bf16 parts for vc_backward_conv_split of M rows (R a
         domain, shared by all domains or not); None where the geometry or the
         rows are outside that kernel, or the fp32 product is the faster one."""
-        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-        bands = _lib.load().vc_backward_conv_split_fits(
-            M, R, 1 if shared else 0, C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
-        if bands == 0 or (bands > 1 and M < _CONV_SPLIT_ROWS
-                          and M * p['n_out'] * C_in * kh * kw < _CONV_SPLIT_MACS):
+        if not self._conv_split_pays(p, M, R, shared):
             return None
-        out = self._made.get((p['name'], 'conv_split'))
-        if out is None:
-            n = _lib.load().vc_conv_split_pack_bytes(C_out, C_in, kh, kw, sh, sw)
-            out = torch.empty(n, dtype=torch.uint8, device=p['K'].device)
-            call('vc_conv_split_pack', ptr(p['K']), C_out, C_in, kh, kw, sh, sw, ptr(out), st)
-            self._made[p['name'], 'conv_split'] = out
-        return out
+        key = (p['name'], 'conv_split')
+        if key not in self._made:
+            want = [p] + [q for q in self._params('conv')
+                          if q is not p and (q['name'], 'conv_split') not in self._made
+                          and self._conv_split_pays(q, M, R, shared)]
+
+            def describe():
+                geom = [[q['geom'][i] for i in (3, 0, 4, 5, 6, 7)] for q in want]
+                return ([_lib.load().vc_conv_split_pack_bytes(*g) for g in geom],
+                        [sum(geom, [])])
+            self._make('vc_conv_split_pack_many', [(q['name'], 'conv_split') for q in want], want,
+                       describe, torch.uint8, st)
+        return self._made[key]
+
+
+def _few_channels(p, window=None):
+    """Whether a conv (of windows: (rows' height and width, the result's)) is the
+    fold kernel's: a few input channels, the network's first layer."""
+    key = ('fold_ok', window)
+    if key not in p:
+        C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
+        if window is not None:
+            (Ho, Wo, H, W), ph, pw = window, 0, 0
+        p[key] = bool(_lib.load().vc_backward_relu_conv_ok(C_out, Ho, Wo, C_in, H, W, kh, kw,
+                                                           sh, sw, ph, pw))
+    return p[key]
 
 
 def _fc_split_pays(M, K, N, once, sweep):
@@ -288,19 +334,24 @@ def _fc_split_pays(M, K, N, once, sweep):
     if K > _TWO_PHASE_MIN_WIDTH and (4 * N >= K or 6 * M * K <= 288 << 20):
         if M >= 8192 or (M >= 4096 if once else M >= 2048) and M * K * N >= (1e9 if once else 4e8):
             return True
-    return sweep and _FC_SPLIT_SWEEP_ROWS <= M < 8192 and K <= 512
+    return sweep and _FC_SPLIT_SWEEP_ROWS <= M < 8192 and (K <= 512 or M >= 2048)
 
 
 def _fc_split_parts(packs, p, M, st, trans=False, once=False, sweep=False):
     """The fc weights' bf16 parts for M rows' vc_backward_fc_split (``trans``:
     for the gradient's products with W^T); None where the fp32 product is the
     faster one."""
-    K, N = (p['n_in'], p['n_out']) if trans else (p['n_out'], p['n_in'])
-    if trans:
-        ok = M >= _FC_SPLIT_SWEEP_ROWS and min(K, N) >= _FC_SPLIT_WIDTH
-    else:
-        ok = _fc_split_pays(M, K, N, once, sweep)
-    return packs.fc(p, st, trans) if ok and M < 1 << 31 else None
+    def pays(q, t):
+        if t:
+            return M >= _FC_SPLIT_SWEEP_ROWS and min(q['n_in'], q['n_out']) >= _FC_SPLIT_WIDTH
+        return _fc_split_pays(M, q['n_out'], q['n_in'], once, sweep)
+    if M >= 1 << 31 or not pays(p, trans):
+        return None
+    if (p['name'], trans) in packs._made:
+        return packs.fc(p, st, trans)
+    forms = (True,) if trans else (False, True) if sweep else (False,)
+    return packs.fc(p, st, trans, [(q, t) for q in packs._params('fc') for t in forms
+                                   if pays(q, t)])
 
 
 def _cut(t, rows):
@@ -461,7 +512,7 @@ def _ibp_forward_graph_batched(xl, xh, gg, device, dtype, relu_clamps=None,
     hi = {gg['input_name']: xh}
     sb = {}
     st = stream()
-    packs = _Packs()
+    packs = _Packs(gg, dev)
     # nodes without a relu below them: their intervals are exact, CROWN's first
     # bounds equal them up to rounding and choose slopes by the larger of the
     # two, so their sums keep their order
@@ -628,7 +679,7 @@ def _zono_forward(xl, xh, gg, dtype, bounds_only):
     vidx = varying.nonzero(as_tuple=True)[0].to(torch.int32).contiguous()
     K = int(vidx.numel())
     ops = gg['ops']
-    packs = _Packs()
+    packs = _Packs(gg, dev)
     users = {}
     for op in ops:
         for i in op['inputs']:
@@ -745,11 +796,10 @@ def _zono_forward(xl, xh, gg, dtype, bounds_only):
             if together and Kc:
                 # queued before the host waits, with those of the layers to come
                 # (generators only grow in number)
-                packs.fcs([_op_params(u, dev) for u in [nxt] + [
-                    v for v in map(one_fc, (o['name'] for o in ops[pos + 1:top]
-                                            if o['type'] == 'relu'))
-                    if v is not None and B * Kc * int(v['W'].numel()) >= _ZONO_SPLIT_MACS]],
-                    st, True)
+                packs.fc(_op_params(nxt, dev), st, True,
+                         [(_op_params(v, dev), True) for v in map(
+                             one_fc, (o['name'] for o in ops[pos + 1:top] if o['type'] == 'relu'))
+                          if v is not None and B * Kc * int(v['W'].numel()) >= _ZONO_SPLIT_MACS])
             k_new = int(cnt.max().item()) if B > 0 else 0
             c_o = torch.empty(B, n, device=dev)
             if together:
@@ -872,6 +922,7 @@ _TWO_PHASE_MIN_WIDTH = 64
 #   512 x 512       576: 15 and 14;   2,304: 30 and 25;   4,608: 47 and 32
 #   784 x 128     4,608: 41 and 32;  36,864: 182 and 137; 73,728: 250 and 248
 #   1024 x 784    1,152: 32 and 34;   2,304: 48 and 42;   4,608: 79 and 67
+#   1024 x 64     2,304: 29 and 26;  18,432: 115 and 75;  73,728: 290 and 286
 #   1024 x 1024     288: 20 and 26;   2,304: 75 and 48;  73,728: 1,202 and 991
 # The gradient's, whose fp32 product sums in 64 bits (slopes on both sides):
 #   128 x 128       288: 10 and 9;  256 x 256: 15 and 10;  1024 x 1024: 52 and 25;
@@ -921,9 +972,9 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
     A of window rows is None.
     """
     once = packs is None
-    packs = _Packs() if once else packs
     B, n_in = xl.shape
     dev = xl.device
+    packs = _Packs(gg, dev) if once else packs
     st = stream()
     widths = _widths(gg, n_in)
     rows = seed if isinstance(seed, _Rows) else _Rows(seed, seed_shared)
@@ -1029,18 +1080,6 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
              ptr(acc), st)
         return _Rows(out, False)
 
-    def few_channels(p, window=None):
-        """Whether the conv (of windows: (rows' height and width, the result's))
-        is the fold kernel's: a few input channels, the network's first layer."""
-        key = ('fold_ok', window)
-        if key not in p:
-            C_in, H, W, C_out, kh, kw, sh, sw, ph, pw, Ho, Wo = p['geom']
-            if window is not None:
-                (Ho, Wo, H, W), ph, pw = window, 0, 0
-            p[key] = bool(_lib.load().vc_backward_relu_conv_ok(C_out, Ho, Wo, C_in, H, W, kh, kw,
-                                                               sh, sw, ph, pw))
-        return p[key]
-
     def conv_fp32(p, ew, M, window, out, bias, acc):
         """M rows through a conv in fp32, acc += rows . bias; the fold kernel
         reads the kernel as it lies, the gathering product its packed taps, or
@@ -1049,7 +1088,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         if window is not None:
             (Ho, Wo, H, W), ph, pw = window, 0, 0
         geom = (C_out, Ho, Wo, C_in, H, W, kh, kw, sh, sw, ph, pw)
-        if few_channels(p, window) or (M * C_out * Ho * Wo * C_in * kh * kw < _CONV_TAPS_MACS
+        if _few_channels(p, window) or (M * C_out * Ho * Wo * C_in * kh * kw < _CONV_TAPS_MACS
                                        and not packs.has_taps(p, window is not None)):
             call('vc_backward_conv', ptr(ew), M, ptr(p['K']), ptr(bias), *geom, ptr(out),
                  ptr(acc), st)
@@ -1111,7 +1150,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
         relaxation's form is outside the fused kernels."""
         if rows.alpha_group is not None or (rows.alpha is not None and rows.alpha_row):
             return None
-        fold = few_channels(p)
+        fold = _few_channels(p)
         parts = (None if fold or not split
                  else packs.conv_split(p, B * R, R, rows.shared, st))
         if not fold and parts is None:
@@ -1290,7 +1329,7 @@ def _backward(tight, xl, xh, gg, seed_name, seed, seed_shared, acc0,
             bias, acc_b = bias_acc(rows, p)
             M = R if rows.shared else B * R
             out = torch.empty(M, p['n_in'], device=dev)
-            parts = (None if not split or few_channels(p)
+            parts = (None if not split or _few_channels(p)
                      else packs.conv_split(p, M, M, False, st))
             if parts is not None:
                 call('vc_backward_conv_split', ptr(rows.ew), M, M, 0, None, None, None, None,
@@ -1451,7 +1490,7 @@ def _crown_intermediate_batched(gg, xl, xh, device, dtype, chunk=2048,
                  if op['type'] == 'relu' and 'layer_idx' in op}
     B = xl.shape[0]
     st = stream()
-    packs = _Packs()
+    packs = _Packs(gg, dev)
     ch = max(1, int(chunk))
     for L in sorted(tight):
         if L not in relu_by_L:
@@ -1523,9 +1562,9 @@ def _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, want_grad, galpha,
     has that shape too.  ``want_A``: returns (lb, A) with A (B*Q, n_in) the
     input linearization of the rows.  ``packs``: the loop's _Packs."""
     B, n_in = xl.shape
-    packs = _Packs() if packs is None else packs
     Q = Wq.shape[0]
     dev = xl.device
+    packs = _Packs(gg, dev) if packs is None else packs
     st = stream()
     trace = BackwardTrace() if want_grad else None
     seed = gg['ops'][-1]['name'] if seed_name is None else seed_name
@@ -1675,7 +1714,7 @@ def _run_alpha_crown_inputsplit_batched(xl, xh, gg, spec_ew, device, dtype,
     n_eval = 0
     step = 0
     cur_lr = float(lr)
-    packs = _Packs()
+    packs = _Packs(gg, dev)
     for it in range(n_iters):
         lb = _alpha_backward_and_grad(sb, xl, xh, gg, Wq, bq, alpha, True,
                                       galpha, packs=packs)
