@@ -15,7 +15,8 @@ from vibecheck_amd import workloads as wk
 F32 = torch.float32
 # entry point: weights and packed buffers of a pack; packed operands of a product
 PACKS = {'vc_fc_split_pack_many': (0, [4]), 'vc_fc_split_pack_abs': (0, [4, 5]),
-         'vc_conv_split_pack_many': (0, [2]), 'vc_conv_t_pack_many': (0, [2])}
+         'vc_conv_split_pack_many': (0, [2]), 'vc_conv_t_pack_many': (0, [2]),
+         'vc_fc_split_pack': (0, [4]), 'vc_conv_split_pack': (0, [7]), 'vc_conv_t_pack': (0, [9])}
 READS = {'vc_backward_fc_split': [9], 'vc_alpha_grad_step_split': [9],
          'vc_alpha_grad_input_split': [6], 'vc_zono_fc_split': [5],
          'vc_ibp_conv_split': [6, 7], 'vc_backward_conv_split': [9],

@@ -213,13 +213,20 @@ class _Packs:
         at = (entry, *keys, *[q.get('geom', (q['n_in'], q['n_out'])) for q in params])
         if at not in shapes:
             sizes, rows = describe()
-            shapes[at] = sizes, sum(sizes), [host_array(ctypes.c_int32, r) for r in rows]
+            shapes[at] = (sizes, sum(sizes), sum(rows, []) if len(keys) == 1 else
+                          [host_array(ctypes.c_int32, r) for r in rows])
         sizes, total, arrays = shapes[at]
-        outs = torch.empty(total, dtype=dtype, device=self.dev).split(sizes)
+        out = torch.empty(total, dtype=dtype, device=self.dev)
+        if len(keys) == 1:
+            q = params[0]
+            call(entry, ptr(q['W'] if 'W' in q else q['K']), *arrays, ptr(out), st)
+            self._made[keys[0]] = out
+            return
+        outs = out.split(sizes)
         src, src_p = host_array(ctypes.c_void_p,
                                 [ptr(q['W'] if 'W' in q else q['K']) for q in params])
         dst, dst_p = host_array(ctypes.c_void_p, [ptr(o) for o in outs])
-        call(entry, src_p, *[p for _, p in arrays], dst_p, len(keys), st)
+        call(entry + '_many', src_p, *[p for _, p in arrays], dst_p, len(keys), st)
         self._made.update(zip(keys, outs))
 
     def fc(self, p, st, trans=False, others=()):
@@ -234,7 +241,7 @@ class _Packs:
                 size = _lib.load().vc_fc_split_pack_bytes
                 return ([size(K, N) for K, N in KN],
                         [[K for K, _ in KN], [N for _, N in KN], [int(t) for _, t in want]])
-            self._make('vc_fc_split_pack_many', [(q['name'], t) for q, t in want],
+            self._make('vc_fc_split_pack', [(q['name'], t) for q, t in want],
                        [q for q, _ in want], describe, torch.uint8, st)
         return self._made[p['name'], trans]
 
@@ -273,7 +280,7 @@ class _Packs:
                         raise RuntimeError(f'vc_conv_t_pack_floats: bad geometry {q["geom"]}')
                 return sizes, [geom]
             # rows of four floats: every buffer starts on 16 bytes
-            self._make('vc_conv_t_pack_many', [(q['name'], 'taps', window) for q in want], want,
+            self._make('vc_conv_t_pack', [(q['name'], 'taps', window) for q in want], want,
                        describe, torch.float32, st)
         return self._made[key]
 
@@ -305,7 +312,7 @@ class _Packs:
                 geom = [[q['geom'][i] for i in (3, 0, 4, 5, 6, 7)] for q in want]
                 return ([_lib.load().vc_conv_split_pack_bytes(*g) for g in geom],
                         [sum(geom, [])])
-            self._make('vc_conv_split_pack_many', [(q['name'], 'conv_split') for q in want], want,
+            self._make('vc_conv_split_pack', [(q['name'], 'conv_split') for q in want], want,
                        describe, torch.uint8, st)
         return self._made[key]
 
